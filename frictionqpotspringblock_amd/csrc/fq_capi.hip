@@ -533,6 +533,7 @@ struct Group {
             auto& r = hrs[i];
             r.status = (mask && !mask[i]) ? fq::ST_IDLE : fq::ST_RUNNING;
             r.steps = 0;
+            r.refilled = 0;
             r.below = 0;
             r.below2 = 0;
             r.dec = 0;
@@ -745,6 +746,12 @@ struct Group {
             HIPC(hipEventElapsedTime(&ms, ev0, ev1));
         }
         pull();
+        for (const auto& r : hrs) { // windows moved inside a launch
+            if (r.refilled) {
+                ++refills;
+                break;
+            }
+        }
         return ms;
     }
 

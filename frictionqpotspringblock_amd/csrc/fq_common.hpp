@@ -130,7 +130,7 @@ struct RunState {
     // reductions written by service kernels
     double red0;
     int32_t red_flag;
-    int32_t pad2;
+    int32_t refilled; // set by a run whose kernel moved a landscape window inside the launch
     // uniform displacement of the particles applied by k_forces(FF_ADD_U)
     double du_add;
     // quasistatic driver: next event of the run (0-based), its phase, and the

@@ -37,20 +37,21 @@ FQ_HD double potential_force_mid(const SysView& S, double u, double yl, double y
     }
 }
 
-template <int POT, int INT, int EXT, int PPT, int MAXT, bool UNIT, bool FULL = false>
-__global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views, RunArgs ra)
+// One entry of k_flow: from the state in memory to the state in memory, until
+// the launch's step budget (of which earlier entries took `launch_done`) or a
+// NaN; without INLINE_REFILL also up to a step that has to move a window
+// (ST_REFILL, `rmask`: this thread's particles). Returns why it stopped.
+template <int POT, int INT, int EXT, int PPT, bool UNIT, bool FULL, bool INLINE_REFILL>
+__device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views, const RunArgs& ra,
+                                              int64_t& launch_done, uint32_t& refill_mask)
 {
-    static_assert(is_chain<INT>(), "k_flow handles chains");
     const SysView& S = views[blockIdx.x];
     // the system's parameters as a local copy: registers for the whole launch
     // instead of a reload of the ones the forces use after every barrier
     const SysView P = S;
     RunState* const rs = S.rs;
-    if (rs->status != ST_RUNNING && rs->status != ST_BUDGET) {
-        return;
-    }
-    const int64_t room = rs->target - rs->steps;
-    const int limit = uniform_i((int)(room < ra.max_steps ? (room > 0 ? room : 0) : ra.max_steps));
+    const int64_t room = rs->target - rs->steps, budget = ra.max_steps - launch_done;
+    const int limit = uniform_i((int)(room < budget ? (room > 0 ? room : 0) : budget));
 
     __shared__ int s_nan[2];
     __shared__ int s_refill[2];
@@ -155,11 +156,12 @@ __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views
         }
     };
 
-    // slips of step `it` from the state x into y, their reachability, and
-    // publication into exchange buffer it&1; pend: some slip of this thread
-    // leaves its well (or is NaN), so that the commit of the step walks and
-    // checks only then
+    // slips of step `it` from the state x into y, and publication into
+    // exchange buffer it&1; pend: some slip of this thread leaves its well (or
+    // is NaN), so that the commit of the step walks only then. Without
+    // INLINE_REFILL their reachability as well (rmask, s_refill).
     int pend = 0;
+    uint32_t rmask = 0;
     auto prepare = [&](int it, const double(&x)[PPT], double(&y)[PPT]) {
         const int b = it & 1;
         int out = 0;
@@ -169,20 +171,25 @@ __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views
             out |= !(yl[i] <= y[i] && y[i] < yr[i]);
         }
         pend = out;
-        if (out) { // rare: some slip leaves its well
-            int refill = 0;
+        if constexpr (!INLINE_REFILL) {
+            rmask = 0;
+            if (out) { // rare: some slip leaves its well
+                // opaque copies: the addresses and comparisons of this rare
+                // path stay in it instead of being evaluated for every step
+                int64_t bq = base;
+                __asm__ volatile("" : "+v"(bq));
 #pragma unroll
-            for (int i = 0; i < PPT; ++i) {
-                // opaque copy: the comparisons of this rare path stay in it
-                // instead of being evaluated for every step
-                double z = y[i];
-                __asm__ volatile("" : "+v"(z));
-                if (!(yl[i] <= z && z < yr[i]) && __builtin_isfinite(z)) {
-                    refill |= !reachable(Y + (base + i) * nch, jl[i], yl[i], yr[i], z, jmin, jmax);
+                for (int i = 0; i < PPT; ++i) {
+                    double z = y[i];
+                    __asm__ volatile("" : "+v"(z));
+                    if (!(yl[i] <= z && z < yr[i]) && __builtin_isfinite(z) &&
+                        !reachable(Y + (bq + i) * nch, jl[i], yl[i], yr[i], z, jmin, jmax)) {
+                        rmask |= 1u << i;
+                    }
                 }
-            }
-            if (refill) {
-                s_refill[b] = it;
+                if (rmask) {
+                    s_refill[b] = it;
+                }
             }
         }
         publish(y, b);
@@ -208,6 +215,7 @@ __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views
     };
 
     int32_t status = ST_RUNNING;
+    int refilled = 0;
 
     // step `it` with the prepared slips in x (the previous state in y, which
     // receives the slips of step it+1); false if the run stops before it
@@ -222,9 +230,11 @@ __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views
         if (it > limit) {
             return false;
         }
-        if (uniform_i(s_refill[b]) == it) {
-            status = ST_REFILL;
-            return false;
+        if constexpr (!INLINE_REFILL) {
+            if (uniform_i(s_refill[b]) == it) {
+                status = ST_REFILL;
+                return false;
+            }
         }
 
         inc += 1;
@@ -270,16 +280,19 @@ __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views
         }
 
         // commit: the slips in x are the state now; walk to their wells
-        // (reachable: checked when they were prepared; a non-finite slip
-        // keeps its well)
+        uint32_t need = 0;
         if (pend) { // rare
             int nanf = 0;
+            // opaque copy of the first index: the window addresses of this
+            // rare path are computed in it, not kept live through the loop
+            int64_t bq = base;
+            __asm__ volatile("" : "+v"(bq));
 #pragma unroll
             for (int i = 0; i < PPT; ++i) {
                 const double z = x[i];
                 nanf |= __builtin_isnan(z);
                 if (!(yl[i] <= z && z < yr[i])) {
-                    const double* row = Y + (base + i) * nch;
+                    const double* row = Y + (bq + i) * nch;
                     int32_t j = jl[i];
                     double lo = yl[i], hi = yr[i];
                     while (z >= hi && j < jmax) {
@@ -298,11 +311,36 @@ __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views
                         yr[i] = hi;
                         ym[i] = 0.5 * (lo + hi);
                     }
+                    else if (INLINE_REFILL && __builtin_isfinite(z)) {
+                        need |= 1u << i;
+                    }
                 }
             }
             if (nanf) {
                 s_nan[b] = it;
             }
+        }
+        // windows that have to move (rare): one particle at a time by the
+        // whole wavefront, the other wavefronts do not wait for it
+        if (INLINE_REFILL && __builtin_expect(__any(need != 0), 0)) {
+#pragma unroll
+            for (int i = 0; i < PPT; ++i) {
+                uint64_t lanes = __ballot((need >> i) & 1u);
+                while (lanes) {
+                    const int src = __builtin_ctzll(lanes);
+                    lanes &= lanes - 1;
+                    const double z = lane_d(x[i], src);
+                    const int64_t p = ((int64_t)(t & ~63) + src) * PPT + i;
+                    const WellAt w = refill_one(&S, p, z, __builtin_amdgcn_readlane(jl[i], src));
+                    if ((t & 63) == src) {
+                        jl[i] = w.j;
+                        yl[i] = w.lo;
+                        yr[i] = w.hi;
+                        ym[i] = 0.5 * (w.lo + w.hi);
+                    }
+                }
+            }
+            refilled = 1;
         }
 
         // the reference's three velocity / acceleration passes (detail.h:1552-1565)
@@ -346,7 +384,7 @@ __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views
     // state and forces of the final configuration (slips in x, `done` steps
     // taken); its slips are in exchange buffer done&1 (published before step
     // `done`, or initially)
-    auto finish = [&](const double(&x)[PPT], int done) {
+    auto finish = [&](const double(&x)[PPT], int done) -> int32_t {
         if (status == ST_RUNNING) {
             status = ST_BUDGET;
         }
@@ -359,7 +397,7 @@ __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views
                 S.v[p] = v[i];
                 S.a[p] = a[i];
                 L.jloc[p] = jl[i];
-                if (status != ST_NAN) {
+                if (status != ST_NAN && status != ST_REFILL) {
                     const double fi = interaction(i, fb, x);
                     const double fp = potential_force_mid<POT>(S, x[i], yl[i], yr[i], ym[i]);
                     const double ff = kf * (uf - x[i]);
@@ -375,6 +413,9 @@ __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views
                 }
             }
         }
+        if (refilled) {
+            rs->refilled = 1;
+        }
         if (t == 0) {
             rs->inc = inc;
             rs->u_frame = uf;
@@ -383,6 +424,9 @@ __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views
             rs->rng_state = rng;
             rs->min_next = min_next;
         }
+        launch_done += done;
+        refill_mask = rmask;
+        return status;
     };
 
     // the current slips into buffer 0 (forces of the final state when no step
@@ -391,12 +435,48 @@ __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views
     prepare(1, sa, sb);
     for (int it = 1;; it += 2) {
         if (!step(it, sb, sa)) {
-            finish(sa, it - 1);
-            return;
+            return finish(sa, it - 1);
         }
         if (!step(it + 1, sa, sb)) {
-            finish(sb, it);
-            return;
+            return finish(sb, it);
+        }
+    }
+}
+
+// Windows that have to move are handled inside the launch: variants of up to
+// 512 threads (256 registers) call the refill from the commit of the step, by
+// the wavefronts that need it; in variants of 1024 threads (128 registers)
+// that call would spill the step loop's registers (4 x 1024 on 1024 chains of
+// 4096: 34 ms instead of 5.1 ms per 1000 steps), so with up to 2 particles per
+// thread the entry ends, refills from memory and starts again. With 4 the
+// loop around the entry alone costs 14% (5.8 ms), so there the launch ends and
+// the host relaunches it after k_refill. Sliding chains (256 x 1999, windows
+// of 100, 4 x 512; a window moves somewhere in nearly every step): 13 ms per
+// 1000 steps, against 273 ms with a relaunch each time.
+template <int POT, int INT, int EXT, int PPT, int MAXT, bool UNIT, bool FULL = false>
+__global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views, RunArgs ra)
+{
+    static_assert(is_chain<INT>(), "k_flow handles chains");
+    const RunState* const rs = views[blockIdx.x].rs;
+    if (rs->status != ST_RUNNING && rs->status != ST_BUDGET) {
+        return;
+    }
+    int64_t launch_done = 0;
+    uint32_t rmask = 0;
+    if constexpr (MAXT <= 512) {
+        flow_entry<POT, INT, EXT, PPT, UNIT, FULL, true>(views, ra, launch_done, rmask);
+    }
+    else if constexpr (PPT > 2) {
+        flow_entry<POT, INT, EXT, PPT, UNIT, FULL, false>(views, ra, launch_done, rmask);
+    }
+    else {
+        while (flow_entry<POT, INT, EXT, PPT, UNIT, FULL, false>(views, ra, launch_done, rmask) == ST_REFILL) {
+            __syncthreads(); // the state of every lane's particles is in memory
+            if (rmask) {
+                views[blockIdx.x].rs->refilled = 1;
+            }
+            refill_wave(views, (int64_t)threadIdx.x * PPT, 0, rmask);
+            __syncthreads();
         }
     }
 }

@@ -131,12 +131,23 @@ __device__ __noinline__ int32_t chunk_align_slow(const Landscape& L, int64_t p, 
     return chunk_align_slow_inl(L, p, u, j0);
 }
 
+// Lane `src`'s value (src uniform), in every lane.
+__device__ __forceinline__ double lane_d(double x, int src)
+{
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, src);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), src);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
 // Wavefront-cooperative form of chunk_shift_to for a window that starts at
 // `s` with pcg32 states (stb, ste), called by all 64 lanes with the same
 // arguments: lane l draws the increments l, l + 64, ... in parallel (each from
 // the stream state advanced to it), and the running sum is then taken in the
 // sequential order, so the row is bit-identical to chunk_shift_to's. Writes
 // the row and updates stb, ste; the caller stores start and the states.
+// (Both directions share one body: the draw's code, with every distribution's
+// transform, is by far its largest part.)
 __device__ __forceinline__ void chunk_shift_wave(const Landscape& L, int64_t p, int64_t s, int64_t ns, uint64_t& stb,
                                                  uint64_t& ste)
 {
@@ -144,75 +155,49 @@ __device__ __forceinline__ void chunk_shift_wave(const Landscape& L, int64_t p, 
     const int64_t n = L.nchunk;
     double* y = L.y + p * n;
     const int64_t d = ns - s;
-    if (d == 0) {
-        return;
-    }
-    if (d > 0) {
-        double val = y[n - 1];
-        if (d < n) {
-            // y[k] = y[k + d]; in each block of 64 the loads precede the stores,
-            // and later blocks read above everything written before
-            for (int64_t c = 0; c < n - d; c += 64) {
-                const int64_t k = c + lane;
-                const double x = k < n - d ? y[k + d] : 0.0;
-                if (k < n - d) {
-                    y[k] = x;
-                }
-            }
-        }
-        for (int64_t c = 0; c < d; c += 64) {
-            const int64_t k = c + lane; // increment of global index s + n + k
-            double dk = 0.0;
-            if (k < d) {
-                uint64_t st = pcg_advance(ste, L.inc, k);
-                dk = draw_increment(L, st);
-            }
-            const int nc = (int)(d - c < 64 ? d - c : 64);
-            double mine = 0.0;
-            for (int q = 0; q < nc; ++q) {
-                val = val + __shfl(dk, q, 64);
-                if (q == lane) {
-                    mine = val;
-                }
-            }
-            const int64_t g = s + n + k;
-            if (k < d && g >= ns) {
-                y[g - ns] = mine;
-            }
+    const bool fwd = d > 0;
+    const int64_t e = fwd ? d : -d; // wells to draw
+    // the running sum starts from the window's end on the side it moves to
+    double val = fwd ? y[n - 1] : y[0];
+    // wells kept: forward y[k] = y[k + e] upwards, backward y[k] = y[k - e]
+    // downwards; in each block of 64 the loads precede the stores, and later
+    // blocks read beyond everything written before
+    for (int64_t c = 0; c < n - e; c += 64) {
+        const int64_t q = c + lane;
+        const int64_t to = fwd ? q : n - 1 - q;
+        const int64_t from = fwd ? to + e : to - e;
+        const bool in = q < n - e;
+        const double x = in ? y[from] : 0.0;
+        if (in) {
+            y[to] = x;
         }
     }
-    else {
-        const int64_t e = -d;
-        double val = y[0];
-        if (e < n) {
-            // y[k] = y[k - e] from the top down, mirrored
-            for (int64_t c = n - 1; c >= e; c -= 64) {
-                const int64_t k = c - lane;
-                const double x = k >= e ? y[k - e] : 0.0;
-                if (k >= e) {
-                    y[k] = x;
-                }
-            }
+    const uint64_t st0 = fwd ? ste : stb;
+    for (int64_t c = 0; c < e; c += 64) {
+        // forward: the increment of global index s + n + k; backward: the draw
+        // of global index s - k, from the state before it
+        const int64_t k = c + lane;
+        double dk = 0.0;
+        if (k < e) {
+            uint64_t st = pcg_advance(st0, L.inc, fwd ? k : -(k + 1));
+            dk = draw_increment(L, st);
         }
-        for (int64_t c = 0; c < e; c += 64) {
-            const int64_t k = c + lane; // the draw of global index s - k, from s - k - 1
-            double dk = 0.0;
-            if (k < e) {
-                uint64_t st = pcg_advance(stb, L.inc, -(k + 1));
-                dk = draw_increment(L, st);
-            }
-            const int nc = (int)(e - c < 64 ? e - c : 64);
-            double mine = 0.0;
-            for (int q = 0; q < nc; ++q) {
-                val = val - __shfl(dk, q, 64);
-                if (q == lane) {
-                    mine = val;
-                }
-            }
-            const int64_t o = e - k - 1; // local index of global s - k - 1
-            if (k < e && o < n) {
-                y[o] = mine;
-            }
+        if (!fwd) {
+            dk = -dk; // val - dk
+        }
+        const int nc = (int)(e - c < 64 ? e - c : 64);
+        double mine = 0.0;
+#pragma unroll 4
+        for (int q = 0; q < nc; ++q) {
+            val = val + lane_d(dk, q);
+            mine = q == lane ? val : mine;
+        }
+        // forward: global s + n + k at local n - e + k; backward: global
+        // s - k - 1 at local e - k - 1 (of a jump beyond the window only the
+        // part inside it is kept)
+        const int64_t o = fwd ? n - e + k : e - k - 1;
+        if (k < e && o >= 0 && o < n) {
+            y[o] = mine;
         }
     }
     stb = pcg_advance(stb, L.inc, d);
@@ -222,71 +207,70 @@ __device__ __forceinline__ void chunk_shift_wave(const Landscape& L, int64_t p, 
 // Wavefront-cooperative chunk_align_slow: all 64 lanes call it with the same
 // particle p, slip u and local index j0 and follow the same control flow;
 // the window shifts are drawn by all lanes (chunk_shift_wave) and lane 0
-// stores the new start, states and index. Returns the new local index.
-__device__ __forceinline__ int32_t chunk_align_wave(const Landscape& L, int64_t p, double u, int32_t j0)
+// stores the new start, states and index. Returns the new local index and
+// the bounds of its well.
+__device__ __forceinline__ int32_t chunk_align_wave(const Landscape& L, int64_t p, double u, int32_t j0, double& lo,
+                                                    double& hi)
 {
-    if (!__builtin_isfinite(u)) {
-        return j0;
-    }
     const int64_t n = L.nchunk;
     const double* y = L.y + p * n;
+    if (!__builtin_isfinite(u)) {
+        lo = y[j0];
+        hi = y[j0 + 1];
+        return j0;
+    }
     const int64_t b = L.buffer, m = L.margin;
     int64_t start = L.start[p];
     uint64_t stb = L.st_begin[p], ste = L.st_end[p];
-    auto shift = [&](int64_t ns) {
-        chunk_shift_wave(L, p, start, ns, stb, ste);
-        start = ns;
-        __threadfence_block(); // the row written by all lanes is read back below
-    };
     int64_t j = j0;
-    int64_t res = -1;
     int64_t budget = MAX_SEARCH_WELLS;
-    while (!(u < y[n - 1])) {
-        if (budget <= 0) {
-            res = n - 2;
-            break;
+    for (bool found = false;;) {
+        int64_t ns;
+        const bool above = !(u < y[n - 1]);
+        if (above || u < y[0]) { // beyond the window: jump, or give up
+            found = budget <= 0;
+            ns = found ? start : (above ? start + (n - 1 - m) : start - (n - 1 - m));
+            j = above ? n - 2 : 0;
+            budget -= n - 1 - m;
         }
-        budget -= n - 1 - m;
-        shift(start + (n - 1 - m));
-        j = m;
-    }
-    if (res < 0) {
-        while (u < y[0]) {
-            if (budget <= 0) {
-                res = 0;
+        else {
+            j = j < 0 ? 0 : (j > n - 2 ? n - 2 : j);
+            while (j < n - 2 && u >= y[j + 1]) {
+                ++j;
+            }
+            while (j > 0 && u < y[j]) {
+                --j;
+            }
+            found = true;
+            ns = j < b || j > n - 2 - b ? start + j - m : start;
+        }
+        if (found) {
+            lo = y[j];
+            hi = y[j + 1];
+            if (ns == start) {
                 break;
             }
-            budget -= n - 1 - m;
-            shift(start - (n - 1 - m));
-            j = n - 1 - m;
         }
-    }
-    if (res < 0) {
-        if (j < 0) {
-            j = 0;
-        }
-        if (j > n - 2) {
-            j = n - 2;
-        }
-        while (j < n - 2 && u >= y[j + 1]) {
-            ++j;
-        }
-        while (j > 0 && u < y[j]) {
-            --j;
-        }
-        if (j < b || j > n - 2 - b) {
-            shift(start + j - m);
+        const int64_t from = start;
+        chunk_shift_wave(L, p, start, ns, stb, ste);
+        start = ns;
+        if (found) { // the well keeps its bounds, at the margin
             j = m;
+            break;
         }
-        res = j;
+        j = ns > from ? m : n - 1 - m;
+        // the row written by all lanes is read back by each (a wavefront's
+        // memory operations take effect in its program order)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     if ((threadIdx.x & 63) == 0) {
         L.start[p] = start;
         L.st_begin[p] = stb;
         L.st_end[p] = ste;
-        L.jloc[p] = (int32_t)res;
+        L.jloc[p] = (int32_t)j;
     }
-    return (int32_t)res;
+    return (int32_t)j;
 }
 
 // Align particle p (registers yl, yr, j hold its current well). Returns the

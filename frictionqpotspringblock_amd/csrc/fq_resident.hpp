@@ -200,6 +200,20 @@ FQ_HD size_t resident_lds_bytes(int64_t N, int threads)
     }
 }
 
+// Align particle p to slip z (outside its window's safe zone) from inside a
+// step loop: called by all lanes of a wavefront with the same arguments;
+// returns the local well index and its bounds.
+struct WellAt {
+    double lo, hi;
+    int32_t j;
+};
+__device__ __noinline__ WellAt refill_one(const SysView* S, int64_t p, double z, int32_t j)
+{
+    WellAt w;
+    w.j = chunk_align_wave(S->ls, p, z, j, w.lo, w.hi);
+    return w;
+}
+
 // Landscape refill inside a resident launch: particle base + i of a lane
 // with bit i of `mask` set left the window's safe zone; it is aligned to the
 // slip of the pending step, u + dt v + dt^2/2 a, or to u itself (at_u, a
@@ -231,7 +245,7 @@ __device__ __noinline__ void refill_wave(const SysView* __restrict__ views, int6
             m &= m - 1;
             const int64_t p = b0 + i;
             const double x = at_u ? vu[p] : vu[p] + dt * vv[p] + c2 * va[p];
-            chunk_align_wave(L, p, x, vj[p]);
+            refill_one(&S, p, x, vj[p]);
         }
     }
 }
@@ -963,6 +977,9 @@ __device__ __forceinline__ void resident_body(const SysView* __restrict__ views,
         // refill from the written-back state, then reload it: the LDS of this
         // entry must no longer be read when the next one publishes
         __syncthreads(); // the state of every lane's particles is in memory
+        if (rmask) {
+            rs->refilled = 1;
+        }
         refill_wave(views, base, refill_u, rmask);
         refill_u = 0;
         __syncthreads();

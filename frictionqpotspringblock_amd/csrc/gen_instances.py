@@ -1,4 +1,4 @@
-"""Generate the resident-kernel instantiation units fq_res_<unit>.hip and the
+"""Generate the resident-kernel instantiation units fq_res_<unit>_<part>.hip and the
 header fq_res_units.hpp that declares them.
 
 Each unit instantiates, for its (potential, interaction, forcing) classes and
@@ -118,22 +118,11 @@ def launcher(name, kernel, pot, ints, chains_only):
     return out
 
 
-def unit(name, pot, ints):
-    out = [HEADER, '#include "fq_flow.hpp"', '#include "fq_launch.hpp"', '#include "fq_quasi.hpp"',
-           '#include "fq_resident.hpp"', "",
-           "namespace fq {", ""]
-    out += launcher(name, "resident", pot, ints, False)
-    out.append("")
-    out += launcher(name, "flow", pot, ints, True)
-    out.append("")
-    out += quasi_launcher(name, pot, ints)
-    out.append("")
-    out.append(f"int resident_variants_{name}(int inter, int ext, int* ppt, int* maxt, int cap)")
-    out.append("{")
-    out.append("    int n = 0;")
-    for it, exts, variants in ints:
+def variants(name, ints):
+    out = [f"int resident_variants_{name}(int inter, int ext, int* ppt, int* maxt, int cap)", "{", "    int n = 0;"]
+    for it, exts, shapes in ints:
         for e in exts:
-            arr = ", ".join(f"{{{p}, {m}}}" for p, m in variants)
+            arr = ", ".join(f"{{{p}, {m}}}" for p, m in shapes)
             out.append(f"    if (inter == {it} && ext == {e}) {{")
             out.append(f"        static const int v[][2] = {{{arr}}};")
             out.append("        for (const auto& x : v) {")
@@ -145,11 +134,22 @@ def unit(name, pot, ints):
             out.append("        }")
             out.append("        return n;")
             out.append("    }")
-    out.append("    return 0;")
-    out.append("}")
-    out.append("")
-    out.append("} // namespace fq")
-    return "\n".join(out) + "\n"
+    out += ["    return 0;", "}"]
+    return out
+
+
+def unit(name, pot, ints, part):
+    """One source of a unit: its k_resident (and the table of variants), its
+    k_flow or its quasistatic kernels (separate sources: they compile in
+    parallel)."""
+    body = {
+        "resident": lambda: launcher(name, "resident", pot, ints, False) + [""] + variants(name, ints),
+        "flow": lambda: launcher(name, "flow", pot, ints, True),
+        "quasi": lambda: quasi_launcher(name, pot, ints),
+    }[part]()
+    out = [HEADER, '#include "fq_flow.hpp"', '#include "fq_launch.hpp"', '#include "fq_quasi.hpp"',
+           '#include "fq_resident.hpp"', "", "namespace fq {", ""]
+    return "\n".join(out + body + ["", "} // namespace fq"]) + "\n"
 
 
 def header():
@@ -185,9 +185,10 @@ def generate(directory):
     unchanged are left alone); returns the unit file names in build order."""
     names = []
     for name, (pot, ints) in UNITS.items():
-        fname = f"fq_res_{name}.hip"
-        _write_if_changed(os.path.join(directory, fname), unit(name, pot, ints))
-        names.append(fname)
+        for part in ("resident", "flow", "quasi"):
+            fname = f"fq_res_{name}_{part}.hip"
+            _write_if_changed(os.path.join(directory, fname), unit(name, pot, ints, part))
+            names.append(fname)
     _write_if_changed(os.path.join(directory, "fq_res_units.hpp"), header())
     return names
 

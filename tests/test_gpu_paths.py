@@ -1,0 +1,85 @@
+"""Kernel paths chosen by size, class or state, against the CPU oracle bit for
+bit: the windows that move inside a launch, and the rules that route a call."""
+
+import numpy as np
+import pytest
+
+from oracle import pyoracle
+from tests import protocols as P
+
+pytestmark = pytest.mark.gpu
+
+
+def _kw(N, **extra):
+    kw = dict(m=1.0, eta=2.0 * np.sqrt(3.0) / 10.0, mu=1.0, k_interactions=1.0, k_frame=1.0 / N, dt=0.1, shape=[N],
+              seed=5, distribution="weibull", parameters=[2.0, 1.0, 0.0], offset=-20.0, nchunk=60)
+    kw.update(extra)
+    return kw
+
+
+def _sliding(v_frame, N, **extra):
+    """A batch of two chains and the oracle's, loaded so that they slide."""
+    from frictionqpotspringblock_amd.batch import Batch
+
+    kw = _kw(N, **extra)
+    b = Batch(2, seed_stride=N, potential="Cuspy", interactions="Laplace1d", **kw)
+    ref = [pyoracle.Line1d.System_Cuspy_Laplace(**dict(kw, seed=kw["seed"] + r * N)) for r in range(2)]
+    load = 0.5 if v_frame > 0 else -0.5
+    b.advanceToFixedForce(load, allow_plastic=True)
+    for s in ref:
+        s.advanceToFixedForce(load, allow_plastic=True)
+    return b, ref
+
+
+def _same(b, ref):
+    for r, s in enumerate(ref):
+        assert np.array_equal(b.u[r], s.u)
+        assert np.array_equal(b.v[r], s.v)
+        assert np.array_equal(b.f[r], s.f)
+        assert np.array_equal(b.index_at_align[r], s.chunk.index_at_align)
+        assert np.array_equal(b._get_state("start").reshape(2, -1)[r], s.chunk.start)
+        assert np.array_equal(b._get_state("y").reshape(2, b.size, -1)[r], s.chunk.data)
+
+
+@pytest.mark.parametrize("v_frame", [0.5, -0.5])
+@pytest.mark.parametrize("ppt,threads,N", [(1, 64, 3), (1, 128, 65), (2, 64, 127), (4, 64, 256), (8, 64, 509), (4, 1024, 4096)])
+def test_windows_move_inside_flow(ppt, threads, N, v_frame):
+    """flowSteps of sliding chains: every window moves several times inside
+    the launch (forward and backward), at each launch shape, with launches
+    that end between any two steps."""
+    b, ref = _sliding(v_frame, N)
+    b.set_launch(ppt, threads)
+    n = 300 if N < 4096 else 120
+    i0 = b.index_at_align
+    b.flowSteps(n, v_frame, block=37)
+    for s in ref:
+        s.flowSteps(n, v_frame)
+    assert np.abs(b.index_at_align - i0).max() > (15 if N < 4096 else 5)
+    _same(b, ref)
+
+
+def test_window_jumps_inside_flow():
+    """Slips that leave the window altogether (fast particles) and slips that
+    stay where they are (a particle at rest next to them)."""
+    b, ref = _sliding(0.5, 64, nchunk=12)
+    v = np.zeros(64)
+    v[3], v[40], v[41] = 400.0, -350.0, 90.0
+    b.v = np.broadcast_to(v, [2, 64])
+    for s in ref:
+        s.v = v
+    b.flowSteps(40, 0.5)
+    for s in ref:
+        s.flowSteps(40, 0.5)
+    _same(b, ref)
+
+
+def test_adjoint_refuses_moved_windows():
+    """A window moved inside a launch is noticed by the adjoint forward pass."""
+    import torch
+
+    from frictionqpotspringblock_amd import adjoint as A
+
+    b, _ = _sliding(0.5, 64)
+    z = torch.zeros((2, 64), dtype=torch.float64, device="cuda")
+    with pytest.raises(RuntimeError, match="left the landscape window"):
+        A.run(b, 300, 50, z, z + 20.0, z, A.parameters(b), flow=True, v_frame=0.5)
