@@ -242,6 +242,8 @@ struct Group {
     ~Group()
     {
         if (stream) {
+    int lr_log2 = 0; // product by transforms of 2^lr_log2 points (0: k_lr_gemm), with their tables
+    double *lr_tw = nullptr, *lr_sd = nullptr;
             (void)hipStreamSynchronize(stream);
         }
         dfree(u);
@@ -283,6 +285,8 @@ struct Group {
         }
         dfree(tiles);
         dfree(tile_first);
+        dfree(lr_tw);
+        dfree(lr_sd);
         dfree(tile_part);
         dfree(tile_flag);
         dfree(tile_part_k);
@@ -1104,6 +1108,68 @@ struct Group {
             throw Error("unknown long-range method");
         }
         if (method == FQSB_LR_MATRIX && pot != FQSB_POT_CUSPY) {
+    // Tables of the transforms (fq_lrfft.hpp) in extended precision: the
+    // roots of unity, and the spectrum of the kernel (real: the kernel is
+    // even) split for the frequency product.
+    void lr_tables()
+    {
+        using real = long double;
+        const size_t L = (size_t)1 << lr_log2, M = 2 * L;
+        std::vector<real> cs(M), sn(M); // exp(-2 pi i k / M)
+        const real step = -2 * std::acos((real)-1) / (real)M;
+        for (size_t k = 0; k < M; ++k) {
+            cs[k] = std::cos(step * (real)k);
+            sn[k] = std::sin(step * (real)k);
+        }
+        std::vector<double> pr((size_t)N);
+        d2h(pr.data(), pref, (size_t)N);
+        // the first column of the (embedding) circulant, and its transform by
+        // the decimation in time
+        std::vector<real> re(M, 0), im(M, 0);
+        for (int64_t d = 1; d < N; ++d) {
+            const real g = pr[(size_t)(d > lr_m ? N - d : d)];
+            re[(size_t)d] = g;
+            re[M - (size_t)d] = g;
+        }
+        for (size_t i = 1, j = 0; i < M; ++i) { // bit reversal
+            size_t bit = M >> 1;
+            for (; j & bit; bit >>= 1) {
+                j ^= bit;
+            }
+            j ^= bit;
+            if (i < j) {
+                std::swap(re[i], re[j]);
+                std::swap(im[i], im[j]);
+            }
+        }
+        for (size_t len = 2; len <= M; len <<= 1) {
+            for (size_t i = 0; i < M; i += len) {
+                for (size_t k = 0; k < len / 2; ++k) {
+                    const real c = cs[k * (M / len)], s = sn[k * (M / len)];
+                    const size_t a = i + k, b = a + len / 2;
+                    const real x = re[b] * c - im[b] * s, y = re[b] * s + im[b] * c;
+                    re[b] = re[a] - x;
+                    im[b] = im[a] - y;
+                    re[a] += x;
+                    im[a] += y;
+                }
+            }
+        }
+        std::vector<double> tw(2 * L), sd(3 * L);
+        for (size_t k = 0; k < L; ++k) {
+            tw[2 * k] = (double)cs[2 * k];
+            tw[2 * k + 1] = (double)sn[2 * k];
+            const real s = (re[k] + re[L - k]) / (2 * (real)L), d = (re[k] - re[L - k]) / (2 * (real)L);
+            sd[3 * k] = (double)s;
+            sd[3 * k + 1] = (double)(d * cs[k]);
+            sd[3 * k + 2] = (double)(d * sn[k]);
+        }
+        lr_tw = dalloc<double>(tw.size());
+        lr_sd = dalloc<double>(sd.size());
+        h2d(lr_tw, tw.data(), tw.size());
+        h2d(lr_sd, sd.data(), sd.size());
+    }
+
             throw Error("the matrix form of long-range interactions needs the Cuspy potential");
         }
         if (method == FQSB_LR_MATRIX && !uniform) {
@@ -1112,17 +1178,27 @@ struct Group {
         if (method == FQSB_LR_MATRIX && !lr_un) {
             const size_t RN = (size_t)(R * N);
             lr_un = dalloc<double>(RN);
-            // split the summation index so that one product launch has about
-            // 1024 workgroups (4 per CU, the occupancy that registers and LDS
-            // allow), each range at least 8 K-blocks long; FQSB_LR_SPLIT
-            // overrides the count (tuning)
-            const int64_t kb = fq::lr_split_blocks();
-            const int64_t nkb = (N + kb - 1) / kb;
-            const int64_t tiles = ((N + 127) / 128) * ((R + 63) / 64);
-            const int64_t cap = std::max<int64_t>(1, std::min<int64_t>(8, nkb / 8));
-            int64_t ns = std::max<int64_t>(1, std::min<int64_t>(cap, (1024 + tiles - 1) / tiles));
-            if (const char* e = std::getenv("FQSB_LR_SPLIT")) {
-                ns = std::max<int64_t>(1, std::min<int64_t>(cap, std::atoll(e)));
+            // chains of 257 to 8192 particles (16384 for powers of two) by
+            // transforms in LDS (256 x 8192: 25 us instead of the 506 us of the
+            // matrix product, and a smaller error, fq_lrfft.hpp)
+            lr_log2 = fq::lr_fft_log2(N);
+            int64_t ns = 1;
+            if (lr_log2) {
+                lr_tables();
+            }
+            else {
+                // split the summation index so that one product launch has about
+                // 1024 workgroups (4 per CU, the occupancy that registers and LDS
+                // allow), each range at least 8 K-blocks long; FQSB_LR_SPLIT
+                // overrides the count (tuning)
+                const int64_t kb = fq::lr_split_blocks();
+                const int64_t nkb = (N + kb - 1) / kb;
+                const int64_t tiles = ((N + 127) / 128) * ((R + 63) / 64);
+                const int64_t cap = std::max<int64_t>(1, std::min<int64_t>(8, nkb / 8));
+                ns = std::max<int64_t>(1, std::min<int64_t>(cap, (1024 + tiles - 1) / tiles));
+                if (const char* e = std::getenv("FQSB_LR_SPLIT")) {
+                    ns = std::max<int64_t>(1, std::min<int64_t>(cap, std::atoll(e)));
+                }
             }
             lr_nsplit = (int)ns;
             lr_part = dalloc<double>(RN * (size_t)ns);
@@ -1178,7 +1254,8 @@ struct Group {
                 if (probe) {
                     HIPC(hipEventRecord(evg0, stream));
                 }
-                HIPC(fq::launch_lr_gemm(pref, lb, lr_m, stream));
+                HIPC(lr_log2 ? fq::launch_lr_fft(lr_log2, lr_tw, lr_sd, lb, stream)
+                             : fq::launch_lr_gemm(pref, lb, lr_m, stream));
                 if (probe) {
                     HIPC(hipEventRecord(evg1, stream));
                 }

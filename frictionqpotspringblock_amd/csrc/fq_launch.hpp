@@ -108,6 +108,8 @@ inline size_t quasi_lds(int inter, int64_t N, int ppt, int maxt, int threads)
 // batched long range (fq_longrange.hip)
 int lr_split_blocks(); // summation ranges are multiples of this many indices
 hipError_t launch_lr_gemm(const double* pref, const LrBuffers& lb, int64_t lr_m, hipStream_t stream);
+int lr_fft_log2(int64_t N); // log2 of the transform's complex points (0: use launch_lr_gemm)
+hipError_t launch_lr_fft(int log2_points, const double* tw, const double* sd, const LrBuffers& lb, hipStream_t stream);
 hipError_t launch_lr_elem(int ext, const SysView* views, const LrBuffers& lb, const RunArgs& ra, hipStream_t stream);
 hipError_t launch_lr_prologue(const SysView* views, const LrBuffers& lb, hipStream_t stream);
 
