@@ -117,7 +117,14 @@ constexpr uint64_t STEP_BLOCK = 1u << 16;
 // LR_TILE_PARTICLES particles (one per thread), each tile holding every slip
 // of the chain in LDS
 constexpr int64_t LR_RESIDENT_MAX = 2048;
+// ... and, while their tiles of one wavefront fit two per CU, above this size:
+// timeSteps, flowSteps and minimise over tiles, everything else resident. A
+// step of one chain takes (resident / tiles, us): N = 448 13.6 / 11.6, 576
+// 22 / 14, 1000 56 / 20, 2000 323 / 36; below 512 a minimise loses what its
+// steps gain to the launches of the last block of steps.
+constexpr int64_t LR_TILE_MIN = 512;
 constexpr int64_t LR_TILE_PARTICLES = 256;
+constexpr int64_t LR_TILE_WAVE = 64;
 // largest chain of the resident no-passing kernel (16 particles per thread on
 // 512 threads); longer chains sweep over tiles
 constexpr int64_t NOPASSING_RESIDENT_MAX = 8192;
@@ -165,7 +172,8 @@ struct Group {
     float adj_record_ms = 0.0f, adj_reverse_ms = 0.0f; // per launch, last backward
     int pot = 0, inter = 0, ext = 0, minim = 0;
     double *u = nullptr, *v = nullptr, *a = nullptr, *f = nullptr, *f_pot = nullptr, *f_int = nullptr,
-           *f_frame = nullptr, *f_damp = nullptr, *f_th = nullptr, *pref = nullptr, *y = nullptr;
+           *f_frame = nullptr, *f_damp = nullptr, *f_th = nullptr, *pref = nullptr, *prefx = nullptr,
+           *y = nullptr;
     int64_t *start = nullptr, *i_ref = nullptr, *next = nullptr, *dinc = nullptr;
     int32_t* jloc = nullptr;
     uint64_t *st_begin = nullptr, *st_end = nullptr;
@@ -234,6 +242,8 @@ struct Group {
     float qs_ms = 0.0f;
     int64_t qs_launches = 0;
     double *lr_un = nullptr, *lr_part = nullptr, *lr_yl = nullptr, *lr_yr = nullptr;
+    int lr_log2 = 0; // product by transforms of 2^lr_log2 points (0: k_lr_gemm), with their tables
+    double *lr_tw = nullptr, *lr_sd = nullptr;
 
     Group() = default;
     Group(const Group&) = delete;
@@ -242,8 +252,6 @@ struct Group {
     ~Group()
     {
         if (stream) {
-    int lr_log2 = 0; // product by transforms of 2^lr_log2 points (0: k_lr_gemm), with their tables
-    double *lr_tw = nullptr, *lr_sd = nullptr;
             (void)hipStreamSynchronize(stream);
         }
         dfree(u);
@@ -256,6 +264,7 @@ struct Group {
         dfree(f_damp);
         dfree(f_th);
         dfree(pref);
+        dfree(prefx);
         dfree(y);
         dfree(start);
         dfree(i_ref);
@@ -276,6 +285,8 @@ struct Group {
         dfree(jl2);
         dfree(lr_un);
         dfree(lr_part);
+        dfree(lr_tw);
+        dfree(lr_sd);
         free_adjoint();
         for (auto& tg : tile_graphs) {
             (void)hipGraphExecDestroy(tg.exec);
@@ -285,8 +296,6 @@ struct Group {
         }
         dfree(tiles);
         dfree(tile_first);
-        dfree(lr_tw);
-        dfree(lr_sd);
         dfree(tile_part);
         dfree(tile_flag);
         dfree(tile_part_k);
@@ -1099,15 +1108,6 @@ struct Group {
         }
     }
 
-    void set_lr_method(int method)
-    {
-        if (inter != FQSB_INT_LONGRANGE1D) {
-            throw Error("the systems have no long-range interactions");
-        }
-        if (method != FQSB_LR_EXACT && method != FQSB_LR_MATRIX) {
-            throw Error("unknown long-range method");
-        }
-        if (method == FQSB_LR_MATRIX && pot != FQSB_POT_CUSPY) {
     // Tables of the transforms (fq_lrfft.hpp) in extended precision: the
     // roots of unity, and the spectrum of the kernel (real: the kernel is
     // even) split for the frequency product.
@@ -1170,6 +1170,15 @@ struct Group {
         h2d(lr_sd, sd.data(), sd.size());
     }
 
+    void set_lr_method(int method)
+    {
+        if (inter != FQSB_INT_LONGRANGE1D) {
+            throw Error("the systems have no long-range interactions");
+        }
+        if (method != FQSB_LR_EXACT && method != FQSB_LR_MATRIX) {
+            throw Error("unknown long-range method");
+        }
+        if (method == FQSB_LR_MATRIX && pot != FQSB_POT_CUSPY) {
             throw Error("the matrix form of long-range interactions needs the Cuspy potential");
         }
         if (method == FQSB_LR_MATRIX && !uniform) {
@@ -1592,7 +1601,7 @@ struct Group {
         qs_launches = 0;
         try {
             set_iref_current();
-            const bool device = !streaming && minim == FQSB_MIN_INERTIAL &&
+            const bool device = !streaming && (!tiled || !own) && minim == FQSB_MIN_INERTIAL &&
                                 (!own || std::getenv("FQSB_HOST_QUASISTATIC") == nullptr);
             if (!device || !quasistatic_device(qa, tol, niter_tol, ms)) {
                 if (!own) {
@@ -1922,6 +1931,7 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
     }
     if (inter == FQSB_INT_LONGRANGE1D) { // LongRange1d ctor detail.h:829-844, per system
         g->pref = dalloc<double>(RN);
+        g->prefx = dalloc<double>(2 * RN);
         for (int64_t r = 0; r < R; ++r) {
             const fqsb_desc& d = ds[(size_t)r];
             const int64_t N = Ns[(size_t)r];
@@ -1930,6 +1940,13 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
                 pr[(size_t)dd] = d.k_interactions / std::pow((double)dd, d.alpha + 1.0);
             }
             g->h2d(g->pref + g->off[(size_t)r], pr.data(), (size_t)N);
+            // the same by the difference i - p of two particles
+            const int64_t half = (N - N % 2) / 2;
+            std::vector<double> px((size_t)(2 * N - 1), 0.0);
+            for (int64_t dd = 1; dd < N; ++dd) {
+                px[(size_t)(N - 1 + dd)] = px[(size_t)(N - 1 - dd)] = pr[(size_t)(dd > half ? N - dd : dd)];
+            }
+            g->h2d(g->prefx + 2 * g->off[(size_t)r], px.data(), px.size());
         }
         g->lr_m = (g->N - g->N % 2) / 2;
     }
@@ -1937,6 +1954,7 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
     // resident workgroup if the largest system fits one, else the streaming
     // path (FQSB_FORCE_STREAMING=1 selects the streaming path for every size;
     // FQSB_RESIDENT_MAX=n for systems above n particles)
+    bool lr_dual = false;
     if (g->minim != FQSB_MIN_OVERDAMPED) {
         const char* force = std::getenv("FQSB_FORCE_STREAMING");
         const char* rmax = std::getenv("FQSB_RESIDENT_MAX");
@@ -1958,6 +1976,16 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
         }
         catch (const Error&) {
             g->streaming = true;
+        }
+        // long-range chains that also fit a workgroup: tiles for the runs that
+        // have them
+        int64_t waves = 0;
+        for (const int64_t N : Ns) {
+            waves += (N + LR_TILE_WAVE - 1) / LR_TILE_WAVE;
+        }
+        lr_dual = !g->streaming && inter == FQSB_INT_LONGRANGE1D && g->N > LR_TILE_MIN && waves <= 2 * (int64_t)g->cus &&
+                  fq::tile_supported(g->pot, inter, g->ext);
+        if (g->streaming || lr_dual) {
             g->u2 = dalloc<double>(RN);
             g->v2 = dalloc<double>(RN);
             g->a2 = dalloc<double>(RN);
@@ -1971,12 +1999,18 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
 
     // tiles of the streaming systems (chains: runs of particles; lattices:
     // whole rows, at most rows - 2 per tile so that the halo rows are distinct)
-    if (g->streaming && fq::tile_supported(g->pot, inter, g->ext)) {
+    if ((g->streaming || lr_dual) && fq::tile_supported(g->pot, inter, g->ext)) {
         const char* nt = std::getenv("FQSB_NO_TILES");
         bool ok = !(nt && nt[0] == '1');
         std::vector<fq::TileDesc> tl;
         std::vector<int32_t> first((size_t)R + 1, 0);
         size_t lds = 0;
+        // long range: tiles of one wavefront while they fit two per CU
+        int64_t lr_tile = 0;
+        for (const int64_t N : Ns) {
+            lr_tile += (N + LR_TILE_WAVE - 1) / LR_TILE_WAVE;
+        }
+        lr_tile = lr_tile <= 2 * (int64_t)g->cus ? LR_TILE_WAVE : LR_TILE_PARTICLES;
         for (int64_t r = 0; r < R && ok; ++r) {
             const fqsb_desc& d = ds[(size_t)r];
             const int64_t N = Ns[(size_t)r];
@@ -1993,7 +2027,7 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
             }
             else {
                 ok = N >= 3;
-                step = lr ? LR_TILE_PARTICLES : 4096;
+                step = lr ? lr_tile : 4096;
             }
             first[(size_t)r] = (int32_t)tl.size();
             for (int64_t p0 = 0; ok && p0 < N; p0 += step) {
@@ -2002,8 +2036,9 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
                 td.p0 = p0;
                 td.p1 = std::min<int64_t>(N, p0 + step);
                 tl.push_back(td);
-                // LDS: the tile's slips and halo (long range: every slip of the system)
-                const int64_t nl = lr ? N : (td.p1 - td.p0) + 2 * (lat ? cols : 1);
+                // LDS: the tile's slips and halo (long range: every slip of the
+                // system and the prefactors of the tile's differences)
+                const int64_t nl = lr ? (N <= fq::LR_TILE_PREF_MAX ? 2 * N + step : N) : (td.p1 - td.p0) + 2 * (lat ? cols : 1);
                 lds = std::max<size_t>(lds, sizeof(double) * (size_t)nl);
             }
         }
@@ -2168,6 +2203,7 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
         S.lr_m = (N - N % 2) / 2;
         const size_t o = (size_t)g->off[(size_t)r];
         S.pref = g->pref ? g->pref + o : nullptr;
+        S.prefx = g->prefx ? g->prefx + 2 * o : nullptr;
         S.u = g->u + o;
         S.v = g->v + o;
         S.a = g->a + o;
@@ -2189,7 +2225,7 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
             S.yl_a = g->yl + o;
             S.yr_a = g->yr + o;
         }
-        if (g->streaming) {
+        if (g->jl2) {
             S.u_b = g->u2 + o;
             S.v_b = g->v2 + o;
             S.a_b = g->a2 + o;

@@ -61,6 +61,14 @@ enum Status : int32_t {
     ST_MAXITER = 9    // quasistatic driver: a minimisation used max_iter steps
 };
 
+// Resident long-range chains up to this size hold the prefactors of all
+// differences in LDS beside the slips (4 N doubles); larger ones read them
+// from memory.
+constexpr int64_t LR_LDS_PREF_MAX = 4096;
+// The same for tiles of long-range chains: N slips and N + tile - 1
+// prefactors (up to here they fit 160 KB).
+constexpr int64_t LR_TILE_PREF_MAX = 9728;
+
 // The quasistatic driver for chains (k_quasi_chain) keeps the state of the
 // last committed step in LDS (8 bytes per particle, beyond the exchange
 // buffers) instead of a second register array for these launch variants
@@ -152,7 +160,8 @@ struct SysView {
     double m, inv_m, eta, mu, kappa, k_frame, dt;
     double k, a1, a2, k2, k4, k4_4, alpha;
     int64_t lr_m;
-    double* pref; // LongRange1d prefactor [N]
+    double* pref;  // LongRange1d prefactor [N]
+    double* prefx; // LongRange1d prefactor of the difference d in [-(N-1), N-1], at d + N - 1 (0 at d = 0)
     double *u, *v, *a, *f, *f_pot, *f_int, *f_frame, *f_damp, *f_th;
     // streaming path (systems larger than a resident workgroup): second state
     // buffer and the yield positions of the current well of both buffers

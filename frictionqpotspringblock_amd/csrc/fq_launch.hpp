@@ -90,7 +90,7 @@ inline size_t resident_lds(int inter, int64_t N, int threads)
         return sizeof(double) * 4 * (size_t)threads;
     }
     if (inter == INT_LONGRANGE1D) {
-        return sizeof(double) * 3 * (size_t)N;
+        return sizeof(double) * (N <= LR_LDS_PREF_MAX ? 4 : 2) * (size_t)N;
     }
     return sizeof(double) * 2 * (size_t)N;
 }

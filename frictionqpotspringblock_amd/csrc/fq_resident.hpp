@@ -185,21 +185,6 @@ __device__ __forceinline__ bool reachable(const double* row, int32_t j, double l
     return lo <= x && x < hi;
 }
 
-// LDS needed by a resident launch (bytes of dynamic shared memory).
-template <int INT>
-FQ_HD size_t resident_lds_bytes(int64_t N, int threads)
-{
-    if constexpr (is_chain<INT>()) {
-        return sizeof(double) * 4 * (size_t)threads;
-    }
-    else if constexpr (INT == INT_LONGRANGE1D) {
-        return sizeof(double) * 3 * (size_t)N;
-    }
-    else {
-        return sizeof(double) * 2 * (size_t)N;
-    }
-}
-
 // Align particle p to slip z (outside its window's safe zone) from inside a
 // step loop: called by all lanes of a wavefront with the same arguments;
 // returns the local well index and its bounds.
@@ -304,7 +289,7 @@ __device__ __forceinline__ void resident_body(const SysView* __restrict__ views,
     double* h_first = s_dyn;        // [2][T]   chain: first slip of each thread
     double* h_last = s_dyn + 2 * T; // [2][T]   chain: last slip of each thread
     double* mir = s_dyn;            // [2][N]   lattice / long range: all slips
-    double* pref = s_dyn + 2 * N;   // [N]      long range prefactor
+    double* pref = s_dyn + 2 * N;   // [2N-1]   long range prefactors (N <= LR_LDS_PREF_MAX)
 
     double u[PPT], v[PPT], a[PPT], yl[PPT], yr[PPT], fth[PPT];
     int32_t jl[PPT], dl[PPT];
@@ -405,8 +390,10 @@ __device__ __forceinline__ void resident_body(const SysView* __restrict__ views,
         };
 
         if constexpr (INT == INT_LONGRANGE1D) {
-            for (int64_t q = t; q < N; q += T) {
-                pref[q] = S.pref[q];
+            if (N <= LR_LDS_PREF_MAX) {
+                for (int64_t q = t; q < 2 * N - 1; q += T) {
+                    pref[q] = S.prefx[q];
+                }
             }
         }
         publish(0, false);
@@ -452,8 +439,14 @@ __device__ __forceinline__ void resident_body(const SysView* __restrict__ views,
             }
             else if constexpr (INT == INT_LONGRANGE1D) {
                 const double* U = mir + (int64_t)b * N;
-                return longrange_force(
-                    S, [&](int64_t q) { return U[q]; }, [&](int64_t d) { return pref[d]; }, base + i);
+                const int64_t o = N - 1 - (base + i);
+                auto slip = [&](int q) { return U[q]; };
+                if (N <= LR_LDS_PREF_MAX) {
+                    const double* G = pref + o;
+                    return longrange_force((int)N, slip, [&](int q) { return G[q]; }, u[i]);
+                }
+                const double* __restrict__ G = S.prefx + o;
+                return longrange_force((int)N, slip, [&](int q) { return G[q]; }, u[i]);
             }
             else {
                 const double* U = mir + (int64_t)b * N;

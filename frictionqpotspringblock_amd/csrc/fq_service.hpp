@@ -118,9 +118,9 @@ __global__ void __launch_bounds__(SVC_THREADS) k_lr_fint(const SysView* __restri
     const SysView& S = views[blockIdx.y];
     const int64_t N = S.N;
     const double* __restrict__ u = S.u;
-    const double* __restrict__ pref = S.pref;
     for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < N; p += (int64_t)gridDim.x * blockDim.x) {
-        S.f_int[p] = longrange_force(S, [&](int64_t q) { return u[q]; }, [&](int64_t d) { return pref[d]; }, p);
+        const double* __restrict__ G = S.prefx + (N - 1 - p);
+        S.f_int[p] = longrange_force((int)N, [&](int q) { return u[q]; }, [&](int q) { return G[q]; }, u[p]);
     }
 }
 
@@ -170,8 +170,8 @@ __global__ void __launch_bounds__(SVC_THREADS) k_forces(const SysView* __restric
                 fi = chain_force<INT>(S, um, up, upp);
             }
             else if constexpr (INT == INT_LONGRANGE1D) {
-                fi = longrange_force(
-                    S, [&](int64_t q) { return S.u[q]; }, [&](int64_t d) { return S.pref[d]; }, p);
+                const double* G = S.prefx + (N - 1 - p);
+                fi = longrange_force((int)N, [&](int q) { return S.u[q]; }, [&](int q) { return G[q]; }, up);
             }
             else if constexpr (INT == INT_LAPLACE2D || INT == INT_QUARTICGRADIENT2D) {
                 fi = lattice_force<INT>(S, [&](int64_t q) { return S.u[q]; }, p / S.cols, p % S.cols);

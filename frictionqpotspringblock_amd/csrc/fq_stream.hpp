@@ -102,8 +102,8 @@ __global__ void __launch_bounds__(STREAM_THREADS) k_stream(const SysView* __rest
             return chain_force<INT>(S, Un[p == 0 ? N - 1 : p - 1], Un[p], Un[p == N - 1 ? 0 : p + 1]);
         }
         else if constexpr (INT == INT_LONGRANGE1D) {
-            return longrange_force(
-                S, [&](int64_t q) { return Un[q]; }, [&](int64_t d) { return S.pref[d]; }, p);
+            const double* G = S.prefx + (N - 1 - p);
+            return longrange_force((int)N, [&](int q) { return Un[q]; }, [&](int q) { return G[q]; }, Un[p]);
         }
         else {
             return lattice_force<INT>(S, [&](int64_t q) { return Un[q]; }, p / S.cols, p % S.cols);

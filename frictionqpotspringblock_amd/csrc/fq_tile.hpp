@@ -117,6 +117,12 @@ __global__ void __launch_bounds__(TILE_THREADS) k_tile_step(const SysView* __res
         q = q < 0 ? q + N : (q >= N ? q - N : q);
         s_x[k] = Uc[q] + dt * Vc[q] + c2 * Ac[q];
     }
+    const bool lr_lds = LR && N <= LR_TILE_PREF_MAX;
+    if (lr_lds) { // prefactors of the differences i - p, p in the tile: -(p1 - 1) .. N - 1 - p0
+        for (int64_t k = t; k < N + n - 1; k += T) {
+            s_x[N + k] = S.prefx[N - p1 + k];
+        }
+    }
     __syncthreads();
 
     // well walk of the tile's own particles (in place)
@@ -176,10 +182,17 @@ __global__ void __launch_bounds__(TILE_THREADS) k_tile_step(const SysView* __res
         }
         else if constexpr (LR) {
             // the reference's sequential sum over all particles (detail.h:
-            // 849-867), slips from LDS (one address per step of the sum:
-            // a broadcast), prefactors from the system's table
-            const double* __restrict__ pref = S.pref;
-            fi = longrange_force(S, [&](int64_t i) { return s_x[i]; }, [&](int64_t d) { return pref[d]; }, p);
+            // 849-867), slips from LDS (one address per term: a broadcast),
+            // prefactors from the tile's window of the table of differences
+            auto slip = [&](int i) { return s_x[i]; };
+            if (lr_lds) {
+                const double* G = s_x + N + (n - 1 - k);
+                fi = longrange_force((int)N, slip, [&](int i) { return G[i]; }, x);
+            }
+            else {
+                const double* __restrict__ G = S.prefx + (N - 1 - p);
+                fi = longrange_force((int)N, slip, [&](int i) { return G[i]; }, x);
+            }
         }
         else if constexpr (LAT) {
             fi = lattice_force<INT>(S, X, p / cols, p % cols);
@@ -960,8 +973,8 @@ __global__ void __launch_bounds__(TILE_THREADS) k_tile_finish(const SysView* __r
                 fi = 0.0;
             }
             else if constexpr (INT == INT_LONGRANGE1D) {
-                const double* __restrict__ pref = S.pref;
-                fi = longrange_force(S, U, [&](int64_t d) { return pref[d]; }, p);
+                const double* __restrict__ G = S.prefx + (N - 1 - p);
+                fi = longrange_force((int)N, U, [&](int q) { return G[q]; }, x);
             }
             else if constexpr (LAT) {
                 fi = lattice_force<INT>(S, U, p / cols, p % cols);

@@ -83,3 +83,64 @@ def test_adjoint_refuses_moved_windows():
     z = torch.zeros((2, 64), dtype=torch.float64, device="cuda")
     with pytest.raises(RuntimeError, match="left the landscape window"):
         A.run(b, 300, 50, z, z + 20.0, z, A.parameters(b), flow=True, v_frame=0.5)
+
+
+def _longrange_kw(N, **extra):
+    return _kw(N, alpha=1.0, offset=-100.0, nchunk=200, **extra)
+
+
+@pytest.mark.parametrize("N", [3, 64, 511, 512, 513, 577, 1000])
+def test_longrange_exact_sum(N):
+    """A long-range chain on both sides of the size at which its steps and
+    minimisations spread over tiles; the operations that stay resident in
+    between (until event, activity, truncation) continue from the same state."""
+    import frictionqpotspringblock_amd as fq
+
+    kw = _longrange_kw(N)
+    g, o = fq.Line1d.System_Cuspy_LongRange(**kw), pyoracle.Line1d.System_Cuspy_LongRange(**kw)
+    v = np.random.default_rng(N).normal(size=N)
+    for s in (g, o):
+        s.v = v
+        s.flowSteps(30, 0.2)
+        s.timeSteps(17)
+    assert np.array_equal(g.u, o.u) and np.array_equal(g.v, o.v) and np.array_equal(g.f, o.f)
+    ret = []
+    for s in (g, o):
+        r = [s.minimise(), s.eventDrivenStep(1e-3, False), s.eventDrivenStep(1e-3, True)]
+        r += [s.timeStepsUntilEvent(), s.minimise(time_activity=True), s.quasistaticActivityLast]
+        s.eventDrivenStep(1e-3, True)
+        r += [s.minimise(), s.inc, s.u_frame]
+        ret.append(r)
+    assert ret[0] == ret[1]
+    assert np.array_equal(g.u, o.u) and np.array_equal(g.f_interactions, o.f_interactions)
+    assert np.array_equal(g.chunk.index_at_align, o.chunk.index_at_align)
+
+
+@pytest.mark.parametrize("N", [255, 256, 257, 511, 512, 513, 1024, 2049, 4095, 4097, 8191, 8192, 8193, 16384])
+def test_longrange_product(N):
+    """The batched long-range forces at the sizes where the transforms change
+    (powers of two, one more, one less; the matrix product below 257 and above
+    8192), against the sum in extended precision. The transforms' error is
+    at most a small multiple of eps log2(M) |g| |w| (2-norms of the kernel and
+    of the shifted slips; forward, product and inverse, 8 for the constants);
+    the matrix product's at most gamma_N times the sum of the terms."""
+    from frictionqpotspringblock_amd.batch import Batch
+
+    R = 2
+    b = Batch(R, seed_stride=N, potential="Cuspy", interactions="LongRange1d", **_longrange_kw(N))
+    u = np.random.default_rng(N).normal(size=(R, N))
+    b.u = u
+    b.timeSteps(1)
+    u = b.u.astype(np.longdouble)
+    d = np.minimum(np.arange(N), N - np.arange(N)).astype(float)
+    g = np.zeros(N)
+    g[1:] = 1.0 / d[1:] ** 2.0
+    gl, uu = g.astype(np.longdouble), np.concatenate([u, u], axis=1)
+    f = np.zeros((R, N), dtype=np.longdouble)
+    for k in range(1, N):
+        f += gl[k] * (uu[:, k:k + N] - u)
+    w = np.linalg.norm((u - u[:, :1]).astype(float), axis=1)
+    eps = np.finfo(float).eps
+    bound = 8.0 * eps * np.log2(4 * N) * np.linalg.norm(g) * w[:, None]
+    bound = np.maximum(bound, 2.0 * N * eps * g.sum() * np.abs(u - u[:, :1]).max()) if N < 257 or N == 8193 else bound
+    assert np.all(np.abs(b.f_interactions - f) <= bound)
