@@ -544,6 +544,19 @@ struct Group {
     {
         for (size_t i = 0; i < hrs.size(); ++i) {
             auto& r = hrs[i];
+        // minimise of chains and lattices: the quasistatic driver's pipelined
+        // steps, which decide the same (without activity tracking and forcing)
+        if (ra.mode == fq::MODE_MINIMISE && inter != FQSB_INT_LONGRANGE1D && !ra.time_activity &&
+            ext == FQSB_EXT_NONE && !general_kernel) {
+            const size_t qlds = fq::quasi_lds(inter, N, ppt, maxt, threads);
+            fq::QsArgs qa{};
+            qa.plain = 1;
+            if (qlds <= lds_limit && fq::launch_quasi(pot, inter, ppt, maxt, threads, qlds, views, (int)R, ra, qa,
+                                                      stream, unit_mass, full)) {
+                HIPC(hipGetLastError());
+                return;
+            }
+        }
             r.status = (mask && !mask[i]) ? fq::ST_IDLE : fq::ST_RUNNING;
             r.steps = 0;
             r.refilled = 0;

@@ -290,6 +290,8 @@ struct QsArgs {
     double eps;
     int32_t direction;
     int32_t kicks;
+    int32_t plain; // k_quasi_chain: only minimise (MODE_MINIMISE of a run), no protocol
+    int32_t pad;
     int64_t max_iter; // steps per minimisation
     int64_t* out_S;
     double* out_uf;
@@ -518,97 +520,71 @@ FQ_HD double fq_ksin(double x, double y)
     return x - ((z * (0.5 * y - v * r) - y) - v * S1);
 }
 
+// (for |x| below 2^-27 fdlibm returns 1 at once: the expression rounds to it)
 FQ_HD double fq_kcos(double x, double y)
 {
     constexpr double C1 = 4.16666666666666019037e-02, C2 = -1.38888888888741095749e-03,
                      C3 = 2.48015872894767294178e-05, C4 = -2.75573143513906633035e-07,
                      C5 = 2.08757232129817482790e-09, C6 = -1.13596475577881948265e-11;
-    uint32_t ix = hiword(x) & 0x7fffffff;
-    if (ix < 0x3e400000) {
-        if ((int)x == 0) {
-            return 1.0;
-        }
-    }
-    double z = x * x;
-    double r = z * (C1 + z * (C2 + z * (C3 + z * (C4 + z * (C5 + z * C6)))));
-    if (ix < 0x3FD33333) {
-        return 1.0 - (0.5 * z - (z * r - x * y));
-    }
-    double qx;
-    if (ix > 0x3fe90000) {
-        qx = 0.28125;
-    }
-    else {
-        qx = __builtin_bit_cast(double, ((uint64_t)(ix - 0x00200000)) << 32);
-    }
-    double hz = 0.5 * z - qx;
-    double a = 1.0 - qx;
+    const uint32_t ix = hiword(x) & 0x7fffffff;
+    const double z = x * x;
+    const double r = z * (C1 + z * (C2 + z * (C3 + z * (C4 + z * (C5 + z * C6)))));
+    // qx about x / 4, 0 below 0.3 (1 - (z / 2 - (z r - x y)) is then the
+    // expression below)
+    double qx = __builtin_bit_cast(double, ((uint64_t)(ix - 0x00200000)) << 32);
+    qx = ix > 0x3fe90000 ? 0.28125 : qx;
+    qx = ix < 0x3FD33333 ? 0.0 : qx;
+    const double hz = 0.5 * z - qx;
+    const double a = 1.0 - qx;
     return a - (hz - (z * r - x * y));
 }
 
 FQ_HD int fq_rem_pio2(double x, double& y0, double& y1)
 {
     constexpr double INVPIO2 = 6.36619772367581382433e-01, PIO2_1 = 1.57079632673412561417e+00,
-                     PIO2_1T = 6.07710050650619224932e-11, PIO2_2 = 6.07710050630396597660e-11,
-                     PIO2_2T = 2.02226624879595063154e-21;
+                     PIO2_2 = 6.07710050630396597660e-11, PIO2_2T = 2.02226624879595063154e-21;
     double t = __builtin_fabs(x);
     int n = (int)(t * INVPIO2 + 0.5);
     double fn = (double)n;
-    double r = t - fn * PIO2_1;
-    double w = fn * PIO2_1T;
-    double tt = r;
-    w = fn * PIO2_2;
-    r = tt - w;
+    double tt = t - fn * PIO2_1;
+    double w = fn * PIO2_2;
+    double r = tt - w;
     w = fn * PIO2_2T - ((tt - r) - w);
     double a = r - w;
     double b = (r - a) - w;
-    if (x < 0.0) {
-        y0 = -a;
-        y1 = -b;
-        return -n;
-    }
-    y0 = a;
-    y1 = b;
-    return n;
+    y0 = x < 0.0 ? -a : a;
+    y1 = x < 0.0 ? -b : b;
+    return x < 0.0 ? -n : n;
 }
 
 // sin / cos for |x| < 823549.6875 (the hot path only produces |x| <= 2 pi).
+// Both kernels are evaluated and one selected: the lanes of a wavefront are
+// in several quadrants, so branches would run one after the other, and the
+// particles of a thread could not be computed side by side.
 FQ_HD double fq_sin(double x)
 {
-    if (__builtin_fabs(x) < 0.7853981633974483) {
-        return fq_ksin(x, 0.0);
-    }
     double y0, y1;
     int n = fq_rem_pio2(x, y0, y1);
-    switch (n & 3) {
-        case 0:
-            return fq_ksin(y0, y1);
-        case 1:
-            return fq_kcos(y0, y1);
-        case 2:
-            return -fq_ksin(y0, y1);
-        default:
-            return -fq_kcos(y0, y1);
-    }
+    const bool small = __builtin_fabs(x) < 0.7853981633974483;
+    y0 = small ? x : y0;
+    y1 = small ? 0.0 : y1;
+    n = small ? 0 : n;
+    const double s = fq_ksin(y0, y1), c = fq_kcos(y0, y1);
+    const double r = (n & 1) ? c : s;
+    return (n & 2) ? -r : r;
 }
 
 FQ_HD double fq_cos(double x)
 {
-    if (__builtin_fabs(x) < 0.7853981633974483) {
-        return fq_kcos(x, 0.0);
-    }
     double y0, y1;
     int n = fq_rem_pio2(x, y0, y1);
-    switch (n & 3) {
-        case 0:
-            return fq_kcos(y0, y1);
-        case 1:
-            return -fq_ksin(y0, y1);
-        case 2:
-            return -fq_kcos(y0, y1);
-        default:
-            return fq_ksin(y0, y1);
-    }
+    const bool small = __builtin_fabs(x) < 0.7853981633974483;
+    y0 = small ? x : y0;
+    y1 = small ? 0.0 : y1;
+    n = small ? 0 : n;
+    const double s = fq_ksin(y0, y1), c = fq_kcos(y0, y1);
+    const double r = (n & 1) ? s : c;
+    return ((n + 1) & 2) ? -r : r;
 }
 
 FQ_HD double fq_pow(double x, double y)

@@ -9,8 +9,8 @@
 //    before step it+1 discards them), checked for reachability and published
 //    to the LDS exchange buffer (it+1)&1 for the neighbours; step it+1 then
 //    commits them. One __syncthreads per step, at the top of the step.
-//  * the mid-point of the current well, 0.5 (y_l + y_r), is kept in a
-//    register (recomputed when the well changes) for the Cuspy force;
+//  * the constants of the current well (well_consts: Cuspy its mid-point) are
+//    kept in registers, recomputed when the well changes;
 //  * with m = 1 the multiplication by 1/m (exact) is skipped;
 //  * no event / residual bookkeeping;
 //  * FULL (every system of the launch has N divisible by PPT, so a thread
@@ -25,17 +25,6 @@
 #include <type_traits>
 
 namespace fq {
-
-template <int POT>
-FQ_HD double potential_force_mid(const SysView& S, double u, double yl, double yr, double ym)
-{
-    if constexpr (POT == POT_CUSPY) {
-        return (ym - u) * S.mu; // (0.5 * (yl + yr) - u) * mu with the mid-point cached
-    }
-    else {
-        return potential_force<POT>(S, u, yl, yr);
-    }
-}
 
 // One entry of k_flow: from the state in memory to the state in memory, until
 // the launch's step budget (of which earlier entries took `launch_done`) or a
@@ -85,11 +74,29 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
     // registers without per-particle branches and only the stores are
     // guarded. The reset runs only in wavefronts that hold padding (a scalar
     // branch: a full wavefront skips it).
-    double sa[PPT], sb[PPT], v[PPT], a[PPT], yl[PPT], yr[PPT], ym[PPT], fth[PPT];
+    double sa[PPT], sb[PPT], v[PPT], a[PPT], yl[PPT], yr[PPT], fth[PPT];
+    // constants of the current well (well_consts)
+    constexpr bool WC1 = POT != POT_CUSPY;
+    double c0[PPT], c1[WC1 ? PPT : 1];
+    auto set_well = [&](int i, double lo, double hi) {
+        yl[i] = lo;
+        yr[i] = hi;
+        double k1;
+        well_consts<POT>(P, lo, hi, c0[i], k1);
+        if constexpr (WC1) {
+            c1[i] = k1;
+        }
+    };
+    auto well_force = [&](int i, double x) -> double {
+        return potential_force_wc<POT>(P, x, yl[i], yr[i], c0[i], c1[WC1 ? i : 0]);
+    };
     int32_t jl[PPT];
 #pragma unroll
     for (int i = 0; i < PPT; ++i) {
-        sa[i] = sb[i] = v[i] = a[i] = ym[i] = fth[i] = 0.0;
+        sa[i] = sb[i] = v[i] = a[i] = c0[i] = fth[i] = 0.0;
+        if constexpr (WC1) {
+            c1[i] = 0.0;
+        }
         yl[i] = -__builtin_inf();
         yr[i] = __builtin_inf();
         jl[i] = 0;
@@ -99,9 +106,7 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
             v[i] = S.v[p];
             a[i] = S.a[p];
             jl[i] = L.jloc[p];
-            yl[i] = Y[p * nch + jl[i]];
-            yr[i] = Y[p * nch + jl[i] + 1];
-            ym[i] = 0.5 * (yl[i] + yr[i]);
+            set_well(i, Y[p * nch + jl[i]], Y[p * nch + jl[i] + 1]);
             if constexpr (EXT) {
                 fth[i] = S.f_th[p];
             }
@@ -307,9 +312,7 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
                     }
                     if (lo <= z && z < hi) {
                         jl[i] = j;
-                        yl[i] = lo;
-                        yr[i] = hi;
-                        ym[i] = 0.5 * (lo + hi);
+                        set_well(i, lo, hi);
                     }
                     else if (INLINE_REFILL && __builtin_isfinite(z)) {
                         need |= 1u << i;
@@ -334,9 +337,7 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
                     const WellAt w = refill_one(&S, p, z, __builtin_amdgcn_readlane(jl[i], src));
                     if ((t & 63) == src) {
                         jl[i] = w.j;
-                        yl[i] = w.lo;
-                        yr[i] = w.hi;
-                        ym[i] = 0.5 * (w.lo + w.hi);
+                        set_well(i, w.lo, w.hi);
                     }
                 }
             }
@@ -347,7 +348,7 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
 #pragma unroll
         for (int i = 0; i < PPT; ++i) {
             const double fi = interaction(i, b, x);
-            const double fp = potential_force_mid<POT>(P, x[i], yl[i], yr[i], ym[i]);
+            const double fp = well_force(i, x[i]);
             const double ff = kf * (uf - x[i]);
             const double sum3 = ff + fp + fi;
             const double vn = v[i], an = a[i];
@@ -399,7 +400,7 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
                 L.jloc[p] = jl[i];
                 if (status != ST_NAN && status != ST_REFILL) {
                     const double fi = interaction(i, fb, x);
-                    const double fp = potential_force_mid<POT>(S, x[i], yl[i], yr[i], ym[i]);
+                    const double fp = well_force(i, x[i]);
                     const double ff = kf * (uf - x[i]);
                     const double fd = meta * v[i];
                     S.f_int[p] = fi;

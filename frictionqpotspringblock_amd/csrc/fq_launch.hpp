@@ -99,10 +99,8 @@ inline size_t resident_lds(int inter, int64_t N, int threads)
 // layouts of k_quasi_chain and k_quasi)
 inline size_t quasi_lds(int inter, int64_t N, int ppt, int maxt, int threads)
 {
-    const bool chain =
-        inter == INT_NONE || inter == INT_LAPLACE1D || inter == INT_QUARTIC1D || inter == INT_QUARTICGRADIENT1D;
     return resident_lds(inter, N, threads) +
-           (chain && quasi_inplace(ppt, maxt) ? sizeof(double) * (size_t)ppt * threads : 0);
+           (inter != INT_LONGRANGE1D && quasi_inplace(ppt, maxt) ? sizeof(double) * (size_t)ppt * threads : 0);
 }
 
 // batched long range (fq_longrange.hip)

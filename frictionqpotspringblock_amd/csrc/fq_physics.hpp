@@ -38,12 +38,28 @@ FQ_HD double potential_force(const SysView& S, double u, double yl, double yr)
     }
 }
 
+// a / b, correctly rounded as the division is, from the correctly rounded
+// reciprocal rb = 1 / b: two residual corrections, the last one from a
+// quotient that is faithful (Markstein, IBM J. Res. Dev. 34, 1990), five
+// operations instead of the division's eleven and no chain through the
+// reciprocal. Exact for 2^-900 <= |a| < 2^900 and 2^-100 < b < 2^100 (no
+// residual underflows); the callers divide outside.
+FQ_HD double div_rcp(double a, double b, double rb)
+{
+    double q = a * rb;
+    q = __builtin_fma(__builtin_fma(-b, q, a), rb, q);
+    q = __builtin_fma(__builtin_fma(-b, q, a), rb, q);
+    return q;
+}
+
 // The same forces with the constants of the current well computed once per
 // well (when it changes) instead of every step: Cuspy its mid-point (c0);
 // SemiSmooth the edges u_l (c0), u_r (c1) of the parabolic part (two
-// divisions); Smooth the prefactor (-mu dy) / pi of the sine (c0). Each
-// constant is the subexpression of potential_force above, so the force is
-// bit-identical.
+// divisions); Smooth the prefactor (-mu dy) / pi of the sine (c0) and 1 / dy
+// (c1). Each constant is the subexpression of potential_force above (the
+// quotient of the sine's argument is the division's, div_rcp), so the force
+// is bit-identical. Selections instead of branches: the particles of a thread
+// are then computed side by side.
 template <int POT, class Sys>
 FQ_HD void well_consts(const Sys& S, double yl, double yr, double& c0, double& c1)
 {
@@ -60,7 +76,7 @@ FQ_HD void well_consts(const Sys& S, double yl, double yr, double& c0, double& c
     else {
         double dy = 0.5 * (yr - yl);
         c0 = -S.mu * dy / FQ_PI;
-        c1 = 0.0;
+        c1 = dy > 0x1p-100 && dy < 0x1p100 ? 1.0 / dy : __builtin_nan("");
     }
 }
 
@@ -71,18 +87,23 @@ FQ_HD double potential_force_wc(const Sys& S, double u, double yl, double yr, do
         return (c0 - u) * S.mu;
     }
     else if constexpr (POT == POT_SEMISMOOTH) {
-        if (u < c0) {
-            return S.kappa * (u - yl);
-        }
-        if (u <= c1) {
-            return S.mu * (0.5 * (yl + yr) - u);
-        }
-        return S.kappa * (u - yr);
+        const bool in = u <= c1, left = u < c0;
+        const double k = S.kappa * (u - (left ? yl : yr));
+        const double m = S.mu * (0.5 * (yl + yr) - u);
+        return in && !left ? m : k;
     }
     else {
-        double umin = 0.5 * (yl + yr);
-        double dy = 0.5 * (yr - yl);
-        return c0 * fq_sin(FQ_PI * (u - umin) / dy);
+        const double umin = 0.5 * (yl + yr);
+        const double dy = 0.5 * (yr - yl);
+        const double a = FQ_PI * (u - umin);
+        double x = div_rcp(a, dy, c1);
+        // outside 2^-900 <= |a| < 2^900 and for wells without a reciprocal:
+        // the division
+        const uint32_t e = (hiword(a) & 0x7fffffff) - 0x07b00000u;
+        if (e >= 0x70800000u || x != x) {
+            x = a / dy;
+        }
+        return c0 * fq_sin(x);
     }
 }
 
@@ -164,6 +185,32 @@ FQ_HD double lattice_force(const Sys& S, const Acc& U, int64_t i, int64_t j)
         double d2udxdy = 0.25 * (U(ip * C + jp) - U(ip * C + jm) - U(im * C + jp) + U(im * C + jm));
         double d2udx2 = uip - 2 * c0 + uim;
         double d2udy2 = ujp - 2 * c0 + ujm;
+        return l * (S.k2 + mk4_3) + mk4_23 * (dudx * dudx * d2udx2 + dudy * dudy * d2udy2 + 2.0 * dudx * dudy * d2udxdy);
+    }
+}
+
+// The same of the site in row offset ric, column cjc (slip c0) with the rows
+// above and below at offsets rim, rip and the columns beside it at cjm, cjp
+// of the slip field U (the periodic wrap and the divisions done once per site
+// instead of every step; 4 c0 is exact, so its subtraction rounds once either
+// way).
+template <int INT, class Sys>
+FQ_HD double lattice_force_at(const Sys& S, const double* U, int rim, int ric, int rip, int cjm, int cjc, int cjp,
+                              double c0)
+{
+    const double uim = U[rim + cjc], uip = U[rip + cjc], ujm = U[ric + cjm], ujp = U[ric + cjp];
+    if constexpr (INT == INT_LAPLACE2D) {
+        return __builtin_fma(-4.0, c0, uim + uip + ujm + ujp) * S.k;
+    }
+    else {
+        const double mk4_3 = S.k4 / 3.0;
+        const double mk4_23 = 2.0 * mk4_3;
+        const double l = __builtin_fma(-4.0, c0, uip + uim + ujp + ujm);
+        const double dudx = 0.5 * (uip - uim);
+        const double dudy = 0.5 * (ujp - ujm);
+        const double d2udxdy = 0.25 * (U[rip + cjp] - U[rip + cjm] - U[rim + cjp] + U[rim + cjm]);
+        const double d2udx2 = __builtin_fma(-2.0, c0, uip) + uim;
+        const double d2udy2 = __builtin_fma(-2.0, c0, ujp) + ujm;
         return l * (S.k2 + mk4_3) + mk4_23 * (dudx * dudx * d2udx2 + dudy * dudy * d2udy2 + 2.0 * dudx * dudy * d2udxdy);
     }
 }

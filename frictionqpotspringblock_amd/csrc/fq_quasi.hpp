@@ -1,4 +1,4 @@
-// Quasistatic driver for chains: the examples' event loop
+// Quasistatic driver for chains and lattices: the examples' event loop
 // (examples/Line1d_Cuspy_Laplace.py:39-61: eventDrivenStep, detail.h:1933-1960,
 // then minimise, detail.h:1676-1792) inside one workgroup per system, as
 // k_quasi (fq_resident.hpp) runs it for every interaction, with the same
@@ -12,7 +12,7 @@
 //    back only when the entry stops, and the next slips replace it). One
 //    __syncthreads per step, at its top, after which the StopList decision on
 //    step it-1 is taken from the wavefronts' residual partial sums;
-//  * the Cuspy mid-point of the current well kept in a register;
+//  * the constants of the current well (well_consts) kept in registers;
 //  * with m = 1 the multiplication by 1/m (exact) is skipped;
 //  * padding registers (i >= cnt) at rest in an unbounded well: no
 //    per-particle branches in the step, the sums masked.
@@ -32,7 +32,8 @@ template <int POT, int INT, int PPT, int MAXT, bool UNIT, bool FULL>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(MAXT <= 256 && PPT <= 8 ? 2 : 1)))
 k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
 {
-    static_assert(is_chain<INT>(), "k_quasi_chain handles chains");
+    constexpr bool CHAIN = is_chain<INT>();
+    static_assert(CHAIN || INT == INT_LAPLACE2D || INT == INT_QUARTICGRADIENT2D, "chains and lattices");
     const SysView& S = views[blockIdx.x];
     // the system's parameters as a local copy (no reload after every barrier)
     const SysView P = S;
@@ -41,9 +42,10 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
         return;
     }
 
-    __shared__ double s_red_d[2][RES_MAX_WAVES][2];
-    __shared__ int s_nan[2];
-    __shared__ int s_refill[2];
+    constexpr int NW = MAXT / 64; // wavefronts of the widest launch
+    __shared__ __attribute__((aligned(16))) double s_red_d[2][NW][2]; // zero beyond the launch's wavefronts
+    // per parity of the step: {step that needs a refill, step before it that met a NaN}
+    __shared__ __attribute__((aligned(8))) int s_flag[2][2];
     __shared__ long long s_qs_i[RES_MAX_WAVES];
     __shared__ double s_qs_d[RES_MAX_WAVES];
     __shared__ QsArgs s_qa; // the protocol's arguments, read where the events use them
@@ -61,8 +63,9 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
     const int64_t nch = L.nchunk;
     const int32_t jmin = (int32_t)L.buffer;
     const int32_t jmax = (int32_t)(L.nchunk - 2 - L.buffer);
-    double* h_first = s_dyn;        // [2][T] first slip of each thread
-    double* h_last = s_dyn + 2 * T; // [2][T] last slip of each thread
+    double* h_first = s_dyn;        // chains: [2][T] first slip of each thread
+    double* h_last = s_dyn + 2 * T; // chains: [2][T] last slip of each thread
+    double* const mir = s_dyn;      // lattices: [2][N] all slips
 
     const double dt = S.dt;
     const double c2 = 0.5 * dt * dt;
@@ -91,7 +94,9 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
     // event, phase, sum of the well index changes when the event began, steps
     // of the current minimisation before this entry
     int64_t ev = rs->qs_event;
-    int32_t phase = rs->qs_phase;
+    // plain: one minimisation (System::minimise) instead of the protocol
+    const bool plain = qa.plain != 0;
+    int32_t phase = plain ? (int32_t)QS_MINIMISE : rs->qs_phase;
     int64_t isum = rs->qs_isum;
     int64_t ev_done0 = rs->steps;
     int32_t refill_u = 0;    // the pending refill aligns at u (a displacement)
@@ -99,6 +104,10 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
     uint32_t rmask = 0;      // this thread's particles that need a refill (bit i)
     int32_t status = ST_RUNNING;
     int limit = 0;
+    // residuals that are certainly not below tol, by the squares of their norms
+    // (the margin covers the roundings of the roots and the quotient)
+    const double tol_clear = ra.tol2 * (1.0 + 1e-9);
+    const bool clear_of_tol = ra.tol <= 1.0 && ra.tol > 1e-100 && ra.niter_tol > 0;
     int64_t maxit = 0; // steps the entry's minimisation may take before max_iter
 
     // sa / sb: the state's slips and the slips prepared for the next step, in
@@ -109,9 +118,13 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
     // next slips are prepared in place: no second register array (8
     // particles per thread: no spills) and one step per loop iteration
     constexpr bool INPLACE = quasi_inplace(PPT, MAXT);
-    double sa[PPT], sb[INPLACE ? 1 : PPT], v[PPT], a[PPT], ym[PPT];
+    double sa[PPT], sb[INPLACE ? 1 : PPT], v[PPT], a[PPT];
+    // constants of the current well (well_consts)
+    constexpr bool WC1 = POT != POT_CUSPY;
+    double c0[PPT], c1[WC1 ? PPT : 1];
     int32_t jl[PPT];
-    double* const s_keep = s_dyn + 4 * T; // INPLACE: [PPT][T] the state of the last committed step
+    // INPLACE: [PPT][T] the state of the last committed step
+    double* const s_keep = s_dyn + (CHAIN ? 4 * (int64_t)T : 2 * N);
     // the bounds (y_l, y_r) of each register's well and, for up to 4 particles
     // per thread (NEXT; 8 would spill), the right bound of the next well to
     // the right (yield position j + 2; +inf past the window's end), read when
@@ -131,8 +144,47 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
         yl_r[i] = lo;
         yr_r[i] = hi;
     };
+    auto set_well = [&](int i, double lo, double hi) {
+        set_bounds(i, lo, hi);
+        double k1;
+        well_consts<POT>(P, lo, hi, c0[i], k1);
+        if constexpr (WC1) {
+            c1[i] = k1;
+        }
+    };
+    auto well_force = [&](int i, double x) -> double {
+        return potential_force_wc<POT>(P, x, yl_r[i], yr_r[i], c0[i], c1[WC1 ? i : 0]);
+    };
+
+    // lattices: for each register the row above, its own and the row below
+    // (as offsets of their first sites) and the columns to the left and right
+    constexpr int NP = CHAIN ? 1 : PPT;
+    int rim[NP], ric[NP], rip[NP], cjm[NP], cjc[NP], cjp[NP];
+    if constexpr (!CHAIN) {
+        const int C = (int)S.cols, R = (int)S.rows;
+#pragma unroll
+        for (int i = 0; i < PPT; ++i) {
+            const int p = base + i < N ? (int)base + i : 0;
+            const int row = p / C, col = p - row * C;
+            rim[i] = (row == 0 ? R - 1 : row - 1) * C;
+            ric[i] = row * C;
+            rip[i] = (row == R - 1 ? 0 : row + 1) * C;
+            cjm[i] = col == 0 ? C - 1 : col - 1;
+            cjc[i] = col;
+            cjp[i] = col == C - 1 ? 0 : col + 1;
+        }
+    }
 
     auto publish = [&](const double(&x)[PPT], int b) {
+        if constexpr (!CHAIN) {
+#pragma unroll
+            for (int i = 0; i < PPT; ++i) {
+                if (own(i)) {
+                    mir[b * N + base + i] = x[i];
+                }
+            }
+            return;
+        }
         if (cnt > 0) {
             h_first[b * T + t] = x[0];
 #pragma unroll
@@ -145,7 +197,7 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
     };
 
     // slips of step `it` from the state x into y, their reachability (rmask,
-    // s_refill) and publication into exchange buffer it&1
+    // s_flag) and publication into exchange buffer it&1
     int pend = 0;
     auto prepare = [&](int it, const double(&x)[PPT], double(&y)[PPT]) {
         const int b = it & 1;
@@ -182,7 +234,7 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
                 }
             }
             if (refill) {
-                s_refill[b] = it;
+                s_flag[b][0] = it;
             }
         }
         rmask = refill;
@@ -191,17 +243,21 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
 
     auto left_of = [&](int b) -> double { return h_last[b * T + (t == 0 ? Tact - 1 : t - 1)]; };
     auto right_of = [&](int b) -> double { return h_first[b * T + (t == Tact - 1 ? 0 : t + 1)]; };
-    auto interaction = [&](int i, int b, const double(&x)[PPT]) -> double {
+    int lat_b = 0; // lattices: the exchange buffer to read
+    auto interaction = [&](int i, double lft, double rgt, const double(&x)[PPT]) -> double {
         if constexpr (INT == INT_NONE) {
             return 0.0;
+        }
+        else if constexpr (!CHAIN) {
+            return lattice_force_at<INT>(P, mir + lat_b * N, rim[i], ric[i], rip[i], cjm[i], cjc[i], cjp[i], x[i]);
         }
         else {
             double um = 0.0, up = 0.0;
 #pragma unroll
             for (int q = 0; q < PPT; ++q) {
                 if (q == i) {
-                    um = (q == 0) ? left_of(b) : x[q > 0 ? q - 1 : 0];
-                    up = (q == last) ? right_of(b) : x[q + 1 < PPT ? q + 1 : q];
+                    um = (q == 0) ? lft : x[q > 0 ? q - 1 : 0];
+                    up = (q == last) ? rgt : x[q + 1 < PPT ? q + 1 : q];
                 }
             }
             return chain_force<INT>(P, um, x[i], up);
@@ -412,30 +468,64 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
         const int b = it & 1;
         __syncthreads(); // slips of step `it` published; flags and residual sums of step it-1 written
 
+        // everything this step reads from LDS, at once
+        const int flag_refill = s_flag[b][0], flag_nan = s_flag[b][1];
+        const double lft = CHAIN ? left_of(b) : 0.0, rgt = CHAIN ? right_of(b) : 0.0;
+        lat_b = b;
+        double sf = 0.0, sff = 0.0;
+        if constexpr (NW <= 8) {
+            double r0[NW], r1[NW];
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                r0[w] = s_red_d[b ^ 1][w][0];
+                r1[w] = s_red_d[b ^ 1][w][1];
+            }
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                sf += r0[w];
+                sff += r1[w];
+            }
+        }
+        else { // one value per lane, summed over each row of 16 lanes
+            double z = s_red_d[b ^ 1][lane & 15][(lane >> 4) & 1];
+            z += dpp_move<0xB1, 0xf>(z);
+            z += dpp_move<0x4E, 0xf>(z);
+            z += dpp_move<0x141, 0xf>(z);
+            z += dpp_move<0x140, 0xf>(z);
+            sf = lane_d(z, 0);
+            sff = lane_d(z, 16);
+        }
+
         // decisions on step it-1 (detail.h:1771-1787 with the StopList as counters)
         if (it > 1) {
-            if (uniform_i(s_nan[(it - 1) & 1]) == it - 1) {
+            if (uniform_i(flag_nan) == it - 1) {
                 status = ST_NAN;
                 return false;
             }
-            const int pb = (it - 1) & 1;
-            double sf = 0.0, sff = 0.0;
-            for (int w = 0; w < nw; ++w) {
-                sf += s_red_d[pb][w][0];
-                sff += s_red_d[pb][w][1];
-            }
             sf = uniform_d(sf);
             sff = uniform_d(sff);
-            const double rf = __builtin_sqrt(sf), rff = __builtin_sqrt(sff);
-            const double r = (rff != 0.0) ? rf / rff : rf;
-            below = !(r >= ra.tol) ? below + 1 : 0;
-            below2 = !(r >= ra.tol2) ? below2 + 1 : 0;
-            dec = !(r >= prev) ? dec + 1 : 0;
-            prev = r;
-            const int64_t nt = ra.niter_tol;
-            if (nt <= 0 || (dec >= nt - 1 && below >= nt) || below2 >= nt) {
-                status = ST_CONVERGED;
-                return false;
+            if (clear_of_tol && sf > tol_clear * sff && sff > 0.0) {
+                // r >= tol for certain: no root or quotient. The counters
+                // start again; what dec and prev were does not matter, since
+                // only decreasing pairs within the last niter_tol residuals,
+                // all of them below tol, count towards a stop.
+                below = 0;
+                below2 = 0;
+                dec = 0;
+                prev = __builtin_inf();
+            }
+            else {
+                const double rf = __builtin_sqrt(sf), rff = __builtin_sqrt(sff);
+                const double r = (rff != 0.0) ? rf / rff : rf;
+                below = !(r >= ra.tol) ? below + 1 : 0;
+                below2 = !(r >= ra.tol2) ? below2 + 1 : 0;
+                dec = !(r >= prev) ? dec + 1 : 0;
+                prev = r;
+                const int64_t nt = ra.niter_tol;
+                if (nt <= 0 || (dec >= nt - 1 && below >= nt) || below2 >= nt) {
+                    status = ST_CONVERGED;
+                    return false;
+                }
             }
             if (it - 1 >= maxit) {
                 status = ST_MAXITER;
@@ -445,7 +535,7 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
         if (it > limit) {
             return false;
         }
-        if (uniform_i(s_refill[b]) == it) {
+        if (uniform_i(flag_refill) == it) {
             status = ST_REFILL;
             return false;
         }
@@ -469,8 +559,7 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
                         const int32_t j = jl[i] + 1;
                         const double hn = yn_r[NEXT ? i : 0];
                         jl[i] = j;
-                        set_bounds(i, hi, hn);
-                        ym[i] = 0.5 * (hi + hn);
+                        set_well(i, hi, hn);
                         yn_r[NEXT ? i : 0] = next_right(row, j);
                     }
                     else {
@@ -487,8 +576,7 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
                         }
                         if (lo <= z && z < hi) {
                             jl[i] = j;
-                            set_bounds(i, lo, hi);
-                            ym[i] = 0.5 * (lo + hi);
+                            set_well(i, lo, hi);
                             if constexpr (NEXT) {
                                 yn_r[i] = next_right(row, j);
                             }
@@ -497,19 +585,18 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
                 }
             }
             if (nanf) {
-                s_nan[b] = it;
+                s_flag[b ^ 1][1] = it; // read by step it + 1
             }
         }
 
         // the reference's three velocity / acceleration passes (detail.h:1552-1565)
         // and the residual's two squared norms (own particles, in register order)
-        double sf = 0.0, sff = 0.0;
+        sf = 0.0;
+        sff = 0.0;
 #pragma unroll
         for (int i = 0; i < PPT; ++i) {
-            const double fi = interaction(i, b, x);
-            double lo, hi;
-            bounds(i, lo, hi);
-            const double fp = potential_force_mid<POT>(P, x[i], lo, hi, ym[i]);
+            const double fi = interaction(i, lft, rgt, x);
+            const double fp = well_force(i, x[i]);
             const double ff = kf * (uf - x[i]);
             const double sum3 = ff + fp + fi;
             const double vn = v[i], an = a[i];
@@ -529,11 +616,9 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
                 sff += ff * ff;
             }
         }
-        sf = wave_sum(sf);
-        sff = wave_sum(sff);
-        if (lane == 0) {
-            s_red_d[b][wave][0] = sf;
-            s_red_d[b][wave][1] = sff;
+        sf = wave_sum2(sf, sff);
+        if ((lane & 31) == 31) {
+            s_red_d[b][wave][lane >> 5] = sf;
         }
         if (pad_wave) { // padding registers stay at rest
             __asm__ volatile("");
@@ -573,10 +658,9 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
                 W.a[p] = a[i];
                 W.ls.jloc[p] = jl[i];
                 if (forces) {
-                    const double fi = interaction(i, fb, x);
-                    double lo, hi;
-                    bounds(i, lo, hi);
-                    const double fp = potential_force_mid<POT>(P, x[i], lo, hi, ym[i]);
+                    lat_b = fb;
+                    const double fi = CHAIN ? interaction(i, left_of(fb), right_of(fb), x) : interaction(i, 0.0, 0.0, x);
+                    const double fp = well_force(i, x[i]);
                     const double ff = kf * (uf - x[i]);
                     const double fd = meta * v[i];
                     W.f_int[p] = fi;
@@ -597,12 +681,19 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
     // state; the step budget, max_iter and a NaN end the launch.
     bool complete = false;
     for (;;) {
-        const int64_t budget = ra.max_steps - launch_done;
+        int64_t budget = ra.max_steps - launch_done;
+        if (plain) {
+            const int64_t room = rs->target - ev_done0;
+            budget = room < budget ? room : budget;
+        }
         limit = uniform_i((int)(budget > 0 ? budget : 0));
         const SysView& W = V();
 #pragma unroll
         for (int i = 0; i < PPT; ++i) {
-            sa[i] = v[i] = a[i] = ym[i] = 0.0;
+            sa[i] = v[i] = a[i] = c0[i] = 0.0;
+            if constexpr (WC1) {
+                c1[i] = 0.0;
+            }
             if constexpr (!INPLACE) {
                 sb[i] = 0.0;
             }
@@ -617,26 +708,24 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
                 v[i] = W.v[p];
                 a[i] = W.a[p];
                 jl[i] = W.ls.jloc[p];
-                const double lo = Y[p * nch + jl[i]], hi = Y[p * nch + jl[i] + 1];
-                set_bounds(i, lo, hi);
-                ym[i] = 0.5 * (lo + hi);
+                set_well(i, Y[p * nch + jl[i]], Y[p * nch + jl[i] + 1]);
                 if constexpr (NEXT) {
                     yn_r[i] = next_right(Y + p * nch, jl[i]);
                 }
             }
         }
-        if (t == 0) {
-            s_nan[0] = 0;
-            s_nan[1] = 0;
-            s_refill[0] = 0;
-            s_refill[1] = 0;
+        if (t < 4) {
+            s_flag[t >> 1][t & 1] = 0;
+        }
+        for (int w = t; w < 4 * NW; w += T) {
+            (&s_red_d[0][0][0])[w] = 0.0;
         }
         status = complete ? ST_DONE : ST_RUNNING;
         __syncthreads(); // flags cleared before any thread sets them
         publish(sa, 0);
         int it = 1;
         const bool minimising = !complete && phase == QS_MINIMISE;
-        maxit = s_qa.max_iter - ev_done0;
+        maxit = plain ? 0x7fffffffffffffffLL : s_qa.max_iter - ev_done0;
         if (minimising) {
             if constexpr (INPLACE) {
                 prepare(1, sa, sa);
@@ -669,6 +758,16 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
         }
         const int done = it - 1;
         launch_done += done;
+        if (plain && status == ST_CONVERGED) { // quench (detail.h:1782) and return
+#pragma unroll
+            for (int i = 0; i < PPT; ++i) {
+                v[i] = 0.0;
+                a[i] = 0.0;
+            }
+            finish(sa, done);
+            ev_done0 += done;
+            break;
+        }
         if (status == ST_CONVERGED || (!complete && !minimising)) {
             if (status == ST_CONVERGED) { // quench (detail.h:1782), then record the event
 #pragma unroll

@@ -98,6 +98,26 @@ __device__ __forceinline__ double wave_sum(double x)
     return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
+// Sums of x and of y over the 64 lanes at once, in a fixed order: the upper
+// half of x and the lower half of y change places, so that lanes 0..31 hold
+// pair sums of x and lanes 32..63 of y, then both halves go through the lane
+// moves of wave_sum together (half its instructions). Lane 31 ends with the
+// total of x and lane 63 with that of y.
+__device__ __forceinline__ double wave_sum2(double x, double y)
+{
+    const uint64_t bx = __builtin_bit_cast(uint64_t, x), by = __builtin_bit_cast(uint64_t, y);
+    const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)bx, (uint32_t)by, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(bx >> 32), (uint32_t)(by >> 32), false, false);
+    double z = __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
+               __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
+    z += dpp_move<0xB1, 0xf>(z);
+    z += dpp_move<0x4E, 0xf>(z);
+    z += dpp_move<0x141, 0xf>(z);
+    z += dpp_move<0x140, 0xf>(z);
+    z += dpp_move<0x142, 0xa>(z); // row_bcast:15 into rows 1 and 3
+    return z;
+}
+
 __device__ __forceinline__ long long wave_sum_i(long long x)
 {
     for (int off = 32; off > 0; off >>= 1) {
@@ -451,7 +471,8 @@ __device__ __forceinline__ void resident_body(const SysView* __restrict__ views,
             else {
                 const double* U = mir + (int64_t)b * N;
                 const int64_t p = base + i;
-                return lattice_force<INT>(S, [&](int64_t q) { return U[q]; }, p / S.cols, p % S.cols);
+                const uint32_t q32 = (uint32_t)p, c32 = (uint32_t)S.cols, row = q32 / c32; // (resident sizes)
+                return lattice_force<INT>(S, [&](int64_t q) { return U[q]; }, row, q32 - row * c32);
             }
         };
 

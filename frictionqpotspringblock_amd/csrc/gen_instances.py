@@ -4,8 +4,8 @@ header fq_res_units.hpp that declares them.
 Each unit instantiates, for its (potential, interaction, forcing) classes and
 the variant table of each, k_resident<POT, INT, EXT, PPT, MAXT> (all modes),
 for chains k_flow<POT, INT, EXT, PPT, MAXT> (timeSteps / flowSteps), and,
-without external forcing, the quasistatic driver (k_quasi_chain for chains,
-k_quasi otherwise); it exposes
+without external forcing, the quasistatic driver (k_quasi_chain; k_quasi for
+long range and large lattices); it exposes
 launch_resident_<unit>(), launch_flow_<unit>(), launch_quasi_<unit>() and
 resident_variants_<unit>(). Small units let hipcc compile them in parallel.
 The build (build_ext.py) generates them before compiling; by hand:
@@ -19,6 +19,7 @@ import os
 HOT = [(1, 1024), (2, 1024), (4, 1024), (4, 512), (8, 1024), (8, 512), (8, 256), (16, 512), (16, 256)]
 STD = [(1, 1024), (2, 1024), (4, 1024), (8, 1024), (8, 512), (16, 512), (16, 256)]
 MIRROR = [(1, 1024), (2, 1024), (4, 1024), (8, 1024)]
+LATTICE = [(1, 1024), (2, 1024), (4, 1024), (4, 512), (8, 1024), (8, 512)]
 
 CHAINS = {"INT_NONE", "INT_LAPLACE1D", "INT_QUARTIC1D", "INT_QUARTICGRADIENT1D"}
 
@@ -35,7 +36,8 @@ UNITS = {
     ),
     "cuspy_field": (
         "POT_CUSPY",
-        [("INT_LONGRANGE1D", [0, 1], MIRROR), ("INT_LAPLACE2D", [0], MIRROR), ("INT_QUARTICGRADIENT2D", [0], MIRROR)],
+        [("INT_LONGRANGE1D", [0, 1], MIRROR), ("INT_LAPLACE2D", [0], LATTICE),
+         ("INT_QUARTICGRADIENT2D", [0], LATTICE)],
     ),
     "semismooth": ("POT_SEMISMOOTH", [("INT_LAPLACE1D", [0], STD), ("INT_QUARTIC1D", [0], STD), ("INT_NONE", [0], STD)]),
     "smooth": ("POT_SMOOTH", [("INT_LAPLACE1D", [0], STD), ("INT_QUARTIC1D", [0], STD), ("INT_NONE", [0], STD)]),
@@ -64,8 +66,12 @@ def quasi_launcher(name, pot, ints):
             continue
         for ppt, mt in variants:
             out.append(f"    if (inter == {it} && ppt == {ppt} && maxt == {mt}) {{")
-            if it in CHAINS:  # k_quasi_chain (fq_quasi.hpp)
+            # k_quasi_chain (fq_quasi.hpp); lattices with 4 or more particles
+            # per thread and 128 registers would spill there
+            if it in CHAINS or (it != "INT_LONGRANGE1D" and (mt <= 512 or ppt <= 2)):
                 forms = [("true", "true", "unit_mass && full"), ("true", "false", "unit_mass")] if name in QUASI_FULL else []
+                if it not in CHAINS:
+                    forms = [("true", "false", "unit_mass")]
                 for unit, full, cond in forms:
                     k = f"k_quasi_chain<{pot}, {it}, {ppt}, {mt}, {unit}, {full}>"
                     out.append(f"        if ({cond}) {{")
@@ -77,6 +83,9 @@ def quasi_launcher(name, pot, ints):
                 k = f"k_quasi_chain<{pot}, {it}, {ppt}, {mt}, false, false>"
             else:
                 k = f"k_quasi<{pot}, {it}, {ppt}, {mt}, false>"
+                out.append("        if (qa.plain) { // the protocol only: minimise runs on k_resident")
+                out.append("            return false;")
+                out.append("        }")
             out.append(f"        hipLaunchKernelGGL(({k}), dim3(nsys), dim3(threads), lds, stream, views, ra, qa);")
             out.append("        return true;")
             out.append("    }")

@@ -144,3 +144,55 @@ def test_longrange_product(N):
     bound = 8.0 * eps * np.log2(4 * N) * np.linalg.norm(g) * w[:, None]
     bound = np.maximum(bound, 2.0 * N * eps * g.sum() * np.abs(u - u[:, :1]).max()) if N < 257 or N == 8193 else bound
     assert np.all(np.abs(b.f_interactions - f) <= bound)
+
+
+CLASSES = [("Line1d", "System_Cuspy_Laplace", dict(k_interactions=1.0)),
+           ("Line1d", "System_SemiSmooth_Laplace", dict(k_interactions=1.0, kappa=1.0)),
+           ("Line1d", "System_Smooth_Laplace", dict(k_interactions=1.0)),
+           ("Line1d", "System_Cuspy_Quartic", dict(a1=1.0, a2=5.0)),
+           ("Particles", "System_Cuspy", {})]
+
+
+def _pair(sub, cls, shape, extra, **more):
+    import frictionqpotspringblock_amd as fq
+
+    kw = _kw(int(np.prod(shape)), **more)
+    del kw["k_interactions"]
+    kw.update(extra, shape=list(shape))
+    return getattr(getattr(fq, sub), cls)(**kw), getattr(getattr(pyoracle, sub), cls)(**kw)
+
+
+def _minimise(g, o):
+    """Minimisations that end by their step limit, by convergence from a
+    moving state, and after a uniform displacement."""
+    v = np.random.default_rng(g.u.size).normal(size=g.u.shape)
+    for s in (g, o):
+        s.v = v
+    assert g.minimise(max_iter=7, max_iter_is_error=False) == o.minimise(max_iter=7, max_iter_is_error=False)
+    for k in ("u", "v", "a", "f"):
+        assert np.array_equal(getattr(g, k), getattr(o, k)), k
+    assert g.minimise() == o.minimise()
+    assert g.inc == o.inc
+    for s in (g, o):
+        s.eventDrivenStep(1e-3, True)
+    assert g.minimise(tol=1e-3, niter_tol=3) == o.minimise(tol=1e-3, niter_tol=3)
+    assert g.inc == o.inc
+    for k in ("u", "v", "f", "f_potential", "f_interactions"):
+        assert np.array_equal(getattr(g, k), getattr(o, k)), k
+    assert np.array_equal(g.chunk.index_at_align, o.chunk.index_at_align)
+    assert np.array_equal(g.chunk.start, o.chunk.start)
+
+
+@pytest.mark.parametrize("N", [3, 65, 511, 513, 2047, 2049, 4096, 4097])
+@pytest.mark.parametrize("sub,cls,extra", CLASSES, ids=[c[1] for c in CLASSES])
+def test_minimise_chains(sub, cls, extra, N):
+    """minimise of single chains on both sides of the sizes at which the launch
+    shape changes; masses other than 1 with the odd sizes."""
+    _minimise(*_pair(sub, cls, [N], extra, m=2.0 if N in (65, 2049) else 1.0))
+
+
+@pytest.mark.parametrize("shape", [(3, 4), (5, 103), (19, 27), (45, 45), (41, 50), (64, 64), (65, 64)])
+@pytest.mark.parametrize("cls,extra", [("System_Cuspy_Laplace", dict(k_interactions=1.0)),
+                                       ("System_Cuspy_QuarticGradient", dict(k2=1.0, k4=1.0))])
+def test_minimise_lattices(cls, extra, shape):
+    _minimise(*_pair("Line2d", cls, shape, extra, m=2.0 if shape[0] == 41 else 1.0))
