@@ -419,24 +419,32 @@ struct Group {
         if (nv <= 0) {
             throw Error("no resident kernel for this potential / interaction / external combination");
         }
-        // Cuspy-Laplace chains (no external forcing) without a requested
-        // shape: 4 particles per thread while the systems' wavefronts fit two
-        // per SIMD (a workgroup's step is shortest there: a lone 1024-chain's
-        // quasistatic step takes 2.37 us, against 2.63 us with 2 x 512 and
-        // 3.04 us with 1 x 1024), else 8 (the most particle-steps per unit of
-        // time with many systems: 1024 chains of 1024 particles), when a
-        // variant of at most 512 threads holds the largest system that way
-        // (variants of 1024 threads have 128 registers per thread and spill).
-        // The other classes keep the fewest particles per thread: their
-        // costlier forces spill at 4 particles per thread.
-        if (want_ppt == 0 && want_threads == 0 && pot == FQSB_POT_CUSPY && inter == FQSB_INT_LAPLACE1D &&
-            ext == FQSB_EXT_NONE) {
+        // Chains and lattices without external forcing and without a requested shape:
+        // variants of at most 512 threads (those of 1024 have 128 registers
+        // per thread, which 4 particles per thread exceed), 4 particles per
+        // thread up to 2048 particles, else 8 (a quench and a kick of 100
+        // chains of 3000, 4 x 768 / 8 x 384: SemiSmooth-Laplace 43 / 7.8 ms,
+        // Smooth-Laplace 104 / 39 ms, Cuspy-Quartic 10.7 / 7.0 ms; of 200
+        // chains of 1537, 2 x 832 / 4 x 448 / 8 x 256: 7.0 / 5.2 / 5.7 ms,
+        // 25 / 21 / 24 ms, 5.6 / 4.7 / 5.1 ms). Many systems (their
+        // wavefronts with 4 particles per thread exceed two per SIMD) take 8
+        // as well, the most particle-steps per unit of time, but for Smooth,
+        // whose sine spills (1024 chains of 1024, 4 x 256 / 8 x 128: Cuspy 4.9
+        // / 4.0 ms, SemiSmooth 8.2 / 7.5 ms, Smooth 26 / 31 ms). Up to 512
+        // particles the classes beside Cuspy-Laplace have one particle per
+        // thread (64 chains of 300, 1 x 320 / 4 x 128: SemiSmooth 2.2 / 2.9
+        // ms, Smooth 5.3 / 8.3 ms). Lattices: 100 of 40 x 50, 2 x 1024 / 4 x
+        // 512: 4.8 / 3.7 ms; 100 of 50 x 50, 4 x 640 / 8 x 320: 14.5 / 6.3 ms;
+        // 600 of 30 x 30, 4 x 256 / 8 x 128: 5.7 / 6.1 ms.
+        const bool cuspy_laplace = pot == FQSB_POT_CUSPY && inter == FQSB_INT_LAPLACE1D;
+        const bool lattice = inter == FQSB_INT_LAPLACE2D || inter == FQSB_INT_QUARTICGRADIENT2D;
+        if (want_ppt == 0 && want_threads == 0 && inter != FQSB_INT_LONGRANGE1D && ext == FQSB_EXT_NONE && (cuspy_laplace || N > 512)) {
             for (const int p : {4, 8}) {
                 const int thr = (int)((((N + p - 1) / p) + 63) / 64 * 64);
                 if (thr > 1024 || fq::resident_lds(inter, N, thr) > lds_limit) {
                     continue;
                 }
-                if (p == 4 && R * (int64_t)(thr / 64) > 2 * 4 * (int64_t)cus) {
+                if (p == 4 && !lattice && pot != FQSB_POT_SMOOTH && R * (int64_t)(thr / 64) > 2 * 4 * (int64_t)cus) {
                     continue;
                 }
                 int best = -1;

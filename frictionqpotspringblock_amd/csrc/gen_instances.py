@@ -17,7 +17,7 @@ import os
 
 # (particles per thread, max threads per workgroup) variants
 HOT = [(1, 1024), (2, 1024), (4, 1024), (4, 512), (8, 1024), (8, 512), (8, 256), (16, 512), (16, 256)]
-STD = [(1, 1024), (2, 1024), (4, 1024), (8, 1024), (8, 512), (16, 512), (16, 256)]
+STD = [(1, 1024), (2, 1024), (4, 1024), (4, 512), (8, 1024), (8, 512), (16, 512), (16, 256)]
 MIRROR = [(1, 1024), (2, 1024), (4, 1024), (8, 1024)]
 LATTICE = [(1, 1024), (2, 1024), (4, 1024), (4, 512), (8, 1024), (8, 512)]
 
