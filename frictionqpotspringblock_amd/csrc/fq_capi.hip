@@ -621,6 +621,10 @@ struct Group {
         const bool blocks = tile_k > 0 && tile_part_k != nullptr && fq::tile_block_supported(pot, inter);
         auto normalise = [&] {
             if (!fq::launch_tile_finish(pot, inter, views, tiles, ntiles, stream)) {
+        bool unit_mass = true;
+        for (const auto& S : hviews) {
+            unit_mass &= S.inv_m == 1.0;
+        }
                 throw Error("no tiled kernel for this potential / interaction");
             }
             HIPC(hipGetLastError());
@@ -635,7 +639,7 @@ struct Group {
                 const int K = block_steps();
                 for (uint64_t s = 0; s < (nb + (uint64_t)K - 1) / (uint64_t)K; ++s) {
                     if (!fq::launch_tile_block(pot, inter, views, tb_tiles, tb_ntiles, tile_part_k, tile_fail, ra, K,
-                                               tb_lds, stream)) {
+                                               tb_lds, unit_mass, stream)) {
                         throw Error("no blocked tile kernel for this potential / interaction");
                     }
                     HIPC(hipGetLastError());

@@ -57,12 +57,18 @@ bool tile_block_supported(int pot, int inter)
 }
 
 bool launch_tile_block(int pot, int inter, const SysView* views, const TileDesc* tiles, int ntiles, double* part,
-                       int32_t* tfail, const RunArgs& ra, int K, size_t lds, hipStream_t stream)
+                       int32_t* tfail, const RunArgs& ra, int K, size_t lds, bool unit_mass, hipStream_t stream)
 {
 #define FQ_BLOCK(P, I)                                                                                         \
     if (pot == P && inter == I) {                                                                              \
-        hipLaunchKernelGGL((k_tile_block<P, I>), dim3((unsigned)ntiles), dim3(TB_THREADS), 0, stream, views,  \
-                           tiles, part, tfail, ra, K);                                                         \
+        if (unit_mass) {                                                                                       \
+            hipLaunchKernelGGL((k_tile_block<P, I, true>), dim3((unsigned)ntiles), dim3(TB_THREADS), 0,        \
+                               stream, views, tiles, part, tfail, ra, K);                                      \
+        }                                                                                                      \
+        else {                                                                                                 \
+            hipLaunchKernelGGL((k_tile_block<P, I, false>), dim3((unsigned)ntiles), dim3(TB_THREADS), 0,       \
+                               stream, views, tiles, part, tfail, ra, K);                                      \
+        }                                                                                                      \
         return true;                                                                                           \
     }
 #define FQ_BLOCK2D(P, I)                                                                                       \

@@ -327,22 +327,27 @@ __device__ __forceinline__ int tb_steps(const RunState* rs, int K)
     return (int)(room < K ? (room > 0 ? room : 0) : K);
 }
 
-template <int POT, int INT>
+// The step is that of k_flow (straight-line over the registers of a thread,
+// padding at rest in an unbounded well, walks behind one branch, constants of
+// the well kept). The residual sums of a step go to LDS per wavefront and to
+// memory after the block. UNIT: every system of the group has m = 1.
+template <int POT, int INT, bool UNIT>
 __global__ void __launch_bounds__(TB_THREADS) k_tile_block(const SysView* __restrict__ views,
                                                            const TileDesc* __restrict__ tiles,
                                                            double* __restrict__ part, int32_t* __restrict__ tfail,
                                                            RunArgs ra, int K)
 {
     constexpr int PPT = TB_PPT;
+    constexpr int NW = TB_THREADS / 64;
     __shared__ double s_first[2][TB_THREADS];
     __shared__ double s_last[2][TB_THREADS];
-    __shared__ double s_red[2][TB_THREADS / 64][2];
+    __shared__ double s_red[TB_KMAX][NW][2];
     __shared__ int s_fail;
     const TileDesc td = tiles[blockIdx.x];
     const SysView& S = views[td.sys];
     const SysView P = S; // parameters in registers (no reload after each barrier)
     const RunState* const rs = S.rs;
-    const int t = threadIdx.x, T = blockDim.x, lane = t & 63, wave = t >> 6, nw = T >> 6;
+    const int t = threadIdx.x, T = blockDim.x, lane = t & 63, wave = t >> 6;
     const int32_t status = uniform_i(rs->status);
     if (status != ST_RUNNING && status != ST_BUDGET) {
         return;
@@ -371,27 +376,39 @@ __global__ void __launch_bounds__(TB_THREADS) k_tile_block(const SysView* __rest
     const bool mini = ra.mode == MODE_MINIMISE;
 
     // extended index i = t * PPT + k, global particle (p0 - K + i) mod N
-    const int64_t base = (int64_t)t * PPT;
+    const int base = t * PPT;
     const int cnt = (int)(next - base >= PPT ? PPT : (next - base > 0 ? next - base : 0));
     const int Tlast = (int)((next - 1) / PPT); // thread holding the last particle
+    const bool pad_wave = uniform_i(__any(cnt < PPT)) != 0;
     double u[PPT], v[PPT], a[PPT], yl[PPT], yr[PPT];
-    // constants of the current well (well_consts), kept for SemiSmooth: they
-    // save its two divisions per step (7-13 % of the kernel's time). Smooth's
-    // one division would cost more in registers (occupancy) than it saves;
-    // Cuspy's mid-point is a single addition and multiplication.
-    constexpr bool WC = POT == POT_SEMISMOOTH;
-    double wc0[PPT], wc1[PPT];
+    constexpr bool WC1 = POT != POT_CUSPY;
+    double c0[PPT], c1[WC1 ? PPT : 1];
     int32_t jl[PPT];
-    auto gidx = [&](int k) -> int64_t { // global index of local particle k (periodic)
-        int64_t q = (p0 - K + base + k) % N;
+    uint32_t own = 0; // registers that hold the tile's own particles
+    auto set_well = [&](int k, double lo, double hi) {
+        yl[k] = lo;
+        yr[k] = hi;
+        double w1;
+        well_consts<POT>(P, lo, hi, c0[k], w1);
+        if constexpr (WC1) {
+            c1[k] = w1;
+        }
+    };
+    auto gidx = [&](int64_t i) -> int64_t { // global index of extended particle i (periodic)
+        int64_t q = (p0 - K + i) % N;
         return q < 0 ? q + N : q;
     };
 #pragma unroll
     for (int k = 0; k < PPT; ++k) {
-        u[k] = v[k] = a[k] = yl[k] = yr[k] = wc0[k] = wc1[k] = 0.0;
+        u[k] = v[k] = a[k] = c0[k] = 0.0;
+        if constexpr (WC1) {
+            c1[k] = 0.0;
+        }
+        yl[k] = -__builtin_inf();
+        yr[k] = __builtin_inf();
         jl[k] = 0;
         if (k < cnt) {
-            const int64_t q = gidx(k);
+            const int64_t q = gidx(base + k);
             u[k] = Uc[q];
             v[k] = Vc[q];
             a[k] = Ac[q];
@@ -400,11 +417,8 @@ __global__ void __launch_bounds__(TB_THREADS) k_tile_block(const SysView* __rest
             // is one word, either value is a well of the window, and the
             // first walk finds the particle's well from either)
             jl[k] = L.jloc[q];
-            yl[k] = L.y[q * nch + jl[k]];
-            yr[k] = L.y[q * nch + jl[k] + 1];
-            if constexpr (WC) {
-                well_consts<POT>(P, yl[k], yr[k], wc0[k], wc1[k]);
-            }
+            set_well(k, L.y[q * nch + jl[k]], L.y[q * nch + jl[k] + 1]);
+            own |= base + k >= K && base + k < K + n ? 1u << k : 0u;
         }
     }
     if (t == 0) {
@@ -417,59 +431,47 @@ __global__ void __launch_bounds__(TB_THREADS) k_tile_block(const SysView* __rest
     for (s = 1; s <= Ke; ++s) {
         const int b = s & 1;
         double* const x = u; // position update in place: x = u + dt v + dt^2/2 a
+        int out = 0;
 #pragma unroll
         for (int k = 0; k < PPT; ++k) {
             x[k] = u[k] + dt * v[k] + c2 * a[k];
+            out |= !(yl[k] <= x[k] && x[k] < yr[k]);
         }
         if (cnt > 0) {
+            s_first[b][t] = x[0];
+            double xl = x[PPT - 1];
+            if (pad_wave) {
 #pragma unroll
-            for (int k = 0; k < PPT; ++k) {
-                if (k == 0) {
-                    s_first[b][t] = x[0];
-                }
-                if (k == cnt - 1) {
-                    s_last[b][t] = x[k];
+                for (int k = 0; k < PPT - 1; ++k) {
+                    xl = k == cnt - 1 ? x[k] : xl;
                 }
             }
+            s_last[b][t] = xl;
         }
         __syncthreads();
-        if (mini && s > 1 && t == 0) { // residual sums of step s - 1
-            double a0 = 0.0, a1 = 0.0;
-            for (int w = 0; w < nw; ++w) {
-                a0 += s_red[b ^ 1][w][0];
-                a1 += s_red[b ^ 1][w][1];
-            }
-            part[((int64_t)blockIdx.x * K + (s - 2)) * 2] = a0;
-            part[((int64_t)blockIdx.x * K + (s - 2)) * 2 + 1] = a1;
-        }
-        if ((uniform_i(s_fail) >> 2) < s) {
+        const int failed = s_fail;
+        // open ends of the extended segment: any finite value (their own)
+        const double left = s_last[b][t == 0 ? 0 : t - 1];
+        const double right = s_first[b][t >= Tlast ? t : t + 1];
+        if ((uniform_i(failed) >> 2) < s) {
             break; // a particle of the tile failed at an earlier step
         }
         if (ra.flow) {
             uf = uf + dv;
         }
-        double xlast = x[0]; // (selected, not indexed: no scratch)
+        if (out) { // rare: some slip left its well (or is NaN)
+            int fail = 0;
+            int bq = base; // (opaque: the addresses of this path stay in it)
+            __asm__ volatile("" : "+v"(bq));
 #pragma unroll
-        for (int k = 1; k < PPT; ++k) {
-            xlast = k == cnt - 1 ? x[k] : xlast;
-        }
-        // open ends of the extended segment: any finite value
-        const double left = (t == 0) ? x[0] : s_last[b][t - 1];
-        const double right = (t == Tlast) ? xlast : s_first[b][t + 1 < T ? t + 1 : t];
-        double sf = 0.0, sff = 0.0;
-        int fail = 0;
-#pragma unroll
-        for (int k = 0; k < PPT; ++k) {
-            if (k < cnt) {
-                const int64_t i = base + k;
-                const bool exact = i >= s - 1 && i < next - s + 1; // the state of step s - 1 is exact
-                const bool own = i >= K && i < K + n;
+            for (int k = 0; k < PPT; ++k) {
                 const double xk = x[k];
-                if (own && __builtin_isnan(xk)) {
+                const bool mine = (own >> k) & 1u;
+                if (mine && __builtin_isnan(xk)) {
                     fail |= TILE_FLAG_NAN;
                 }
-                if (exact && !(yl[k] <= xk && xk < yr[k]) && __builtin_isfinite(xk)) {
-                    const double* row = L.y + gidx(k) * nch;
+                if (!(yl[k] <= xk && xk < yr[k]) && __builtin_isfinite(xk)) {
+                    const double* row = L.y + gidx(bq + k) * nch;
                     int32_t j = jl[k];
                     double lo = yl[k], hi = yr[k];
                     while (xk >= hi && j < jmax) {
@@ -484,87 +486,93 @@ __global__ void __launch_bounds__(TB_THREADS) k_tile_block(const SysView* __rest
                     }
                     if (lo <= xk && xk < hi) {
                         jl[k] = j;
-                        yl[k] = lo;
-                        yr[k] = hi;
-                        if constexpr (WC) {
-                            well_consts<POT>(P, lo, hi, wc0[k], wc1[k]);
-                        }
+                        set_well(k, lo, hi);
                     }
-                    else if (own) {
+                    else if (mine) {
                         fail |= TILE_FLAG_REFILL;
                     }
                 }
-                double fi;
-                if constexpr (INT == INT_NONE) {
-                    fi = 0.0;
-                }
-                else {
-                    double um = 0.0, up = 0.0;
+            }
+            if (fail) { // a refill before a NaN of the same step
+                atomicMin(&s_fail, (s << 2) | ((fail & TILE_FLAG_REFILL) ? TILE_FLAG_REFILL : TILE_FLAG_NAN));
+            }
+        }
+        double sf = 0.0, sff = 0.0;
 #pragma unroll
-                    for (int q = 0; q < PPT; ++q) {
-                        if (q == k) {
-                            um = (q == 0) ? left : x[q > 0 ? q - 1 : 0];
-                            up = (q == cnt - 1) ? right : x[q + 1 < PPT ? q + 1 : q];
-                        }
-                    }
-                    fi = chain_force<INT>(P, um, xk, up);
+        for (int k = 0; k < PPT; ++k) {
+            const double xk = x[k];
+            double fi;
+            if constexpr (INT == INT_NONE) {
+                fi = 0.0;
+            }
+            else {
+                const double um = k == 0 ? left : x[k > 0 ? k - 1 : 0];
+                double up = k == PPT - 1 ? right : x[k + 1 < PPT ? k + 1 : k];
+                if (pad_wave) {
+                    up = k == cnt - 1 ? right : up;
                 }
-                const double fp = WC ? potential_force_wc<POT>(P, xk, yl[k], yr[k], wc0[k], wc1[k])
-                                     : potential_force<POT>(P, xk, yl[k], yr[k]);
-                const double ff = kf * (uf - xk);
-                const double sum3 = ff + fp + fi;
-                const double vn = v[k], an = a[k];
-                double vv = vn + dt * an;
-                double f = sum3 + meta * vv;
-                double aa = f * inv_m;
-                vv = vn + hdt * (an + aa);
-                f = sum3 + meta * vv;
-                aa = f * inv_m;
-                vv = vn + hdt * (an + aa);
-                f = sum3 + meta * vv;
-                aa = f * inv_m;
-                v[k] = vv;
-                a[k] = aa;
-                if (own) {
-                    sf += f * f;
-                    sff += ff * ff;
+                fi = chain_force<INT>(P, um, xk, up);
+            }
+            const double fp = potential_force_wc<POT>(P, xk, yl[k], yr[k], c0[k], c1[WC1 ? k : 0]);
+            const double ff = kf * (uf - xk);
+            const double sum3 = ff + fp + fi;
+            const double vn = v[k], an = a[k];
+            double vv = vn + dt * an;
+            double f = sum3 + meta * vv;
+            double aa = UNIT ? f : f * inv_m;
+            vv = vn + hdt * (an + aa);
+            f = sum3 + meta * vv;
+            aa = UNIT ? f : f * inv_m;
+            vv = vn + hdt * (an + aa);
+            f = sum3 + meta * vv;
+            aa = UNIT ? f : f * inv_m;
+            v[k] = vv;
+            a[k] = aa;
+            const bool mine = (own >> k) & 1u;
+            sf += mine ? f * f : 0.0;
+            sff += mine ? ff * ff : 0.0;
+        }
+        if (pad_wave) { // padding registers stay at rest
+            __asm__ volatile("");
+            if (cnt < PPT) {
+#pragma unroll
+                for (int k = 0; k < PPT; ++k) {
+                    if (k >= cnt) {
+                        v[k] = 0.0;
+                        a[k] = 0.0;
+                    }
                 }
             }
         }
-        if (fail) { // a refill before a NaN of the same step
-            atomicMin(&s_fail, (s << 2) | ((fail & TILE_FLAG_REFILL) ? TILE_FLAG_REFILL : TILE_FLAG_NAN));
-        }
         if (mini) {
-            sf = wave_sum(sf);
-            sff = wave_sum(sff);
-            if (lane == 0) {
-                s_red[b][wave][0] = sf;
-                s_red[b][wave][1] = sff;
+            sf = wave_sum2(sf, sff);
+            if ((lane & 31) == 31) {
+                s_red[s - 1][wave][lane >> 5] = sf;
             }
         }
     }
     const int done = s - 1;
     __syncthreads();
-    if (t == 0) {
-        if (mini && done >= 1 && done == Ke) { // sums of the last step
-            const int lb = done & 1;
-            double a0 = 0.0, a1 = 0.0;
-            for (int w = 0; w < nw; ++w) {
-                a0 += s_red[lb][w][0];
-                a1 += s_red[lb][w][1];
+    if (mini) {
+        for (int q = t; q < 2 * done; q += T) { // residual sums of the steps taken
+            const int st = q >> 1, c = q & 1;
+            double z = 0.0;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                z += s_red[st][w][c];
             }
-            part[((int64_t)blockIdx.x * K + (done - 1)) * 2] = a0;
-            part[((int64_t)blockIdx.x * K + (done - 1)) * 2 + 1] = a1;
+            part[((int64_t)blockIdx.x * K + st) * 2 + c] = z;
         }
+    }
+    if (t == 0) {
         tfail[blockIdx.x] = s_fail;
     }
     // the tile's particles: state after the block into the other buffer (used
     // only if the decision commits all Ke steps), wells in place
 #pragma unroll
     for (int k = 0; k < PPT; ++k) {
-        const int64_t i = base + k;
-        if (k < cnt && i >= K && i < K + n) {
-            const int64_t q = gidx(k);
+        if ((own >> k) & 1u) {
+            const int64_t q = gidx(base + k);
             Un[q] = u[k];
             Vn[q] = v[k];
             An[q] = a[k];

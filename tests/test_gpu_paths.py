@@ -196,3 +196,23 @@ def test_minimise_chains(sub, cls, extra, N):
                                        ("System_Cuspy_QuarticGradient", dict(k2=1.0, k4=1.0))])
 def test_minimise_lattices(cls, extra, shape):
     _minimise(*_pair("Line2d", cls, shape, extra, m=2.0 if shape[0] == 41 else 1.0))
+
+
+@pytest.mark.parametrize("sub,cls,extra", CLASSES[:4], ids=[c[1] for c in CLASSES[:4]])
+def test_tiles_windows_and_forces(sub, cls, extra):
+    """A chain over tiles whose windows move between blocks of steps, and the
+    operations over many workgroups around it (uniform displacement, largest
+    elastic displacement, forces)."""
+    g, o = _pair(sub, cls, [9001], extra, m=2.0 if cls == "System_SemiSmooth_Laplace" else 1.0)
+    for s in (g, o):
+        s.advanceToFixedForce(0.6, allow_plastic=True)
+        s.flowSteps(300, 0.5)
+    assert np.array_equal(g.u, o.u) and np.array_equal(g.f, o.f)
+    assert np.array_equal(g.chunk.start, o.chunk.start) and g.chunk.start.max() > 0
+    assert np.array_equal(g.chunk.data, o.chunk.data)
+    if "_Smooth_" not in cls:
+        for s in (g, o):
+            s.minimise()
+        assert g.maxUniformDisplacement() == o.maxUniformDisplacement()
+        assert g.eventDrivenStep(1e-3, False) == o.eventDrivenStep(1e-3, False)
+        assert np.array_equal(g.u, o.u) and np.array_equal(g.f, o.f)
