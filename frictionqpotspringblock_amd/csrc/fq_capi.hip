@@ -542,16 +542,6 @@ struct Group {
             HIPC(hipGetLastError());
             return;
         }
-        if (!fq::launch_resident(pot, inter, ext, ppt, maxt, threads, lds, views, (int)R, ra, stream)) {
-            throw Error("no resident kernel variant for this launch shape");
-        }
-        HIPC(hipGetLastError());
-    }
-
-    void reset_run(int mode)
-    {
-        for (size_t i = 0; i < hrs.size(); ++i) {
-            auto& r = hrs[i];
         // minimise of chains and lattices: the quasistatic driver's pipelined
         // steps, which decide the same (without activity tracking and forcing)
         if (ra.mode == fq::MODE_MINIMISE && inter != FQSB_INT_LONGRANGE1D && !ra.time_activity &&
@@ -565,6 +555,16 @@ struct Group {
                 return;
             }
         }
+        if (!fq::launch_resident(pot, inter, ext, ppt, maxt, threads, lds, views, (int)R, ra, stream)) {
+            throw Error("no resident kernel variant for this launch shape");
+        }
+        HIPC(hipGetLastError());
+    }
+
+    void reset_run(int mode)
+    {
+        for (size_t i = 0; i < hrs.size(); ++i) {
+            auto& r = hrs[i];
             r.status = (mask && !mask[i]) ? fq::ST_IDLE : fq::ST_RUNNING;
             r.steps = 0;
             r.refilled = 0;
@@ -619,12 +619,12 @@ struct Group {
         }
         HIPC(fq::launch_tile_prologue(views, tiles, ntiles, stream));
         const bool blocks = tile_k > 0 && tile_part_k != nullptr && fq::tile_block_supported(pot, inter);
-        auto normalise = [&] {
-            if (!fq::launch_tile_finish(pot, inter, views, tiles, ntiles, stream)) {
         bool unit_mass = true;
         for (const auto& S : hviews) {
             unit_mass &= S.inv_m == 1.0;
         }
+        auto normalise = [&] {
+            if (!fq::launch_tile_finish(pot, inter, views, tiles, ntiles, stream)) {
                 throw Error("no tiled kernel for this potential / interaction");
             }
             HIPC(hipGetLastError());
