@@ -383,7 +383,7 @@ struct Group {
     void forces(int32_t flags)
     {
         push();
-        if (!fq::launch_forces(pot, inter, ext, views, (int)R, flags, stream)) {
+        if (!fq::launch_forces(pot, inter, ext, views, (int)R, N, flags, stream)) {
             throw Error("no force kernel for this potential / interaction / external combination");
         }
         HIPC(hipGetLastError());
@@ -712,7 +712,7 @@ struct Group {
             todo = (uint64_t)lag;
             if (refill) {
                 normalise();
-                HIPC(fq::launch_refill(views, (int)R, stream));
+                HIPC(fq::launch_refill(views, (int)R, N, stream));
                 ++refills;
                 for (auto& r : hrs) {
                     if (r.status == fq::ST_REFILL) {
@@ -764,7 +764,7 @@ struct Group {
                 more |= (r.status == fq::ST_RUNNING || r.status == fq::ST_BUDGET) && r.steps < r.target;
             }
             if (refill) {
-                HIPC(fq::launch_refill(views, (int)R, stream));
+                HIPC(fq::launch_refill(views, (int)R, N, stream));
                 ++refills;
                 for (auto& r : hrs) {
                     if (r.status == fq::ST_REFILL) {
@@ -1311,7 +1311,7 @@ struct Group {
                 }
             }
             if (refill) {
-                HIPC(fq::launch_refill(views, (int)R, stream));
+                HIPC(fq::launch_refill(views, (int)R, N, stream));
                 HIPC(fq::launch_lr_prologue(views, lb, stream));
                 for (auto& r : hrs) {
                     if (r.status == fq::ST_REFILL) {
@@ -1377,7 +1377,7 @@ struct Group {
             throw Error("Operation not possible.");
         }
         push();
-        if (!fq::launch_max_uniform(pot, views, (int)R, direction, stream)) {
+        if (!fq::launch_max_uniform(pot, views, (int)R, N, direction, stream)) {
             throw Error("maxUniformDisplacement not available");
         }
         HIPC(hipGetLastError());
@@ -1722,7 +1722,7 @@ struct Group {
                 more |= r.status == fq::ST_RUNNING || r.status == fq::ST_BUDGET;
             }
             if (refill) {
-                HIPC(fq::launch_refill(views, (int)R, stream));
+                HIPC(fq::launch_refill(views, (int)R, N, stream));
                 ++refills;
                 for (auto& r : hrs) {
                     if (r.status == fq::ST_REFILL) {
@@ -1755,7 +1755,7 @@ struct Group {
                 }
             }
             push();
-            HIPC(fq::launch_qs_record(views, (int)R, qa, e, begin, stream));
+            HIPC(fq::launch_qs_record(views, (int)R, N, qa, e, begin, stream));
             pull();
         };
         HIPC(hipEventRecord(ev0, stream));

@@ -146,15 +146,18 @@ bool launch_stream(int pot, int inter, int ext, const SysView* views, int nsys, 
 hipError_t launch_landscape_init(const SysView* views, int nsys, int64_t maxN, hipStream_t stream);
 hipError_t launch_restore(const SysView* views, int64_t N, const uint64_t* state, const double* value,
                           const int64_t* index, hipStream_t stream);
-bool launch_forces(int pot, int inter, int ext, const SysView* views, int nsys, int32_t flags, hipStream_t stream);
-bool launch_max_uniform(int pot, const SysView* views, int nsys, int32_t direction, hipStream_t stream);
+// (maxN: particles of the largest system)
+bool launch_forces(int pot, int inter, int ext, const SysView* views, int nsys, int64_t maxN, int32_t flags,
+                   hipStream_t stream);
+bool launch_max_uniform(int pot, const SysView* views, int nsys, int64_t maxN, int32_t direction, hipStream_t stream);
 hipError_t launch_trigger(const SysView* views, int64_t p, double eps, int32_t direction, int32_t do_align,
                           hipStream_t stream);
 hipError_t launch_set_iref(const SysView* views, int nsys, int64_t maxN, hipStream_t stream);
-hipError_t launch_refill(const SysView* views, int nsys, hipStream_t stream);
+hipError_t launch_refill(const SysView* views, int nsys, int64_t maxN, hipStream_t stream);
 hipError_t launch_trigger_each(const SysView* views, int nsys, const int64_t* ps, double eps, int32_t direction,
                                int32_t do_align, hipStream_t stream);
-hipError_t launch_qs_record(const SysView* views, int nsys, const QsArgs& qa, int64_t e, int begin, hipStream_t stream);
+hipError_t launch_qs_record(const SysView* views, int nsys, int64_t maxN, const QsArgs& qa, int64_t e, int begin,
+                            hipStream_t stream);
 // no-passing sweeps over tiles (fq_tile.hip): chains of any length; one call
 // enqueues one sweep (sweep, residual sums, StopList and buffer flip)
 hipError_t launch_np_sweep(const SysView* views, const TileDesc* tiles, int ntiles, int nsys,

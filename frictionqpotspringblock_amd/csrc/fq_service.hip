@@ -1,5 +1,8 @@
 // Launchers of the service kernels (fq_service.hpp).
 #include "fq_launch.hpp"
+
+#include <algorithm>
+
 #include "fq_service.hpp"
 
 namespace fq {
@@ -33,15 +36,25 @@ hipError_t launch_trigger_each(const SysView* views, int nsys, const int64_t* ps
     return hipGetLastError();
 }
 
-hipError_t launch_refill(const SysView* views, int nsys, hipStream_t stream)
+// threads of a reduction over a whole system
+static dim3 sum_threads(int64_t maxN)
 {
-    hipLaunchKernelGGL(k_refill, dim3(nsys), dim3(SVC_THREADS), 0, stream, views);
+    return dim3(maxN > SVC_THREADS ? SVC_SUM_THREADS : SVC_THREADS);
+}
+
+hipError_t launch_refill(const SysView* views, int nsys, int64_t maxN, hipStream_t stream)
+{
+    const dim3 grid((unsigned)std::min<int64_t>((maxN + SVC_THREADS - 1) / SVC_THREADS, 256), (unsigned)nsys);
+    hipLaunchKernelGGL(k_refill, grid, dim3(SVC_THREADS), 0, stream, views);
+    hipLaunchKernelGGL(k_refill_done, dim3((unsigned)(nsys + SVC_THREADS - 1) / SVC_THREADS), dim3(SVC_THREADS), 0,
+                       stream, views, nsys);
     return hipGetLastError();
 }
 
-hipError_t launch_qs_record(const SysView* views, int nsys, const QsArgs& qa, int64_t e, int begin, hipStream_t stream)
+hipError_t launch_qs_record(const SysView* views, int nsys, int64_t maxN, const QsArgs& qa, int64_t e, int begin,
+                            hipStream_t stream)
 {
-    hipLaunchKernelGGL(k_qs_record, dim3(nsys), dim3(SVC_THREADS), 0, stream, views, qa, e, (int32_t)begin);
+    hipLaunchKernelGGL(k_qs_record, dim3(nsys), sum_threads(maxN), 0, stream, views, qa, e, (int32_t)begin);
     return hipGetLastError();
 }
 
@@ -54,30 +67,42 @@ hipError_t launch_set_iref(const SysView* views, int nsys, int64_t maxN, hipStre
 
 #define FQ_FORCES(P, I, E)                                                                                     \
     if (pot == P && inter == I && ext == E) {                                                                  \
-        hipLaunchKernelGGL((k_forces<P, I, E>), dim3(nsys), dim3(SVC_THREADS), 0, stream, views, flags);       \
+        hipLaunchKernelGGL((k_forces<P, I, E>), grid, dim3(SVC_THREADS), 0, stream, views, flags);             \
         return true;                                                                                           \
     }
 
-static bool launch_forces_one(int pot, int inter, int ext, const SysView* views, int nsys, int32_t flags,
+static bool launch_forces_one(int pot, int inter, int ext, const SysView* views, dim3 grid, int32_t flags,
                               hipStream_t stream);
 
-// Long-range systems: the interaction forces by k_lr_fint (many workgroups
-// per system) between the updates that k_forces applies first (uniform
-// displacement, quench, thermal draws) and the other forces.
-bool launch_forces(int pot, int inter, int ext, const SysView* views, int nsys, int32_t flags, hipStream_t stream)
+// The updates that come first (uniform displacement, quench, thermal draws)
+// have a launch of their own for systems above FORCES_FUSED_MAX particles (a
+// chain of 250007: 4.2 ms in one workgroup) and for long-range systems, whose
+// interaction forces k_lr_fint computes before the other forces.
+constexpr int64_t FORCES_FUSED_MAX = 2048;
+
+bool launch_forces(int pot, int inter, int ext, const SysView* views, int nsys, int64_t maxN, int32_t flags,
+                   hipStream_t stream)
 {
-    if (inter != INT_LONGRANGE1D || !(flags & FF_INT)) {
-        return launch_forces_one(pot, inter, ext, views, nsys, flags, stream);
-    }
+    const dim3 one(1, (unsigned)nsys);
+    // at most 64 workgroups per system, a few thousand in all
+    const int64_t cap = std::max<int64_t>(1, std::min<int64_t>(64, 8192 / std::max(1, nsys)));
+    const dim3 many((unsigned)std::min<int64_t>((maxN + SVC_THREADS - 1) / SVC_THREADS, cap), (unsigned)nsys);
+    const bool lr = inter == INT_LONGRANGE1D && (flags & FF_INT);
     const int32_t first = flags & (FF_ADD_U | FF_QUENCH | FF_THERMAL);
-    if (first && !launch_forces_one(pot, inter, ext, views, nsys, first, stream)) {
+    if (first && !lr && maxN <= FORCES_FUSED_MAX) {
+        return launch_forces_one(pot, inter, ext, views, one, flags, stream);
+    }
+    if (first &&
+        !launch_forces_one(pot, inter, ext, views, (flags & FF_THERMAL) ? one : many, first, stream)) {
         return false;
     }
-    hipLaunchKernelGGL(k_lr_fint, dim3(64, (unsigned)nsys), dim3(SVC_THREADS), 0, stream, views);
-    return launch_forces_one(pot, inter, ext, views, nsys, flags & ~(first | FF_INT), stream);
+    if (lr) {
+        hipLaunchKernelGGL(k_lr_fint, dim3(64, (unsigned)nsys), dim3(SVC_THREADS), 0, stream, views);
+        flags &= ~FF_INT;
+    }
+    return launch_forces_one(pot, inter, ext, views, many, flags & ~first, stream);
 }
-
-static bool launch_forces_one(int pot, int inter, int ext, const SysView* views, int nsys, int32_t flags,
+static bool launch_forces_one(int pot, int inter, int ext, const SysView* views, dim3 grid, int32_t flags,
                               hipStream_t stream)
 {
     FQ_FORCES(POT_CUSPY, INT_LAPLACE1D, 0)
@@ -100,14 +125,14 @@ static bool launch_forces_one(int pot, int inter, int ext, const SysView* views,
     return false;
 }
 
-bool launch_max_uniform(int pot, const SysView* views, int nsys, int32_t direction, hipStream_t stream)
+bool launch_max_uniform(int pot, const SysView* views, int nsys, int64_t maxN, int32_t direction, hipStream_t stream)
 {
     if (pot == POT_CUSPY) {
-        hipLaunchKernelGGL((k_max_uniform<POT_CUSPY>), dim3(nsys), dim3(SVC_THREADS), 0, stream, views, direction);
+        hipLaunchKernelGGL((k_max_uniform<POT_CUSPY>), dim3(nsys), sum_threads(maxN), 0, stream, views, direction);
         return true;
     }
     if (pot == POT_SEMISMOOTH) {
-        hipLaunchKernelGGL((k_max_uniform<POT_SEMISMOOTH>), dim3(nsys), dim3(SVC_THREADS), 0, stream, views,
+        hipLaunchKernelGGL((k_max_uniform<POT_SEMISMOOTH>), dim3(nsys), sum_threads(maxN), 0, stream, views,
                            direction);
         return true;
     }

@@ -13,6 +13,9 @@
 namespace fq {
 
 constexpr int SVC_THREADS = 256;
+// workgroups that reduce a whole system (one per system): SVC_THREADS up to
+// that many particles, else this
+constexpr int SVC_SUM_THREADS = 1024;
 
 // First window of every particle's landscape: cumsum of nchunk increments,
 // then += offset; align to u (which is 0 at construction).
@@ -124,24 +127,29 @@ __global__ void __launch_bounds__(SVC_THREADS) k_lr_fint(const SysView* __restri
     }
 }
 
+// System blockIdx.y, its particles over gridDim.x workgroups. With several
+// workgroups the updates that other particles read (FF_ADD_U; FF_THERMAL draws
+// in particle order) have a launch of their own, the latter of one workgroup.
 template <int POT, int INT, int EXT>
 __global__ void __launch_bounds__(SVC_THREADS) k_forces(const SysView* __restrict__ views, int32_t flags)
 {
-    const SysView S = views[blockIdx.x];
+    const SysView S = views[blockIdx.y];
     RunState* rs = S.rs;
     const Landscape& L = S.ls;
     const int64_t N = S.N;
+    const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     if (flags & FF_ADD_U) {
         const double du = rs->du_add;
         if (du != 0.0) {
-            for (int64_t p = threadIdx.x; p < N; p += blockDim.x) {
+            for (int64_t p = first; p < N; p += stride) {
                 S.u[p] += du;
             }
         }
         __syncthreads();
     }
     if (flags & FF_QUENCH) {
-        for (int64_t p = threadIdx.x; p < N; p += blockDim.x) {
+        for (int64_t p = first; p < N; p += stride) {
             S.v[p] = 0.0;
             S.a[p] = 0.0;
         }
@@ -154,7 +162,7 @@ __global__ void __launch_bounds__(SVC_THREADS) k_forces(const SysView* __restric
     __syncthreads();
     const double uf = rs->u_frame;
     const double meta = -S.eta;
-    for (int64_t p = threadIdx.x; p < N; p += blockDim.x) {
+    for (int64_t p = first; p < N; p += stride) {
         const double up = S.u[p];
         if (flags & FF_POT) {
             int32_t j = L.jloc[p];
@@ -197,7 +205,7 @@ __global__ void __launch_bounds__(SVC_THREADS) k_forces(const SysView* __restric
 // maxUniformDisplacement: rs->red0 = min over particles, rs->red_flag = 1 if
 // a SemiSmooth particle is outside the parabolic part of its well.
 template <int POT>
-__global__ void __launch_bounds__(SVC_THREADS) k_max_uniform(const SysView* __restrict__ views, int32_t direction)
+__global__ void __launch_bounds__(SVC_SUM_THREADS) k_max_uniform(const SysView* __restrict__ views, int32_t direction)
 {
     __shared__ double s_d[RES_MAX_WAVES];
     __shared__ int s_f[RES_MAX_WAVES];
@@ -206,13 +214,33 @@ __global__ void __launch_bounds__(SVC_THREADS) k_max_uniform(const SysView* __re
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     double r = __builtin_inf();
     int outside = 0;
-    for (int64_t p = threadIdx.x; p < S.N; p += blockDim.x) {
-        const double up = S.u[p];
-        int32_t j = L.jloc[p];
-        double yl = L.y[p * L.nchunk + j], yr = L.y[p * L.nchunk + j + 1];
-        align_particle(L, p, up, yl, yr, j);
-        const double x = max_uniform_particle<POT>(S, up, yl, yr, direction, outside);
-        r = x < r ? x : r;
+    // four particles at a time: the load of a well waits for that of its index
+    constexpr int C = 4;
+    const int64_t T = blockDim.x;
+    for (int64_t p0 = threadIdx.x; p0 < S.N; p0 += C * T) {
+        double up[C], yl[C], yr[C];
+        int32_t j[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int64_t p = p0 + c * T < S.N ? p0 + c * T : p0;
+            up[c] = S.u[p];
+            j[c] = L.jloc[p];
+        }
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int64_t p = p0 + c * T < S.N ? p0 + c * T : p0;
+            yl[c] = L.y[p * L.nchunk + j[c]];
+            yr[c] = L.y[p * L.nchunk + j[c] + 1];
+        }
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int64_t p = p0 + c * T;
+            if (p < S.N) {
+                align_particle(L, p, up[c], yl[c], yr[c], j[c]);
+                const double x = max_uniform_particle<POT>(S, up[c], yl[c], yr[c], direction, outside);
+                r = x < r ? x : r;
+            }
+        }
     }
     for (int off = 32; off > 0; off >>= 1) {
         double y = __shfl_xor(r, off, 64);
@@ -269,28 +297,46 @@ __global__ void k_trigger_each(const SysView* __restrict__ views, const int64_t*
 // Landscape refill requested by a launch (status ST_REFILL): align every
 // particle to its slip after the position update of the pending step,
 // u + dt v + dt^2/2 a (bit-identical to the launching kernel), shifting and
-// regenerating its window like the CPU align; then the run continues.
+// regenerating its window like the CPU align; then the run continues
+// (k_refill_done, after every workgroup of the system). System blockIdx.y, its
+// particles over gridDim.x workgroups; a window is drawn by the whole
+// wavefront that holds its particle.
 __global__ void __launch_bounds__(SVC_THREADS) k_refill(const SysView* __restrict__ views)
 {
-    const SysView& S = views[blockIdx.x];
-    RunState* rs = S.rs;
-    if (rs->status != ST_REFILL) {
+    const SysView& S = views[blockIdx.y];
+    if (S.rs->status != ST_REFILL) {
         return;
     }
     const Landscape& L = S.ls;
     const double dt = S.dt;
     const double c2 = 0.5 * dt * dt;
-    for (int64_t p = threadIdx.x; p < S.N; p += blockDim.x) {
-        const double x = S.u[p] + dt * S.v[p] + c2 * S.a[p];
-        const int32_t j = L.jloc[p];
-        const double* row = L.y + p * L.nchunk;
-        if (!(row[j] <= x && x < row[j + 1])) {
-            chunk_align_slow(L, p, x, j);
+    const int64_t N = S.N, stride = (int64_t)gridDim.x * blockDim.x;
+    const int lane = threadIdx.x & 63;
+    for (int64_t w0 = (int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63); w0 < N; w0 += stride) {
+        const int64_t p = w0 + lane;
+        double x = 0.0;
+        int32_t j = 0;
+        bool need = false;
+        if (p < N) {
+            x = S.u[p] + dt * S.v[p] + c2 * S.a[p];
+            j = L.jloc[p];
+            const double* row = L.y + p * L.nchunk;
+            need = !(row[j] <= x && x < row[j + 1]);
+        }
+        uint64_t lanes = __ballot(need);
+        while (lanes) {
+            const int src = __builtin_ctzll(lanes);
+            lanes &= lanes - 1;
+            refill_one(&S, w0 + src, lane_d(x, src), __builtin_amdgcn_readlane(j, src));
         }
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        rs->status = ST_RUNNING;
+}
+
+__global__ void __launch_bounds__(SVC_THREADS) k_refill_done(const SysView* __restrict__ views, int nsys)
+{
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < nsys && views[r].rs->status == ST_REFILL) {
+        views[r].rs->status = ST_RUNNING;
     }
 }
 
@@ -308,7 +354,7 @@ __global__ void __launch_bounds__(SVC_THREADS) k_set_iref(const SysView* __restr
 // variant): begin = 1 stores rs->qs_isum = sum_p (start + jloc - i_ref);
 // begin = 0 records event e, out_*[r * nevents + e] = (sum - qs_isum,
 // u_frame, mean f_frame, inc). Fixed summation order.
-__global__ void __launch_bounds__(SVC_THREADS) k_qs_record(const SysView* __restrict__ views, QsArgs qa, int64_t e,
+__global__ void __launch_bounds__(SVC_SUM_THREADS) k_qs_record(const SysView* __restrict__ views, QsArgs qa, int64_t e,
                                                            int32_t begin)
 {
     __shared__ long long s_i[RES_MAX_WAVES];
@@ -322,6 +368,7 @@ __global__ void __launch_bounds__(SVC_THREADS) k_qs_record(const SysView* __rest
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     long long si = 0;
     double sd = 0.0;
+#pragma unroll 4
     for (int64_t p = threadIdx.x; p < S.N; p += blockDim.x) {
         si += L.start[p] + L.jloc[p] - S.i_ref[p];
         sd += S.f_frame[p];
