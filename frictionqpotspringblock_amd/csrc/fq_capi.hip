@@ -129,7 +129,9 @@ constexpr int64_t LR_TILE_WAVE = 64;
 // 512 threads); longer chains sweep over tiles
 constexpr int64_t NOPASSING_RESIDENT_MAX = 8192;
 // sweeps between host checks of a tiled no-passing run, and particles per tile
-constexpr uint64_t NP_BLOCK = 256;
+// (a relaxation takes about a hundred sweeps; the launches of a block after
+// the last one cost 7 us each)
+constexpr uint64_t NP_BLOCK = 64;
 constexpr int64_t NP_TILE_PARTICLES = 4096;
 // steps between host checks of a batched long-range run (matrix form)
 constexpr uint64_t LR_BLOCK = 128;
@@ -3535,7 +3537,16 @@ int fqsb_ragged_create(const fqsb_desc* descs, uint64_t n, fqsb_ragged** out)
             throw Error("at least one system is needed");
         }
         std::unique_ptr<fqsb_ragged> rg(new fqsb_ragged());
-        // key: kernel class and size class (ceil(log2 N))
+        int64_t resident_max = RAGGED_RESIDENT_MAX;
+        if (const char* e = std::getenv("FQSB_RAGGED_RESIDENT_MAX")) {
+            resident_max = std::max<int64_t>(0, std::atoll(e));
+        }
+        // key: kernel class and size class (ceil(log2 N)); systems that spread
+        // over tiles are one size class (their launches do not depend on the
+        // size, and a group's operations cost about as long as its slowest
+        // system's: three events of 96 systems, 41 groups on the GPU's four
+        // queues: 97 ms, 19 groups: 53 ms)
+        constexpr int TILED = 64;
         typedef std::tuple<int, int, int, int, int, int> Key;
         std::map<Key, std::vector<uint64_t>> classes;
         rg->sizes.resize((size_t)n);
@@ -3549,13 +3560,13 @@ int fqsb_ragged_create(const fqsb_desc* descs, uint64_t n, fqsb_ragged** out)
             while ((int64_t(1) << lg) < N) {
                 ++lg;
             }
+            if (d.minimisation == FQSB_MIN_OVERDAMPED ? N > NOPASSING_RESIDENT_MAX
+                                                      : resident_max > 0 && N > resident_max) {
+                lg = TILED;
+            }
             classes[Key(d.rank, d.potential, d.interactions, d.external, d.minimisation, lg)].push_back(i);
         }
         rg->where.resize((size_t)n);
-        int64_t resident_max = RAGGED_RESIDENT_MAX;
-        if (const char* e = std::getenv("FQSB_RAGGED_RESIDENT_MAX")) {
-            resident_max = std::max<int64_t>(0, std::atoll(e));
-        }
         for (auto& kv : classes) {
             std::vector<fqsb_desc> ds;
             for (uint64_t i : kv.second) {
