@@ -524,7 +524,7 @@ def run_adjoint(args):
     g = leaves[3].grad
     assert torch.all(torch.isfinite(g))
     value = AD_R * AD_N * AD_T * args.steps / wall
-    tape_bytes = 28.0 * AD_R * AD_N * AD_K  # u, v, a (FP64) and well index (int32) per particle-step
+    tape_bytes = 16.0 * AD_R * AD_N * AD_K  # u, v (FP64) per particle-step
     achieved = tape_bytes / (rev_ms * 1e-3) / 1e9
     cpu = None if args.no_cpu else cpu_leg("adjoint", args)
     return {

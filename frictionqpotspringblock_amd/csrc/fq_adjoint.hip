@@ -2,6 +2,8 @@
 #include "fq_adjoint.hpp"
 #include "fq_launch.hpp"
 
+#include <algorithm>
+
 namespace fq {
 
 // record: (particles per thread, threads per workgroup) variants; the host
@@ -44,6 +46,15 @@ bool launch_adj_record(int ppt, int threads, const SysView* views, const AdjBuff
     }
 }
 
+// checkpoint: one launch in place of four copies
+hipError_t launch_adj_checkpoint(const double* u, const double* v, const double* a, const int32_t* j, double* cu,
+                                 double* cv, double* ca, int32_t* cj, int64_t n, hipStream_t stream)
+{
+    const unsigned grid = (unsigned)std::min<int64_t>((n + 255) / 256, 4096);
+    hipLaunchKernelGGL(k_adj_checkpoint, dim3(grid), dim3(256), 0, stream, u, v, a, j, cu, cv, ca, cj, n);
+    return hipGetLastError();
+}
+
 // reverse: particles of the extended segment per thread
 #define FQ_ADJ_SLOTS(X) X(1) X(2) X(3) X(4) X(6) X(8)
 
@@ -60,10 +71,11 @@ int adj_reverse_slots(int64_t extended)
 
 bool launch_adj_reverse(const SysView* views, const AdjBuffers& ab, int slots, int steps, hipStream_t stream)
 {
+    const size_t lds = 4 * sizeof(double) * (size_t)adj_rev_stride(slots);
     switch (slots) {
 #define FQ_REV(P)                                                                                              \
     case P:                                                                                                    \
-        hipLaunchKernelGGL((k_adj_reverse<P>), dim3((unsigned)(ab.R * ab.nt)), dim3(ADJ_REV_THREADS), 0,       \
+        hipLaunchKernelGGL((k_adj_reverse<P>), dim3((unsigned)(ab.R * ab.nt)), dim3(ADJ_REV_THREADS), lds,     \
                            stream, views, ab, steps);                                                          \
         break;
         FQ_ADJ_SLOTS(FQ_REV)

@@ -14,8 +14,16 @@
 // A run of n steps is split into windows of K steps. For each window, last
 // to first: k_adj_record re-runs the window from its checkpoint (the same
 // expressions in the same order as the resident kernel, so the same
-// trajectory and the same wells) and writes a tape of u1, v and a of every
-// step and the well used by it; k_adj_reverse then walks the tape backwards.
+// trajectory and the same wells) and writes a tape of u1 and v of every step;
+// k_adj_reverse then walks the tape backwards. What else a step used follows
+// from these and is not written: its acceleration is that of the preceding
+// step's last stage, (g - eta v) / m with the g of the preceding u1, and its
+// well is the one that holds u1 (a window's wells are walked to from those of
+// its checkpoint). Both kernels are bound by the tape's bytes: 64 chains of
+// 4096, 2000 steps, record / reverse with u1, v, a and the well (28 bytes per
+// particle-step): 3.0 / 4.6 ms, with u1 and v (16 bytes): 1.9 / 3.3
+// ms (4.5 / 2.6 TB/s; in the reverse kernel the instructions of a step come
+// next).
 // The tape is particle-major per step ([step][replica][particle]) and both
 // kernels give a thread the particles t, t + T, t + 2T, ... of its segment,
 // so that every tape load and store of a wavefront is contiguous; neighbours
@@ -24,7 +32,8 @@
 // k_adj_reverse spreads each replica over tiles (many workgroups per
 // replica): a tile walks its particles together with a halo of K + 1
 // particles on each side, whose cotangents start from the adjoint state of
-// their owners. The cotangent of a particle at the open end of the extended
+// their owners (the cotangents of the forces do not depend on the tape, so a
+// halo reads none of it, but for the slip next to the tile's own particles). The cotangent of a particle at the open end of the extended
 // segment lacks one neighbour, and the error this makes moves inwards by one
 // particle per reversed step (through the second difference of the
 // cotangents of the forces), so after the K steps of a window the tile's own
@@ -36,6 +45,8 @@
 
 #include "fq_physics.hpp"
 #include "fq_resident.hpp"
+
+#include <type_traits>
 
 namespace fq {
 
@@ -69,8 +80,6 @@ __global__ void __launch_bounds__(MAXT) k_adj_record(const SysView* __restrict__
     ab.wuf += blockIdx.y * ab.R;
     ab.tu += blockIdx.y * ab.ts;
     ab.tv += blockIdx.y * ab.ts;
-    ab.ta += blockIdx.y * ab.ts;
-    ab.tj += blockIdx.y * ab.ts;
     ab.tuf += blockIdx.y * ab.K * ab.R;
     const SysView& S = views[r];
     constexpr int T = MAXT; // launched with exactly MAXT threads
@@ -132,13 +141,10 @@ __global__ void __launch_bounds__(MAXT) k_adj_record(const SysView* __restrict__
             const int e = t + T * k;
             if (e < E) {
                 const int64_t q = tn + (RING ? t + T * k : pp[k]);
-                if (own[k]) {
-                    ab.tv[q] = v[k];
-                    ab.ta[q] = a[k];
-                }
                 u[k] = u[k] + dt * v[k] + c2 * a[k];
                 const double x = u[k];
                 if (own[k]) {
+                    ab.tv[q] = v[k];
                     ab.tu[q] = x;
                 }
                 if (!(yl[k] <= x && x < yr[k])) {
@@ -159,9 +165,6 @@ __global__ void __launch_bounds__(MAXT) k_adj_record(const SysView* __restrict__
                     jl[k] = j;
                     yl[k] = lo;
                     yr[k] = hi;
-                }
-                if (own[k]) {
-                    ab.tj[q] = jl[k];
                 }
                 xb[e] = x;
             }
@@ -212,15 +215,19 @@ __global__ void __launch_bounds__(MAXT) k_adj_record(const SysView* __restrict__
 // dg/dy_r = mu/2, one accumulator per particle collects the derivative for
 // both yield positions of its current well; it is added to the output when
 // the well changes.
+//
+// One barrier per step: the cotangent G of the force is linear in the
+// cotangents after the step alone, so it is exchanged together with the slips
+// of the step before, whose force gives this step's acceleration. The tape is
+// loaded two steps ahead.
 template <int SLOTS>
 __global__ void __launch_bounds__(ADJ_REV_THREADS) k_adj_reverse(const SysView* __restrict__ views, AdjBuffers ab,
                                                                    int steps)
 {
-    // neighbour exchange: slips u1 (su) and cotangents of g (sg) of a step;
-    // two barriers per step (a buffer is rewritten only after the barrier
-    // that follows every read of it)
-    __shared__ double su[ADJ_REV_THREADS * SLOTS];
-    __shared__ double sg[ADJ_REV_THREADS * SLOTS];
+    // neighbour exchange: cotangents of g and slips u1, double-buffered by
+    // the parity of their step (a buffer is rewritten two barriers after the
+    // one that precedes its reads)
+    extern __shared__ double s_x[]; // [2][B] cotangents, [2][B] slips
     __shared__ double s_red[4][ADJ_REV_THREADS / 64];
     const int r = blockIdx.x / ab.nt, tile = blockIdx.x % ab.nt;
     const SysView& S = views[r];
@@ -234,173 +241,232 @@ __global__ void __launch_bounds__(ADJ_REV_THREADS) k_adj_reverse(const SysView* 
     const int p1 = p0 + (int)ab.tp < N ? p0 + (int)ab.tp : N;
     const int H = ring ? 0 : (int)ab.halo;
     const int E = ring ? N : (p1 - p0) + 2 * H; // particles of the extended segment
+    constexpr int B = adj_rev_stride(SLOTS); // local index e at 1 + e: a neighbour's place on each side
     const double* const Y = S.ls.y;
     const int64_t nch = S.ls.nchunk;
+    const int32_t jmin = (int32_t)S.ls.buffer;
+    const int32_t jmax = (int32_t)(nch - 2 - S.ls.buffer);
     const int64_t Rnp = ab.R * ab.np;
 
-    const double dt = S.dt, c2 = 0.5 * dt * dt, hdt = 0.5 * dt, meta = -S.eta, w = S.inv_m, kf = S.k_frame;
+    const double dt = S.dt, c2 = 0.5 * dt * dt, h = 0.5 * dt, meta = -S.eta, w = S.inv_m, kf = S.k_frame;
     const double mu = S.mu, k = S.k;
-    const double mweta = meta * w; // -eta / m
-    const double hmu = 0.5 * mu;
+    const double e1 = meta * w; // -eta / m
+    // The stages' cotangents, a3 = w (g - eta v3), v3 = v + h a + h a2 and so
+    // on down to v1 = v + dt a, are multiples of V3 = V + e1 A: of a2 h V3, of
+    // v2 e1 h V3, of a1 e1 h^2 V3, of v1 (e1 h)^2 V3
+    const double eh = e1 * h, ehh = eh * eh, dehh = dt * ehh, kfm = -(kf + mu);
 
-    // slot i: local index e = t + T i of the extended segment, particle p
+    // slot i: local index e = t + T i of the extended segment, particle p;
+    // own: this tile's; slip: its u1 is read (its own particles and the one
+    // next to them on each side)
     int pp[SLOTS];
-    bool own[SLOTS], live[SLOTS];
+    bool own[SLOTS], slip[SLOTS], live[SLOTS];
 #pragma unroll
     for (int i = 0; i < SLOTS; ++i) {
         const int e = t + T * i;
         live[i] = e < E;
         own[i] = live[i] && (ring || (e >= H && e < H + (p1 - p0)));
+        slip[i] = live[i] && (ring || (e >= H - 1 && e < H + (p1 - p0) + 1));
         int q = ring ? e : p0 - H + e;
         q = q < 0 ? q + N : (q >= N ? q - N : q);
         pp[i] = q;
     }
     // U, V, A: cotangents of u, v, a after the step being reversed
-    // jc, ymc: the well of the current tape step and its mid-point (read from
-    // the chunk only when the well changes)
-    double U[SLOTS], V[SLOTS], A[SLOTS], acc[SLOTS], ymc[SLOTS];
+    // x, v, lu, d, g, lo, hi: slip, velocity, second difference of the slips,
+    // distance to the well's middle, force without damping and the well
+    // (index jc) of that step; acc: sum of G over the steps in that well
+    double U[SLOTS], V[SLOTS], A[SLOTS], acc[SLOTS];
+    double x[SLOTS], v[SLOTS], lu[SLOTS], d[SLOTS], g[SLOTS], lo[SLOTS], hi[SLOTS];
     int32_t jc[SLOTS];
 #pragma unroll
     for (int i = 0; i < SLOTS; ++i) {
-        U[i] = V[i] = A[i] = acc[i] = ymc[i] = 0.0;
-        jc[i] = -1;
+        U[i] = V[i] = A[i] = acc[i] = 0.0;
+        x[i] = v[i] = lu[i] = d[i] = g[i] = lo[i] = hi[i] = 0.0;
+        jc[i] = 0;
         if (live[i]) {
             U[i] = ab.au[off + pp[i]];
             V[i] = ab.av[off + pp[i]];
             A[i] = ab.aa[off + pp[i]];
         }
+        if (own[i]) {
+            jc[i] = ab.wj[off + pp[i]];
+            lo[i] = Y[(int64_t)pp[i] * nch + jc[i]];
+            hi[i] = Y[(int64_t)pp[i] * nch + jc[i] + 1];
+        }
     }
     double gmu = 0.0, gk = 0.0, gkf = 0.0, geta = 0.0;
 
     auto flush = [&](int i) {
-        if (ab.gy && own[i] && jc[i] >= 0) {
+        if (ab.gy && own[i]) {
             double* row = ab.gy + (off + pp[i]) * nch;
-            row[jc[i]] += acc[i];
-            row[jc[i] + 1] += acc[i];
+            const double dy = 0.5 * mu * acc[i];
+            row[jc[i]] += dy;
+            row[jc[i] + 1] += dy;
         }
         acc[i] = 0.0;
     };
-    // neighbour of local index e at offset d (+1 or -1): periodic on the
-    // ring; at the open ends of a tile's segment, any finite value (the
-    // error zone that never reaches the tile's own particles)
-    auto nb = [&](const double* s, int e, int d, double self) -> double {
-        int q = e + d;
-        if (ring) {
-            q = q < 0 ? q + E : (q >= E ? q - E : q);
-            return s[q];
+    // the well of slip y of an own particle, from the current one
+    auto walk = [&](int i, double y) {
+        if (!(lo[i] <= y && y < hi[i])) {
+            if (acc[i] != 0.0) {
+                flush(i);
+            }
+            const double* row = Y + (int64_t)pp[i] * nch;
+            int32_t j = jc[i];
+            double a = lo[i], b = hi[i];
+            while (y >= b && j < jmax) {
+                ++j;
+                a = b;
+                b = row[j + 1];
+            }
+            while (y < a && j > jmin) {
+                --j;
+                b = a;
+                a = row[j];
+            }
+            jc[i] = j;
+            lo[i] = a;
+            hi[i] = b;
         }
-        return (q < 0 || q >= E) ? self : s[q];
+    };
+    // the ends' neighbours: on the ring copies of the other end's values; at
+    // the open ends of a tile's segment 0, any finite value would do (the
+    // error zone that never reaches the tile's own particles)
+    if (!ring && t < 8) {
+        s_x[(t >> 1) * B + ((t & 1) ? E + 1 : 0)] = 0.0;
+    }
+    double* const sx = s_x + 1 + t;
+    auto put = [&](int buf, int i, double y) {
+        sx[buf * B + T * i] = y;
+        if (ring && t + T * i == 0) {
+            s_x[buf * B + E + 1] = y;
+        }
+        if (ring && t + T * i == E - 1) {
+            s_x[buf * B] = y;
+        }
+    };
+    auto neighbours = [&](int buf, int i) { return sx[buf * B + T * i - 1] + sx[buf * B + T * i + 1]; };
+
+    // force of an own particle from its slip and the neighbours'
+    auto force = [&](int buf, int i, double f) {
+        lu[i] = __builtin_fma(-2.0, x[i], neighbours(buf, i));
+        walk(i, x[i]);
+        d[i] = __builtin_fma(0.5, lo[i] + hi[i], -x[i]);
+        g[i] = __builtin_fma(k, lu[i], __builtin_fma(mu, d[i], kf * (f - x[i])));
     };
 
-    // the tape of step n is loaded while step n + 1 is reversed (registers
-    // qu, qv, qa, qj, quf), so its memory latency is hidden behind that work
-    double qu[SLOTS], qv[SLOTS], qa[SLOTS], quf = 0.0;
-    int32_t qj[SLOTS];
-    auto load = [&](int n) {
-        const int64_t tn = (int64_t)n * Rnp + (int64_t)r * ab.np;
-#pragma unroll
-        for (int i = 0; i < SLOTS; ++i) {
-            qu[i] = qv[i] = qa[i] = 0.0;
-            qj[i] = 0;
-            if (live[i]) {
-                const int64_t q = tn + pp[i];
-                qu[i] = ab.tu[q];
-                qv[i] = ab.tv[q];
-                qa[i] = ab.ta[q];
-                qj[i] = ab.tj[q];
-            }
-        }
-        quf = ab.tuf[(int64_t)n * ab.R + r];
+    // the tape of step n (n = -1: the checkpoint's acceleration in qu), loaded
+    // two steps before its use
+    struct Tape {
+        double u[SLOTS], v[SLOTS], uf;
     };
-    if (steps > 0) {
-        load(steps - 1);
-    }
-    for (int n = steps - 1; n >= 0; --n) {
-        const double uf = quf;
-        double x[SLOTS], pv[SLOTS], pa[SLOTS];
-        int32_t pj[SLOTS];
+    auto load = [&](Tape& q, int n) {
+        const int64_t tn = (n >= 0 ? n * Rnp : 0) + (int64_t)r * ab.np;
+        const double* const tu = (n >= 0 ? ab.tu : ab.wa) + tn;
+        const double* const tv = ab.tv + tn;
 #pragma unroll
         for (int i = 0; i < SLOTS; ++i) {
-            x[i] = qu[i];
-            pv[i] = qv[i];
-            pa[i] = qa[i];
-            pj[i] = qj[i];
+            if (slip[i]) {
+                q.u[i] = tu[(uint32_t)pp[i]];
+            }
+            if (own[i] && n >= 0) {
+                q.v[i] = tv[(uint32_t)pp[i]];
+            }
+        }
+        if (n >= 0) {
+            q.uf = ab.tuf[(int64_t)n * ab.R + r];
+        }
+    };
+    double uf = 0.0;
+    // reverse step n; q: the tape of step n - 1
+    auto step = [&](int n, Tape& q, auto odd) {
+        constexpr int gb = decltype(odd)::value, xb = 2 + (1 - decltype(odd)::value);
+        double G[SLOTS], V3[SLOTS], px[SLOTS], pv[SLOTS];
+        const double puf = q.uf;
+#pragma unroll
+        for (int i = 0; i < SLOTS; ++i) {
+            px[i] = q.u[i];
+            pv[i] = q.v[i];
             if (live[i]) {
-                su[t + T * i] = x[i];
+                V3[i] = __builtin_fma(e1, A[i], V[i]);
+                G[i] = w * __builtin_fma(h, __builtin_fma(eh, V3[i], V3[i]), A[i]);
+                put(gb, i, G[i]);
+            }
+            if (n > 0 && slip[i]) {
+                put(xb, i, px[i]);
             }
         }
         __syncthreads();
-        if (n > 0) {
-            load(n - 1);
+        if (n > 1) {
+            load(q, n - 3);
         }
 #pragma unroll
         for (int i = 0; i < SLOTS; ++i) {
-            if (live[i]) {
-                const int e = t + T * i;
-                const int64_t p = pp[i];
-                const double u1 = x[i];
-                const double lu = nb(su, e, -1, u1) - 2 * u1 + nb(su, e, +1, u1);
-                const int32_t j = pj[i];
-                if (j != jc[i]) {
-                    flush(i);
-                    jc[i] = j;
-                    ymc[i] = 0.5 * (Y[p * nch + j] + Y[p * nch + j + 1]);
+            if (own[i]) {
+                // the force of the step before gives the acceleration at the
+                // start of this one, and from it the velocities of its stages
+                const double gn = g[i];
+                gkf = __builtin_fma(uf - x[i], G[i], gkf);
+                gmu = __builtin_fma(d[i], G[i], gmu);
+                gk = __builtin_fma(lu[i], G[i], gk);
+                acc[i] += G[i];
+                double a = px[i];
+                if (n > 0) {
+                    x[i] = px[i];
+                    force(xb, i, puf);
+                    a = w * __builtin_fma(meta, v[i], g[i]);
                 }
-                const double ym = ymc[i];
-                const double v = pv[i], a = pa[i];
-                // forward quantities of the step
-                const double g = kf * (uf - u1) + (ym - u1) * mu + lu * k;
-                const double v1 = v + dt * a;
-                const double a1 = (g + meta * v1) * w;
-                const double v2 = v + hdt * (a + a1);
-                const double a2 = (g + meta * v2) * w;
-                const double v3 = v + hdt * (a + a2);
-                // a3 = w (g - eta v3)
-                double G = w * A[i];
-                const double V3 = V[i] + mweta * A[i];
-                double ge = -(w * v3 * A[i]);
-                // v3 = v + hdt a + hdt a2
-                double vb = V3, ab_ = hdt * V3;
-                const double A2 = hdt * V3;
-                G += w * A2;
-                const double V2 = mweta * A2;
-                ge -= w * v2 * A2;
-                // v2 = v + hdt a + hdt a1
-                vb += V2;
-                ab_ += hdt * V2;
-                const double A1 = hdt * V2;
-                G += w * A1;
-                const double V1 = mweta * A1;
-                ge -= w * v1 * A1;
-                // v1 = v + dt a
-                vb += V1;
-                ab_ += dt * V1;
-                if (own[i]) {
-                    geta += ge;
-                    gkf += (uf - u1) * G;
-                    gmu += (ym - u1) * G;
-                    gk += lu * G;
-                    acc[i] += hmu * G;
-                }
-                V[i] = vb; // partial cotangents of v, a (the u1 part follows)
-                A[i] = ab_;
-                x[i] = G;
-                sg[e] = G;
+                const double v1 = __builtin_fma(dt, a, v[i]);
+                const double a1 = w * __builtin_fma(meta, v1, gn);
+                const double v2 = __builtin_fma(h, a + a1, v[i]);
+                const double a2 = w * __builtin_fma(meta, v2, gn);
+                const double v3 = __builtin_fma(h, a + a2, v[i]);
+                geta = __builtin_fma(h * V3[i], __builtin_fma(eh, v1, v2), __builtin_fma(v3, A[i], geta));
+                v[i] = pv[i];
             }
+            if (live[i]) {
+                // g depends on u1 through -(k_frame + mu) u1 + k L u1 (L
+                // symmetric); u1 = u + dt v + c2 a
+                const double s2 = __builtin_fma(eh, V3[i], V3[i]);
+                U[i] = __builtin_fma(k, __builtin_fma(-2.0, G[i], neighbours(gb, i)),
+                                     __builtin_fma(kfm, G[i], U[i]));
+                V[i] = __builtin_fma(dt, U[i], __builtin_fma(ehh, V3[i], s2));
+                A[i] = __builtin_fma(c2, U[i], __builtin_fma(dehh, V3[i], h * s2));
+            }
+        }
+        uf = puf;
+    };
+    if (steps > 0) { // the last step's slips, wells and velocities
+        Tape q0 = {}, q1 = {};
+        load(q0, steps - 1);
+        uf = q0.uf;
+#pragma unroll
+        for (int i = 0; i < SLOTS; ++i) {
+            x[i] = q0.u[i];
+            v[i] = q0.v[i];
+            if (slip[i]) {
+                put(2, i, x[i]);
+            }
+        }
+        load(q0, steps - 2);
+        if (steps > 1) {
+            load(q1, steps - 3);
         }
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < SLOTS; ++i) {
-            if (live[i]) {
-                const int e = t + T * i;
-                const double G = x[i];
-                // g depends on u1 through -(k_frame + mu) u1 + k L u1 (L symmetric)
-                const double U1 = U[i] - (kf + mu) * G + k * (nb(sg, e, -1, G) - 2 * G + nb(sg, e, +1, G));
-                // u1 = u + dt v + c2 a
-                U[i] = U1;
-                V[i] = V[i] + dt * U1;
-                A[i] = A[i] + c2 * U1;
+            if (own[i]) {
+                force(2, i, uf);
             }
+        }
+        // (the first step's slips go to the other buffer)
+        int n = steps - 1;
+        for (; n > 0; n -= 2) {
+            step(n, q0, std::integral_constant<int, 0>());
+            step(n - 1, q1, std::integral_constant<int, 1>());
+        }
+        if (n == 0) {
+            step(0, q0, std::integral_constant<int, 0>());
         }
     }
 #pragma unroll
@@ -416,7 +482,7 @@ __global__ void __launch_bounds__(ADJ_REV_THREADS) k_adj_reverse(const SysView* 
     gmu = wave_sum(gmu);
     gk = wave_sum(gk);
     gkf = wave_sum(gkf);
-    geta = wave_sum(geta);
+    geta = wave_sum(-w * geta);
     if (lane == 0) {
         s_red[0][wave] = gmu;
         s_red[1][wave] = gk;
@@ -430,6 +496,20 @@ __global__ void __launch_bounds__(ADJ_REV_THREADS) k_adj_reverse(const SysView* 
             s += s_red[t][q];
         }
         ab.gpart[(int64_t)blockIdx.x * 4 + t] = s;
+    }
+}
+
+// The state of all replicas at the start of a window.
+__global__ void __launch_bounds__(256) k_adj_checkpoint(const double* __restrict__ u, const double* __restrict__ v,
+                                                        const double* __restrict__ a, const int32_t* __restrict__ j,
+                                                        double* __restrict__ cu, double* __restrict__ cv,
+                                                        double* __restrict__ ca, int32_t* __restrict__ cj, int64_t n)
+{
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        cu[i] = u[i];
+        cv[i] = v[i];
+        ca[i] = a[i];
+        cj[i] = j[i];
     }
 }
 

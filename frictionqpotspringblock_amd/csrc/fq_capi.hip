@@ -161,8 +161,7 @@ struct Group {
     double *ck_u = nullptr, *ck_v = nullptr, *ck_a = nullptr;
     int32_t* ck_j = nullptr;
     std::vector<double> ck_uf; // [nw][R]
-    double *tp_u = nullptr, *tp_v = nullptr, *tp_a = nullptr, *tp_uf = nullptr;
-    int32_t* tp_j = nullptr;
+    double *tp_u = nullptr, *tp_v = nullptr, *tp_uf = nullptr;
     double* ck_uf_d = nullptr; // device copy of ck_uf
     double *ad_u = nullptr, *ad_v = nullptr, *ad_a = nullptr, *ad_par = nullptr;
     double *ad_u2 = nullptr, *ad_v2 = nullptr, *ad_a2 = nullptr, *ad_gpart = nullptr;
@@ -798,12 +797,12 @@ struct Group {
 
     void free_adjoint()
     {
-        for (double** q : {&ck_u, &ck_v, &ck_a, &tp_u, &tp_v, &tp_a, &tp_uf, &ck_uf_d, &ad_u, &ad_v, &ad_a,
+        for (double** q : {&ck_u, &ck_v, &ck_a, &tp_u, &tp_v, &tp_uf, &ck_uf_d, &ad_u, &ad_v, &ad_a,
                            &ad_par, &ad_u2, &ad_v2, &ad_a2, &ad_gpart}) {
             dfree(*q);
             *q = nullptr;
         }
-        for (int32_t** q : {&ck_j, &tp_j, &ad_err}) {
+        for (int32_t** q : {&ck_j, &ad_err}) {
             dfree(*q);
             *q = nullptr;
         }
@@ -824,8 +823,6 @@ struct Group {
         fq::AdjBuffers ab{};
         ab.tu = tp_u;
         ab.tv = tp_v;
-        ab.ta = tp_a;
-        ab.tj = tp_j;
         ab.tuf = tp_uf;
         ab.au = ad_u;
         ab.av = ad_v;
@@ -883,10 +880,7 @@ struct Group {
         const int64_t refills0 = refills;
         for (int64_t w = 0; w < nw; ++w) {
             const size_t o = (size_t)w * RN;
-            HIPC(hipMemcpyAsync(ck_u + o, u, sizeof(double) * RN, hipMemcpyDeviceToDevice, stream));
-            HIPC(hipMemcpyAsync(ck_v + o, v, sizeof(double) * RN, hipMemcpyDeviceToDevice, stream));
-            HIPC(hipMemcpyAsync(ck_a + o, a, sizeof(double) * RN, hipMemcpyDeviceToDevice, stream));
-            HIPC(hipMemcpyAsync(ck_j + o, jloc, sizeof(int32_t) * RN, hipMemcpyDeviceToDevice, stream));
+            HIPC(fq::launch_adj_checkpoint(u, v, a, jloc, ck_u + o, ck_v + o, ck_a + o, ck_j + o, (int64_t)RN, stream));
             for (int64_t r = 0; r < R; ++r) {
                 ck_uf[(size_t)(w * R + r)] = hrs[(size_t)r].u_frame;
             }
@@ -965,6 +959,13 @@ struct Group {
             while (R * nt < 256 && (N + 2 * nt - 1) / (2 * nt) >= 4 * halo) {
                 nt *= 2;
             }
+            // more than 4 particles per thread spill (64 chains of 4096, 2 tiles
+            // of 6 per thread: 0.80 ms per window; 4 tiles of 3: 0.17 ms; 8 of
+            // 2: 0.22 ms, more of it in halos)
+            while (fq::adj_reverse_slots(nt == 1 ? N : (N + nt - 1) / nt + 2 * halo) > 4 &&
+                   (N + 2 * nt - 1) / (2 * nt) >= halo) {
+                nt *= 2;
+            }
         }
         // at least as many tiles as make a tile and its halos fit the kernel
         const int64_t rev_cap = (int64_t)fq::ADJ_REV_THREADS * fq::ADJ_REV_MAX_SLOTS;
@@ -986,20 +987,16 @@ struct Group {
         }
         // the tape of a group of windows, recorded by one launch (every window
         // starts from its checkpoint): as many windows as fit in ADJ_TAPE_BYTES
-        const size_t per_window = RNt * (size_t)adj_K * (3 * sizeof(double) + sizeof(int32_t)) +
+        const size_t per_window = RNt * (size_t)adj_K * 2 * sizeof(double) +
                                   (size_t)(R * adj_K) * sizeof(double);
         const int64_t G = std::max<int64_t>(1, std::min<int64_t>(adj_nw, (int64_t)(ADJ_TAPE_BYTES / per_window)));
         if ((size_t)(G * adj_K) * RNt > tp_cap) {
             dfree(tp_u);
             dfree(tp_v);
-            dfree(tp_a);
-            dfree(tp_j);
             dfree(tp_uf);
             const size_t steps = (size_t)(G * adj_K);
             tp_u = dalloc<double>(RNt * steps);
             tp_v = dalloc<double>(RNt * steps);
-            tp_a = dalloc<double>(RNt * steps);
-            tp_j = dalloc<int32_t>(RNt * steps);
             tp_uf = dalloc<double>((size_t)R * steps);
             tp_cap = steps * RNt;
         }
@@ -1063,8 +1060,8 @@ struct Group {
                 const size_t to = (size_t)(w - w0) * (size_t)adj_K;
                 abw.tu = tp_u + to * RNt;
                 abw.tv = tp_v + to * RNt;
-                abw.ta = tp_a + to * RNt;
-                abw.tj = tp_j + to * RNt;
+                abw.wa = ck_a + (size_t)w * RN;
+                abw.wj = ck_j + (size_t)w * RN;
                 abw.tuf = tp_uf + to * (size_t)R;
                 // adjoint state: read from one buffer, written to the other
                 abw.au = ad_u;

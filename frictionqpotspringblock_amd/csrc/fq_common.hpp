@@ -218,6 +218,11 @@ struct LrBuffers {
 // particles of a tile's extended segment per thread
 constexpr int ADJ_REV_THREADS = 512;
 constexpr int ADJ_REV_MAX_SLOTS = 8;
+// LDS entries of one exchange buffer of k_adj_reverse
+constexpr int adj_rev_stride(int slots)
+{
+    return ADJ_REV_THREADS * slots + 2;
+}
 
 // Buffers of the adjoint of a batch (fq_adjoint.hpp); [R*N] arrays are
 // replica after replica. The tape holds, per step, R blocks of np = N entries
@@ -225,8 +230,6 @@ constexpr int ADJ_REV_MAX_SLOTS = 8;
 struct AdjBuffers {
     double* tu;     // tape [K][R*np]: u1 = u + dt v + dt^2/2 a of step n
     double* tv;     // tape: v at the start of step n
-    double* ta;     // tape: a at the start of step n
-    int32_t* tj;    // tape: chunk-local well index used by step n
     double* tuf;    // tape [K][R]: frame position of step n
     double* wu;     // state at the window start [R*N] (its checkpoint)
     double* wv;

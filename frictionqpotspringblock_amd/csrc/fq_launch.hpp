@@ -117,6 +117,8 @@ bool launch_adj_record(int ppt, int threads, const SysView* views, const AdjBuff
                        double v_frame, hipStream_t stream);
 // extended-segment particles per thread of the reverse kernel for a segment
 // of `extended` particles (0: too long)
+hipError_t launch_adj_checkpoint(const double* u, const double* v, const double* a, const int32_t* j, double* cu,
+                                 double* cv, double* ca, int32_t* cj, int64_t n, hipStream_t stream);
 int adj_reverse_slots(int64_t extended);
 bool launch_adj_reverse(const SysView* views, const AdjBuffers& ab, int slots, int steps, hipStream_t stream);
 

@@ -212,3 +212,35 @@ def test_backward_of_a_replaced_tape_raises():
     with pytest.raises(RuntimeError, match="tape of this forward pass is gone"):
         u4.sum().backward()
     del u2
+
+
+@pytest.mark.parametrize("K", [1, 2, 3, 7])
+@pytest.mark.parametrize("R,N", [(2, 3), (2, 64), (2, 513), (300, 2049)])
+def test_window_lengths(R, N, K):
+    """Windows of 1, 2, 3 steps (the reverse kernel's first, last and paired
+    steps) and one longer than the run; N = 2049 with 300 replicas needs tiles
+    only to keep 4 particles per thread. The identity <c, J d> = <J^T c, d>
+    holds to the rounding of its terms: about 40 operations per step and the
+    sums over R N terms, far below 1e-12 of the terms' sum."""
+    import torch
+
+    from frictionqpotspringblock_amd import adjoint as A
+
+    rng = np.random.default_rng(N + K)
+    n = 5
+    b = _batch(R, N)
+    u0, v0, a0, par, y = _setup(b, rng, vscale=1.0)
+    uf0 = torch.tensor(b.u_frame)
+    leaves = [x.clone().requires_grad_(True) for x in (u0, v0, a0, par, y)]
+    out = A.run(b, n, K, *leaves, flow=True, v_frame=0.05)
+    args = [x.detach().cpu().numpy() for x in (u0, v0, a0)]
+    d = [rng.normal(size=x.shape) for x in args] + [rng.normal(size=(R, 4)) * 1e-2, rng.normal(size=tuple(y.shape))]
+    _, dout = TLM.run(
+        *args, y.cpu().numpy(), par.numpy(), uf0.numpy(), n, DT, M, flow=True, v_frame=0.05, tangent=d
+    )
+    c = [rng.normal(size=(R, N)) for _ in range(3)]
+    loss = sum((torch.tensor(ci, device="cuda") * o).sum() for ci, o in zip(c, out))
+    loss.backward()
+    grads = [x.grad.detach().cpu().numpy() for x in leaves]
+    terms = [ci * q for ci, q in zip(c, dout)] + [-g * di for g, di in zip(grads, d)]
+    assert abs(sum(t.sum() for t in terms)) <= 1e-12 * sum(np.abs(t).sum() for t in terms)
