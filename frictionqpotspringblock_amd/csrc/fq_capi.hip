@@ -98,6 +98,11 @@ void dfree(T*& p)
     }
 }
 
+// a group's pinned memory: run states of at most PINNED_RS_MAX bytes each way
+// and transfers of at most PINNED_XFER bytes
+constexpr size_t PINNED_RS_MAX = size_t(1) << 20;
+constexpr size_t PINNED_XFER = size_t(1) << 16;
+
 // steps per resident launch of a minimise-type run (bounds one kernel's duration)
 constexpr uint64_t MIN_BLOCK = 1u << 18;
 // adjoint: device memory for the tape of the windows recorded by one launch
@@ -182,6 +187,14 @@ struct Group {
     fq::SysView* views = nullptr;
     std::vector<fq::SysView> hviews;
     std::vector<fq::RunState> hrs;
+    // Pinned memory that the run states (both ways) and small transfers pass
+    // through: a copy of pageable memory costs the host more than the copy
+    // itself (flowSteps of 20 steps on a chain of 1000 and three fields read
+    // back: 124 us with pageable copies, 70 us).
+    unsigned char* pinned = nullptr;
+    size_t pinned_rs = 0;      // bytes of the run states, 0: they are copied directly
+    bool push_pending = false; // the pinned copy of the last push may not have been read yet
+    std::mutex pinned_mutex;   // for small transfers: fields may be read by several threads
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // ragged sets: time of the group's part of every operation on its stream
@@ -322,33 +335,90 @@ struct Group {
         if (evg1) {
             (void)hipEventDestroy(evg1);
         }
+        if (pinned) {
+            (void)hipHostFree(pinned);
+        }
         if (stream) {
             (void)hipStreamDestroy(stream);
         }
     }
 
+    // (after hrs has its size)
+    void create_pinned()
+    {
+        const size_t n = sizeof(fq::RunState) * (size_t)R;
+        pinned_rs = n <= PINNED_RS_MAX ? n : 0;
+        void* p = nullptr;
+        HIPC(hipHostMalloc(&p, 2 * pinned_rs + PINNED_XFER, hipHostMallocDefault));
+        pinned = static_cast<unsigned char*>(p);
+    }
+
     void push()
     {
-        HIPC(hipMemcpyAsync(rs, hrs.data(), sizeof(fq::RunState) * R, hipMemcpyHostToDevice, stream));
+        const size_t n = sizeof(fq::RunState) * (size_t)R;
+        if (pinned_rs == n && !push_pending) {
+            std::memcpy(pinned, hrs.data(), n);
+            push_pending = true;
+            HIPC(hipMemcpyAsync(rs, pinned, n, hipMemcpyHostToDevice, stream));
+            return;
+        }
+        HIPC(hipMemcpyAsync(rs, hrs.data(), n, hipMemcpyHostToDevice, stream));
     }
 
     void pull()
     {
-        HIPC(hipMemcpyAsync(hrs.data(), rs, sizeof(fq::RunState) * R, hipMemcpyDeviceToHost, stream));
+        const size_t n = sizeof(fq::RunState) * (size_t)R;
+        void* const to = pinned_rs == n ? (void*)(pinned + n) : (void*)hrs.data();
+        HIPC(hipMemcpyAsync(to, rs, n, hipMemcpyDeviceToHost, stream));
         HIPC(hipStreamSynchronize(stream));
+        push_pending = false;
+        if (pinned_rs == n) {
+            std::memcpy(hrs.data(), to, n);
+        }
     }
 
     template <class T>
     void d2h(T* host, const T* dev, size_t n)
     {
-        HIPC(hipMemcpyAsync(host, dev, sizeof(T) * n, hipMemcpyDeviceToHost, stream));
+        std::unique_lock<std::mutex> lock(pinned_mutex, std::defer_lock);
+        const bool staged = pinned && sizeof(T) * n <= PINNED_XFER && lock.try_lock();
+        void* const to = staged ? (void*)(pinned + 2 * pinned_rs) : (void*)host;
+        HIPC(hipMemcpyAsync(to, dev, sizeof(T) * n, hipMemcpyDeviceToHost, stream));
         HIPC(hipStreamSynchronize(stream));
+        if (staged) {
+            std::memcpy(host, to, sizeof(T) * n);
+        }
+    }
+
+    // two arrays behind one synchronisation
+    template <class T, class V>
+    void d2h(T* host, const T* dev, V* host2, const V* dev2, size_t n)
+    {
+        std::unique_lock<std::mutex> lock(pinned_mutex, std::defer_lock);
+        const bool staged = pinned && (sizeof(T) + sizeof(V)) * n <= PINNED_XFER && lock.try_lock();
+        unsigned char* const stage = pinned + 2 * pinned_rs;
+        void* const to = staged ? (void*)stage : (void*)host;
+        void* const to2 = staged ? (void*)(stage + sizeof(T) * n) : (void*)host2;
+        HIPC(hipMemcpyAsync(to, dev, sizeof(T) * n, hipMemcpyDeviceToHost, stream));
+        HIPC(hipMemcpyAsync(to2, dev2, sizeof(V) * n, hipMemcpyDeviceToHost, stream));
+        HIPC(hipStreamSynchronize(stream));
+        if (staged) {
+            std::memcpy(host, to, sizeof(T) * n);
+            std::memcpy(host2, to2, sizeof(V) * n);
+        }
     }
 
     template <class T>
     void h2d(T* dev, const T* host, size_t n)
     {
-        HIPC(hipMemcpyAsync(dev, host, sizeof(T) * n, hipMemcpyHostToDevice, stream));
+        std::unique_lock<std::mutex> lock(pinned_mutex, std::defer_lock);
+        const bool staged = pinned && sizeof(T) * n <= PINNED_XFER && lock.try_lock();
+        const void* from = host;
+        if (staged) {
+            std::memcpy(pinned + 2 * pinned_rs, host, sizeof(T) * n);
+            from = pinned + 2 * pinned_rs;
+        }
+        HIPC(hipMemcpyAsync(dev, from, sizeof(T) * n, hipMemcpyHostToDevice, stream));
         HIPC(hipStreamSynchronize(stream));
     }
 
@@ -784,7 +854,6 @@ struct Group {
             HIPC(hipEventSynchronize(ev1));
             HIPC(hipEventElapsedTime(&ms, ev0, ev1));
         }
-        pull();
         for (const auto& r : hrs) { // windows moved inside a launch
             if (r.refilled) {
                 ++refills;
@@ -1327,7 +1396,9 @@ struct Group {
             HIPC(hipEventElapsedTime(&ms, ev0, ev1));
             lr_product_ms = product_n ? (float)(product_ms / (double)product_n) : 0.0f;
         }
-        pull();
+        if (total == 0) { // every other run ended with the states of its last block
+            pull();
+        }
         return ms;
     }
 
@@ -2180,6 +2251,7 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
 
     g->hviews.resize((size_t)R);
     g->hrs.assign((size_t)R, fq::RunState{});
+    g->create_pinned();
     for (int64_t r = 0; r < R; ++r) {
         const fqsb_desc& d = ds[(size_t)r];
         const int64_t N = Ns[(size_t)r];
@@ -2945,8 +3017,7 @@ int fqsb_chunk_index_at_align(fqsb_system* s, int64_t* out)
     return guard([&] {
         Group& g = *s->g;
         std::vector<int32_t> jl((size_t)g.N);
-        g.d2h(out, g.start, (size_t)g.N);
-        g.d2h(jl.data(), g.jloc, (size_t)g.N);
+        g.d2h(out, g.start, jl.data(), g.jloc, (size_t)g.N);
         for (int64_t p = 0; p < g.N; ++p) {
             out[p] += jl[(size_t)p];
         }
@@ -3408,8 +3479,7 @@ int fqsb_batch_chunk_index_at_align(fqsb_batch* b, int64_t* out)
         Group& g = *b->g;
         const size_t n = (size_t)g.total;
         std::vector<int32_t> jl(n);
-        g.d2h(out, g.start, n);
-        g.d2h(jl.data(), g.jloc, n);
+        g.d2h(out, g.start, jl.data(), g.jloc, n);
         for (size_t p = 0; p < n; ++p) {
             out[p] += jl[p];
         }

@@ -216,3 +216,36 @@ def test_tiles_windows_and_forces(sub, cls, extra):
         assert g.maxUniformDisplacement() == o.maxUniformDisplacement()
         assert g.eventDrivenStep(1e-3, False) == o.eventDrivenStep(1e-3, False)
         assert np.array_equal(g.u, o.u) and np.array_equal(g.f, o.f)
+
+
+@pytest.mark.parametrize("N", [8191, 8192, 8193])
+def test_transfers(N):
+    """Fields on both sides of the size that passes through pinned memory
+    (64 KiB), read by several threads at once."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    import frictionqpotspringblock_amd as fq
+
+    s = fq.Line1d.System_Cuspy_Laplace(**_kw(N))
+    rng = np.random.default_rng(N)
+    x, v = 1e-3 * rng.normal(size=N), rng.normal(size=N)
+    s.u, s.v = x, v
+    assert np.array_equal(s.u, x) and np.array_equal(s.v, v)
+    with ThreadPoolExecutor(4) as ex:
+        got = list(ex.map(lambda k: getattr(s, k).copy(), ["u", "v"] * 16))
+    assert all(np.array_equal(q, (x, v)[i % 2]) for i, q in enumerate(got))
+
+
+def test_many_run_states():
+    """More replicas than the run states' pinned memory holds."""
+    from frictionqpotspringblock_amd.batch import Batch
+
+    R = 8000
+    kw = _kw(3)
+    b = Batch(R, potential="Cuspy", interactions="Laplace1d", seed_stride=3, **kw)
+    b.flowSteps(50, 0.1)
+    u = b.u
+    for r in (0, 4321, R - 1):
+        o = pyoracle.Line1d.System_Cuspy_Laplace(**dict(kw, seed=kw["seed"] + 3 * r))
+        o.flowSteps(50, 0.1)
+        assert np.array_equal(u[r], o.u)
