@@ -131,10 +131,12 @@ hipError_t launch_tile_decide(const SysView* views, int nsys, const int32_t* til
                               int32_t* tflag, const RunArgs& ra, hipStream_t stream);
 // blocks of K steps per launch (chains: k_tile_block; lattices:
 // k_tile_block2d with `lds` bytes of dynamic LDS, 2 x 8 x the extended sites
-// of the largest tile; false for other interactions)
+// of the largest tile; lone: no more tiles than compute units; false for other
+// interactions)
 bool tile_block_supported(int pot, int inter);
 bool launch_tile_block(int pot, int inter, const SysView* views, const TileDesc* tiles, int ntiles, double* part,
-                       int32_t* tfail, const RunArgs& ra, int K, size_t lds, bool unit_mass, hipStream_t stream);
+                       int32_t* tfail, const RunArgs& ra, int K, size_t lds, bool unit_mass, bool lone,
+                       hipStream_t stream);
 hipError_t launch_tile_block_decide(const SysView* views, int nsys, const int32_t* tile_first, const double* part,
                                     const int32_t* tfail, const RunArgs& ra, int K, hipStream_t stream);
 bool launch_tile_finish(int pot, int inter, const SysView* views, const TileDesc* tiles, int ntiles,

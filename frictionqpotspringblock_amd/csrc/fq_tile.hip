@@ -57,17 +57,27 @@ bool tile_block_supported(int pot, int inter)
 }
 
 bool launch_tile_block(int pot, int inter, const SysView* views, const TileDesc* tiles, int ntiles, double* part,
-                       int32_t* tfail, const RunArgs& ra, int K, size_t lds, bool unit_mass, hipStream_t stream)
+                       int32_t* tfail, const RunArgs& ra, int K, size_t lds, bool unit_mass, bool lone,
+                       hipStream_t stream)
 {
+#define FQ_BLOCK_LAUNCH(P, I, PPT, UNIT)                                                                       \
+    hipLaunchKernelGGL((k_tile_block<P, I, PPT, UNIT>), dim3((unsigned)ntiles), dim3(TB_THREADS<PPT>), 0,      \
+                       stream, views, tiles, part, tfail, ra, K)
 #define FQ_BLOCK(P, I)                                                                                         \
     if (pot == P && inter == I) {                                                                              \
-        if (unit_mass) {                                                                                       \
-            hipLaunchKernelGGL((k_tile_block<P, I, true>), dim3((unsigned)ntiles), dim3(TB_THREADS), 0,        \
-                               stream, views, tiles, part, tfail, ra, K);                                      \
+        if (lone) {                                                                                            \
+            if (unit_mass) {                                                                                   \
+                FQ_BLOCK_LAUNCH(P, I, 3, true);                                                                \
+            }                                                                                                  \
+            else {                                                                                             \
+                FQ_BLOCK_LAUNCH(P, I, 3, false);                                                               \
+            }                                                                                                  \
+        }                                                                                                      \
+        else if (unit_mass) {                                                                                  \
+            FQ_BLOCK_LAUNCH(P, I, 5, true);                                                                    \
         }                                                                                                      \
         else {                                                                                                 \
-            hipLaunchKernelGGL((k_tile_block<P, I, false>), dim3((unsigned)ntiles), dim3(TB_THREADS), 0,       \
-                               stream, views, tiles, part, tfail, ra, K);                                      \
+            FQ_BLOCK_LAUNCH(P, I, 5, false);                                                                   \
         }                                                                                                      \
         return true;                                                                                           \
     }
@@ -85,6 +95,7 @@ bool launch_tile_block(int pot, int inter, const SysView* views, const TileDesc*
 #undef FQ_BLOCK_ALL
 #undef FQ_BLOCK2D
 #undef FQ_BLOCK
+#undef FQ_BLOCK_LAUNCH
     return false;
 }
 

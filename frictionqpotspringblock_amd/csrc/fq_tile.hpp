@@ -310,10 +310,16 @@ __global__ void __launch_bounds__(64) k_tile_decide(const SysView* __restrict__ 
 // NAN, as k_tile_decide does).
 // ---------------------------------------------------------------------------
 
-constexpr int TB_THREADS = 256;
-constexpr int TB_PPT = 5;                 // particles per thread of the extended segment
-constexpr int TB_KMAX = (TB_THREADS * TB_PPT - TB_TILE_PARTICLES) / 2; // 128
-static_assert(TB_KMAX == TB_KMAX_STEPS, "extended segment and block length disagree");
+// threads of a tile's workgroup with PPT particles of the extended segment per
+// thread: 256 x 5, or 512 x 3 where every tile has a compute unit to itself
+// (two wavefronts per SIMD then hide each other's latencies; flowSteps of 512
+// steps on 250007 particles, 245 tiles: 611 us with 256 x 5, 574 us; with more
+// tiles their workgroups share the units, and 512 x 3 has a fifth more padding)
+template <int PPT>
+constexpr int TB_THREADS = PPT == 3 ? 512 : 256;
+constexpr int TB_KMAX = (TB_THREADS<5> * 5 - TB_TILE_PARTICLES) / 2; // 128
+static_assert(TB_KMAX == TB_KMAX_STEPS && TB_THREADS<3> * 3 >= TB_THREADS<5> * 5,
+              "extended segment and block length disagree");
 constexpr int32_t TB_NO_FAIL = 0x7fffffff;
 
 // steps the block of system S takes (the redo count, or min(K, target - steps))
@@ -331,16 +337,15 @@ __device__ __forceinline__ int tb_steps(const RunState* rs, int K)
 // padding at rest in an unbounded well, walks behind one branch, constants of
 // the well kept). The residual sums of a step go to LDS per wavefront and to
 // memory after the block. UNIT: every system of the group has m = 1.
-template <int POT, int INT, bool UNIT>
-__global__ void __launch_bounds__(TB_THREADS) k_tile_block(const SysView* __restrict__ views,
+template <int POT, int INT, int PPT, bool UNIT>
+__global__ void __launch_bounds__(TB_THREADS<PPT>) k_tile_block(const SysView* __restrict__ views,
                                                            const TileDesc* __restrict__ tiles,
                                                            double* __restrict__ part, int32_t* __restrict__ tfail,
                                                            RunArgs ra, int K)
 {
-    constexpr int PPT = TB_PPT;
-    constexpr int NW = TB_THREADS / 64;
-    __shared__ double s_first[2][TB_THREADS];
-    __shared__ double s_last[2][TB_THREADS];
+    constexpr int NW = TB_THREADS<PPT> / 64;
+    __shared__ double s_first[2][TB_THREADS<PPT>];
+    __shared__ double s_last[2][TB_THREADS<PPT>];
     __shared__ double s_red[TB_KMAX][NW][2];
     __shared__ int s_fail;
     const TileDesc td = tiles[blockIdx.x];

@@ -249,3 +249,15 @@ def test_many_run_states():
         o = pyoracle.Line1d.System_Cuspy_Laplace(**dict(kw, seed=kw["seed"] + 3 * r))
         o.flowSteps(50, 0.1)
         assert np.array_equal(u[r], o.u)
+
+
+@pytest.mark.parametrize("N,m", [(256 * 1024, 1.0), (256 * 1024 + 1, 1.0), (256 * 1024 + 1, 2.0)])
+def test_tiles_share_units(N, m):
+    """Chains of as many tiles as compute units, and one more."""
+    g, o = _pair("Line1d", "System_Cuspy_Laplace", [N], dict(k_interactions=1.0), m=m)
+    v = np.random.default_rng(N).normal(size=N)
+    for s in (g, o):
+        s.v = v
+        s.flowSteps(150, 0.5)
+    assert np.array_equal(g.u, o.u) and np.array_equal(g.f, o.f)
+    assert np.array_equal(g.chunk.index_at_align, o.chunk.index_at_align)
