@@ -75,8 +75,14 @@ bool launch_adj_reverse(const SysView* views, const AdjBuffers& ab, int slots, i
     switch (slots) {
 #define FQ_REV(P)                                                                                              \
     case P:                                                                                                    \
-        hipLaunchKernelGGL((k_adj_reverse<P>), dim3((unsigned)(ab.R * ab.nt)), dim3(ADJ_REV_THREADS), lds,     \
-                           stream, views, ab, steps);                                                          \
+        if (ab.tj) {                                                                                           \
+            hipLaunchKernelGGL((k_adj_reverse<P, true>), dim3((unsigned)(ab.R * ab.nt)),                       \
+                               dim3(ADJ_REV_THREADS), lds, stream, views, ab, steps);                          \
+        }                                                                                                      \
+        else {                                                                                                 \
+            hipLaunchKernelGGL((k_adj_reverse<P, false>), dim3((unsigned)(ab.R * ab.nt)),                      \
+                               dim3(ADJ_REV_THREADS), lds, stream, views, ab, steps);                          \
+        }                                                                                                      \
         break;
         FQ_ADJ_SLOTS(FQ_REV)
 #undef FQ_REV

@@ -19,7 +19,10 @@
 // from these and is not written: its acceleration is that of the preceding
 // step's last stage, (g - eta v) / m with the g of the preceding u1, and its
 // well is the one that holds u1 (a window's wells are walked to from those of
-// its checkpoint). Both kernels are bound by the tape's bytes: 64 chains of
+// its checkpoint). Where a walk of the window passed yield positions that do not
+// ascend (a user may set any), two wells can hold a slip: the record kernel
+// reports it (ADJ_ERR_ROWS) and the host repeats the pass with the wells on
+// the tape (tj). Both kernels are bound by the tape's bytes: 64 chains of
 // 4096, 2000 steps, record / reverse with u1, v, a and the well (28 bytes per
 // particle-step): 3.0 / 4.6 ms, with u1 and v (16 bytes): 1.9 / 3.3
 // ms (4.5 / 2.6 TB/s; in the reverse kernel the instructions of a step come
@@ -81,6 +84,7 @@ __global__ void __launch_bounds__(MAXT) k_adj_record(const SysView* __restrict__
     ab.tu += blockIdx.y * ab.ts;
     ab.tv += blockIdx.y * ab.ts;
     ab.tuf += blockIdx.y * ab.K * ab.R;
+    ab.tj = ab.tj ? ab.tj + blockIdx.y * ab.ts : nullptr;
     const SysView& S = views[r];
     constexpr int T = MAXT; // launched with exactly MAXT threads
     const int t = threadIdx.x;
@@ -155,16 +159,21 @@ __global__ void __launch_bounds__(MAXT) k_adj_record(const SysView* __restrict__
                         ++j;
                         lo = hi;
                         hi = row[j + 1];
+                        bad |= own[k] && hi < lo ? ADJ_ERR_ROWS : 0;
                     }
                     while (x < lo && j > jmin) {
                         --j;
                         hi = lo;
                         lo = row[j];
+                        bad |= own[k] && hi < lo ? ADJ_ERR_ROWS : 0;
                     }
-                    bad |= own[k] && !(lo <= x && x < hi);
+                    bad |= own[k] && !(lo <= x && x < hi) ? ADJ_ERR_WALK : 0;
                     jl[k] = j;
                     yl[k] = lo;
                     yr[k] = hi;
+                }
+                if (ab.tj && own[k]) {
+                    ab.tj[q] = jl[k];
                 }
                 xb[e] = x;
             }
@@ -205,7 +214,7 @@ __global__ void __launch_bounds__(MAXT) k_adj_record(const SysView* __restrict__
         }
     }
     if (bad) {
-        *ab.err = 1;
+        atomicOr(ab.err, bad);
     }
 }
 
@@ -220,7 +229,8 @@ __global__ void __launch_bounds__(MAXT) k_adj_record(const SysView* __restrict__
 // cotangents after the step alone, so it is exchanged together with the slips
 // of the step before, whose force gives this step's acceleration. The tape is
 // loaded two steps ahead.
-template <int SLOTS>
+// WELLS: with the wells on the tape.
+template <int SLOTS, bool WELLS>
 __global__ void __launch_bounds__(ADJ_REV_THREADS) k_adj_reverse(const SysView* __restrict__ views, AdjBuffers ab,
                                                                    int steps)
 {
@@ -305,9 +315,18 @@ __global__ void __launch_bounds__(ADJ_REV_THREADS) k_adj_reverse(const SysView* 
         }
         acc[i] = 0.0;
     };
-    // the well of slip y of an own particle, from the current one
-    auto walk = [&](int i, double y) {
-        if (!(lo[i] <= y && y < hi[i])) {
+    // the well of slip y of an own particle at step n, from the current one
+    auto walk = [&](int i, double y, int n) {
+        if constexpr (WELLS) {
+            const int32_t j = ab.tj[(int64_t)n * Rnp + (int64_t)r * ab.np + pp[i]];
+            if (j != jc[i]) {
+                flush(i);
+                jc[i] = j;
+                lo[i] = Y[(int64_t)pp[i] * nch + j];
+                hi[i] = Y[(int64_t)pp[i] * nch + j + 1];
+            }
+        }
+        else if (!(lo[i] <= y && y < hi[i])) {
             if (acc[i] != 0.0) {
                 flush(i);
             }
@@ -348,9 +367,9 @@ __global__ void __launch_bounds__(ADJ_REV_THREADS) k_adj_reverse(const SysView* 
     auto neighbours = [&](int buf, int i) { return sx[buf * B + T * i - 1] + sx[buf * B + T * i + 1]; };
 
     // force of an own particle from its slip and the neighbours'
-    auto force = [&](int buf, int i, double f) {
+    auto force = [&](int buf, int i, double f, int n) {
         lu[i] = __builtin_fma(-2.0, x[i], neighbours(buf, i));
-        walk(i, x[i]);
+        walk(i, x[i], n);
         d[i] = __builtin_fma(0.5, lo[i] + hi[i], -x[i]);
         g[i] = __builtin_fma(k, lu[i], __builtin_fma(mu, d[i], kf * (f - x[i])));
     };
@@ -413,7 +432,7 @@ __global__ void __launch_bounds__(ADJ_REV_THREADS) k_adj_reverse(const SysView* 
                 double a = px[i];
                 if (n > 0) {
                     x[i] = px[i];
-                    force(xb, i, puf);
+                    force(xb, i, puf, n - 1);
                     a = w * __builtin_fma(meta, v[i], g[i]);
                 }
                 const double v1 = __builtin_fma(dt, a, v[i]);
@@ -456,7 +475,7 @@ __global__ void __launch_bounds__(ADJ_REV_THREADS) k_adj_reverse(const SysView* 
 #pragma unroll
         for (int i = 0; i < SLOTS; ++i) {
             if (own[i]) {
-                force(2, i, uf);
+                force(2, i, uf, steps - 1);
             }
         }
         // (the first step's slips go to the other buffer)

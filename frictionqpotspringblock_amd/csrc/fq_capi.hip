@@ -975,6 +975,29 @@ struct Group {
     void adjoint_backward(const double* gu, const double* gv, const double* ga, double* gu0, double* gv0,
                           double* ga0, double* gpar, double* gy)
     {
+        int32_t err = adjoint_reverse(gu, gv, ga, gu0, gv0, ga0, gpar, gy, nullptr);
+        if (err == fq::ADJ_ERR_ROWS) { // once more with the wells on the tape
+            int32_t* tj = dalloc<int32_t>(tp_cap);
+            try {
+                err = adjoint_reverse(gu, gv, ga, gu0, gv0, ga0, gpar, gy, tj) & fq::ADJ_ERR_WALK;
+            }
+            catch (...) {
+                (void)hipStreamSynchronize(stream);
+                dfree(tj);
+                throw;
+            }
+            dfree(tj);
+        }
+        if (err) {
+            throw Error("a well walk left the landscape window while recomputing the trajectory");
+        }
+    }
+
+    // the pass itself; tj: tape of wells (tp_cap entries) or null. Returns
+    // ADJ_ERR_* (the results are then not written)
+    int32_t adjoint_reverse(const double* gu, const double* gv, const double* ga, double* gu0, double* gv0,
+                            double* ga0, double* gpar, double* gy, int32_t* tj)
+    {
         if (!adj_valid) {
             throw Error("no adjoint forward run to differentiate");
         }
@@ -1115,6 +1138,7 @@ struct Group {
             ab.K = adj_K;
             ab.n = adj_n;
             ab.w0 = w0;
+            ab.tj = tj;
             ab.rnt = (int32_t)rnt;
             ab.rtp = rtp;
             ab.rhalo = rnt == 1 ? 0 : adj_K;
@@ -1131,6 +1155,7 @@ struct Group {
                 abw.tv = tp_v + to * RNt;
                 abw.wa = ck_a + (size_t)w * RN;
                 abw.wj = ck_j + (size_t)w * RN;
+                abw.tj = tj ? tj + to * RNt : nullptr;
                 abw.tuf = tp_uf + to * (size_t)R;
                 // adjoint state: read from one buffer, written to the other
                 abw.au = ad_u;
@@ -1164,14 +1189,15 @@ struct Group {
         adj_reverse_ms = (float)(rev_ms / (double)adj_nw);
         int32_t err = 0;
         d2h(&err, ad_err, 1);
-        if (err) {
-            throw Error("a well walk left the landscape window while recomputing the trajectory");
+        if ((tj ? err & fq::ADJ_ERR_WALK : err) != 0) {
+            return err;
         }
         HIPC(hipMemcpyAsync(gu0, ad_u, sizeof(double) * RN, hipMemcpyDeviceToDevice, stream));
         HIPC(hipMemcpyAsync(gv0, ad_v, sizeof(double) * RN, hipMemcpyDeviceToDevice, stream));
         HIPC(hipMemcpyAsync(ga0, ad_a, sizeof(double) * RN, hipMemcpyDeviceToDevice, stream));
         HIPC(hipMemcpyAsync(gpar, ad_par, sizeof(double) * (size_t)R * 4, hipMemcpyDeviceToDevice, stream));
         HIPC(hipStreamSynchronize(stream));
+        return 0;
     }
 
     // per-replica mu, k_interactions, k_frame, eta (the parameters the adjoint

@@ -218,6 +218,8 @@ struct LrBuffers {
 // particles of a tile's extended segment per thread
 constexpr int ADJ_REV_THREADS = 512;
 constexpr int ADJ_REV_MAX_SLOTS = 8;
+constexpr int ADJ_ERR_WALK = 1; // a well walk left the landscape window
+constexpr int ADJ_ERR_ROWS = 2; // a well walk passed yield positions that do not ascend
 // LDS entries of one exchange buffer of k_adj_reverse
 constexpr int adj_rev_stride(int slots)
 {
@@ -230,6 +232,7 @@ constexpr int adj_rev_stride(int slots)
 struct AdjBuffers {
     double* tu;     // tape [K][R*np]: u1 = u + dt v + dt^2/2 a of step n
     double* tv;     // tape: v at the start of step n
+    int32_t* tj;    // tape: well of step n, or null (the one that holds u1)
     double* tuf;    // tape [K][R]: frame position of step n
     double* wu;     // state at the window start [R*N] (its checkpoint)
     double* wv;
@@ -245,7 +248,7 @@ struct AdjBuffers {
     double* gpar;   // [R][4] accumulated d/d(mu, k_interactions, k_frame, eta)
     double* gpart;  // [R][nt][4] the window's partial sums per tile
     double* gy;     // [R][N][nchunk] accumulated d/dy, or null
-    int32_t* err;   // set to 1 if a well walk left the landscape window
+    int32_t* err;   // ADJ_ERR_* of the recorded windows
     int64_t N;
     int64_t R;
     // k_adj_record over several windows at once (workgroup row blockIdx.y =

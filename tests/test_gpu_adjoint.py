@@ -244,3 +244,38 @@ def test_window_lengths(R, N, K):
     grads = [x.grad.detach().cpu().numpy() for x in leaves]
     terms = [ci * q for ci, q in zip(c, dout)] + [-g * di for g, di in zip(grads, d)]
     assert abs(sum(t.sum() for t in terms)) <= 1e-12 * sum(np.abs(t).sum() for t in terms)
+
+
+@pytest.mark.parametrize("N,K", [(8, 25), (600, 7)])
+def test_rows_that_do_not_ascend(N, K):
+    """Every fourth yield position of a row lies below the one before it, so
+    that two wells hold the slips in between and a step's well depends on where
+    the particle came from. Central differences of a linear loss along the
+    trajectory (exact but for rounding while no well changes)."""
+    import torch
+
+    from frictionqpotspringblock_amd import adjoint as A
+
+    rng = np.random.default_rng(N)
+    R, n, h = 2, 60, 1e-6
+    b = _batch(R, N)
+    u0, _, a0, par, y = _setup(b, rng, vscale=0.0)
+    y = y.clone()
+    y[..., 5::4] = y[..., 4:-1:4] - 0.3 * (y[..., 4:-1:4] - y[..., 3:-2:4])
+    v0 = torch.tensor(rng.uniform(1.0, 3.0, size=(R, N)), device="cuda")
+    c = [torch.tensor(rng.normal(size=(R, N)), device="cuda") for _ in range(3)]
+
+    def loss(*leaves):
+        return sum((ci * o).sum() for ci, o in zip(c, A.run(b, n, K, *leaves)))
+
+    d = [torch.tensor(rng.normal(size=(R, N)), device="cuda") for _ in range(3)]
+    leaves = [x.clone().requires_grad_(True) for x in (u0, v0, a0, par, y)]
+    loss(*leaves).backward()
+    for q in range(3):
+        ends = []
+        for s in (h, -h):
+            x = [u0, v0, a0, par, y]
+            x[q] = x[q] + s * d[q]
+            ends.append(loss(*x).item())
+        fd, got = (ends[0] - ends[1]) / (2 * h), (leaves[q].grad * d[q]).sum().item()
+        assert abs(fd - got) <= 1e-6 * float((leaves[q].grad * d[q]).abs().sum()), (q, fd, got)
