@@ -1053,10 +1053,15 @@ struct Group {
             }
             // more than 4 particles per thread spill (64 chains of 4096, 2 tiles
             // of 6 per thread: 0.80 ms per window; 4 tiles of 3: 0.17 ms; 8 of
-            // 2: 0.22 ms, more of it in halos)
-            while (fq::adj_reverse_slots(nt == 1 ? N : (N + nt - 1) / nt + 2 * halo) > 4 &&
-                   (N + 2 * nt - 1) / (2 * nt) >= halo) {
-                nt *= 2;
+            // 2: 0.22 ms, more of it in halos): more tiles while that gives
+            // a thread fewer particles (a long window's halos may outweigh it)
+            auto slots_of = [&](int64_t n) {
+                return fq::adj_reverse_slots(n == 1 ? N : (N + n - 1) / n + 2 * halo);
+            };
+            for (int64_t n = 2 * nt; slots_of(nt) > 4 && (N + n - 1) / n >= halo; n *= 2) {
+                if (slots_of(n) > 0 && slots_of(n) < slots_of(nt)) {
+                    nt = n;
+                }
             }
         }
         // at least as many tiles as make a tile and its halos fit the kernel

@@ -246,6 +246,35 @@ def test_window_lengths(R, N, K):
     assert abs(sum(t.sum() for t in terms)) <= 1e-12 * sum(np.abs(t).sum() for t in terms)
 
 
+@pytest.mark.parametrize("n", [5, 1100])
+@pytest.mark.parametrize("N,K", [(4096, 1024), (4096, 1499), (4096, 2047), (3500, 1173), (3000, 1400), (2500, 1000), (2049, 600)])
+def test_long_windows(N, K, n):
+    """Windows whose halos are about as long as a tile (a run shorter than the
+    window and one longer than the shortest): every length that the forward
+    pass takes has tiles in the backward pass. The identity and its bound are
+    those of test_window_lengths, with the operations of n steps."""
+    import torch
+
+    from frictionqpotspringblock_amd import adjoint as A
+
+    rng = np.random.default_rng(N + K)
+    R = 1
+    b = _batch(R, N)
+    u0, v0, a0, par, y = _setup(b, rng, vscale=1.0)
+    uf0 = torch.tensor(b.u_frame)
+    leaves = [x.clone().requires_grad_(True) for x in (u0, v0, a0, par, y)]
+    out = A.run(b, n, K, *leaves)
+    args = [x.detach().cpu().numpy() for x in (u0, v0, a0)]
+    d = [rng.normal(size=x.shape) for x in args] + [rng.normal(size=(R, 4)) * 1e-2, rng.normal(size=tuple(y.shape))]
+    _, dout = TLM.run(*args, y.cpu().numpy(), par.numpy(), uf0.numpy(), n, DT, M, tangent=d)
+    c = [rng.normal(size=(R, N)) for _ in range(3)]
+    loss = sum((torch.tensor(ci, device="cuda") * o).sum() for ci, o in zip(c, out))
+    loss.backward()
+    grads = [x.grad.detach().cpu().numpy() for x in leaves]
+    terms = [ci * q for ci, q in zip(c, dout)] + [-g * di for g, di in zip(grads, d)]
+    assert abs(sum(t.sum() for t in terms)) <= max(1e-12, 1e-14 * n) * sum(np.abs(t).sum() for t in terms)
+
+
 @pytest.mark.parametrize("N,K", [(8, 25), (600, 7)])
 def test_rows_that_do_not_ascend(N, K):
     """Every fourth yield position of a row lies below the one before it, so
