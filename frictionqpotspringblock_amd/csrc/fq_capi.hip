@@ -223,11 +223,13 @@ struct Group {
     int32_t* tb_first = nullptr;      // [R + 1]
     double* tile_part_k = nullptr;    // [tb_ntiles][tile_k][2]
     int32_t* tile_fail = nullptr;     // [tb_ntiles]
-    // captured blocks of tiled steps (hipGraph), keyed by the run arguments and
-    // the number of steps; FQSB_NO_GRAPHS=1 launches the kernels one by one
+    // captured blocks of tiled steps (hipGraph), keyed by what the recorded
+    // launches hold: the run arguments, the number of steps and the steps per
+    // launch; FQSB_NO_GRAPHS=1 launches the kernels one by one
     struct TileGraph {
         fq::RunArgs ra;
         uint64_t steps;
+        int k;
         hipGraphExec_t exec;
     };
     std::vector<TileGraph> tile_graphs;
@@ -735,8 +737,9 @@ struct Group {
                 enqueue(nb);
                 return;
             }
+            const int k = blocks ? block_steps() : 1;
             for (const auto& tg : tile_graphs) {
-                if (tg.steps == nb && std::memcmp(&tg.ra, &ra, sizeof(ra)) == 0) {
+                if (tg.steps == nb && tg.k == k && std::memcmp(&tg.ra, &ra, sizeof(ra)) == 0) {
                     HIPC(hipGraphLaunch(tg.exec, stream));
                     return;
                 }
@@ -762,7 +765,7 @@ struct Group {
                 (void)hipGraphExecDestroy(tile_graphs.front().exec);
                 tile_graphs.erase(tile_graphs.begin());
             }
-            tile_graphs.push_back(TileGraph{ra, nb, exec});
+            tile_graphs.push_back(TileGraph{ra, nb, k, exec});
             HIPC(hipGraphLaunch(exec, stream));
         };
         uint64_t todo = total;
@@ -2473,7 +2476,7 @@ static void nopassing_tiled(Group& g, const fq::RunArgs& ra, uint64_t max_iter)
             (void)hipGraphExecDestroy(g.np_graphs.front().exec);
             g.np_graphs.erase(g.np_graphs.begin());
         }
-        g.np_graphs.push_back(Group::TileGraph{ra, nb, exec});
+        g.np_graphs.push_back(Group::TileGraph{ra, nb, 1, exec});
         HIPC(hipGraphLaunch(exec, g.stream));
     };
     while (true) {
@@ -3727,6 +3730,17 @@ int fqsb_ragged_group_info(const fqsb_ragged* r, uint64_t group, int64_t* info)
                                g.pot,       g.inter, g.ext,   g.minim, g.total,
                                blocked ? g.tb_kmax : 0};
         std::copy(v, v + 13, info);
+    });
+}
+
+int fqsb_ragged_group_plans(const fqsb_ragged* r, uint64_t group, int* count)
+{
+    return guard([&] {
+        if (group >= r->groups.size()) {
+            throw Error("group index out of range");
+        }
+        const Group& g = *r->groups[(size_t)group];
+        *count = (int)(g.tile_graphs.size() + g.np_graphs.size());
     });
 }
 

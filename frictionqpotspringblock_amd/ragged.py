@@ -137,15 +137,16 @@ class Ragged:
     PATHS = {0: "resident", 1: "tiles", 2: "streaming", 3: "nopassing-resident", 4: "nopassing-tiles"}
 
     def group_info(self, g):
-        """Launch group g: its systems (indices), largest size, path and
-        current launch shape / block length."""
+        """Launch group g: its systems (indices), largest size, path,
+        current launch shape / block length and captured plans."""
         info = np.empty(13, dtype=np.int64)
         _check(capi().fqsb_ragged_group_info(self._h, int(g), info.ctypes.data_as(_ip)))
         idx = np.empty(int(info[0]), dtype=np.uint64)
         _check(capi().fqsb_ragged_group_systems(self._h, int(g), idx.ctypes.data_as(_up)))
         ppt = (C.c_int * 32)()
         thr = (C.c_int * 32)()
-        cnt = C.c_int()
+        cnt, plans = C.c_int(), C.c_int()
+        _check(capi().fqsb_ragged_group_plans(self._h, int(g), C.byref(plans)))
         _check(capi().fqsb_ragged_group_shapes(self._h, int(g), ppt, thr, 32, C.byref(cnt)))
         return {
             "systems": idx.astype(int),
@@ -155,6 +156,7 @@ class Ragged:
             "launch": (int(info[3]), int(info[4])),
             "block": int(info[5]),
             "block_max": int(info[12]),
+            "plans": plans.value,
             "key": "-".join(str(int(x)) for x in info[6:11]) + f"-{int(np.ceil(np.log2(max(int(info[1]), 1))))}",
             "shapes": [(int(ppt[i]), int(thr[i])) for i in range(min(cnt.value, 32))],
         }

@@ -424,6 +424,9 @@ enum {
  * external, minimisation, particles, longest block the tiles' halos allow
  * (chains 128; lattices: K halo rows, 8 unless FQSB_LATTICE_K is set). */
 int fqsb_ragged_group_info(const fqsb_ragged* r, uint64_t group, int64_t* info);
+/* Captured launch plans the group keeps (tiled groups; one for each set of run
+ * arguments, number of steps and block length, at most 8). */
+int fqsb_ragged_group_plans(const fqsb_ragged* r, uint64_t group, int* count);
 /* Time (ms) of the group's part of every operation since the last reset,
  * between HIP events on the group's stream, and the particle-steps (no-passing
  * groups: particle-sweeps) it took. */

@@ -214,3 +214,22 @@ def test_ragged_autotune(oracle, tmp_path):
     res2 = c.autotune(cache=cache, smooth=smooth)
     assert all(r["cached"] for r in res2.values())
     assert [r["choice"] for r in res2.values()] == [r["choice"] for r in res.values()]
+
+
+def test_block_length_of_captured_plans(oracle):
+    """A run with the arguments of an earlier one and another block length is
+    captured anew instead of replaying blocks of the earlier length; going
+    back to that length uses its plan again."""
+    from frictionqpotspringblock_amd.ragged import Ragged
+
+    systems = [("System_Cuspy_Laplace", _par(5000, 3))]
+    rg, (s,) = Ragged(systems), [_oracle_system(oracle, n, kw) for n, kw in systems]
+    assert rg.group_info(0)["path"] == "tiles"
+    plans = []
+    for block in (128, 16, 128, 7):
+        rg.set_group_block(0, block)
+        rg.flowSteps(128, 0.1)
+        s.flowSteps(128, 0.1)
+        plans.append(rg.group_info(0)["plans"])
+        _assert_same(rg, [s], block)
+    assert plans == [1, 2, 2, 3]
