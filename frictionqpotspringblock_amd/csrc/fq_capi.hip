@@ -1966,6 +1966,51 @@ int64_t validate_desc(const fqsb_desc& d)
     return N;
 }
 
+// Dynamic LDS of a workgroup at most (the kernels' static arrays beside it).
+size_t lds_limit_of(const hipDeviceProp_t& prop)
+{
+    return prop.sharedMemPerBlock - 2048;
+}
+
+// Particles per tile of a system on the tiled path, where its tiles fit the
+// LDS (0: they do not), and the LDS they take. Chains: runs of particles;
+// lattices: whole rows, at most rows - 2 per tile so that the halo rows are
+// distinct; long range: lr_tile particles and every slip of the system.
+struct TileShape {
+    int64_t step;
+    size_t lds;
+};
+TileShape tile_shape(const fqsb_desc& d, int64_t N, int64_t lr_tile, size_t lds_limit)
+{
+    TileShape t{0, 0};
+    int64_t doubles;
+    if (d.interactions == FQSB_INT_LAPLACE2D || d.interactions == FQSB_INT_QUARTICGRADIENT2D) {
+        const int64_t rows = (int64_t)d.rows, cols = (int64_t)d.cols;
+        if (rows < 3) {
+            return t;
+        }
+        t.step = std::min<int64_t>(std::max<int64_t>(1, 4096 / cols), rows - 2) * cols;
+        doubles = t.step + 2 * cols;
+    }
+    else if (N < 3) {
+        return t;
+    }
+    else if (d.interactions == FQSB_INT_LONGRANGE1D) {
+        // with the prefactors of the tile's differences where they fit
+        t.step = lr_tile;
+        doubles = N <= fq::LR_TILE_PREF_MAX ? 2 * N + t.step : N;
+    }
+    else {
+        t.step = 4096;
+        doubles = std::min<int64_t>(N, t.step) + 2;
+    }
+    t.lds = sizeof(double) * (size_t)doubles;
+    if (t.lds > lds_limit) {
+        t.step = 0;
+    }
+    return t;
+}
+
 // A group of systems that share rank, potential, interactions, external
 // forcing and minimisation (one kernel instantiation), each with its own size
 // and parameters. Fields are stored system after system ([sum N]); the
@@ -2020,7 +2065,7 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
     g->device = dev;
     hipDeviceProp_t prop;
     HIPC(hipGetDeviceProperties(&prop, dev));
-    g->lds_limit = prop.sharedMemPerBlock - 2048;
+    g->lds_limit = lds_limit_of(prop);
     g->cus = prop.multiProcessorCount;
     if (const char* gk = std::getenv("FQSB_GENERAL_KERNEL")) {
         g->general_kernel = gk[0] == '1';
@@ -2126,8 +2171,7 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
         }
     }
 
-    // tiles of the streaming systems (chains: runs of particles; lattices:
-    // whole rows, at most rows - 2 per tile so that the halo rows are distinct)
+    // tiles of the streaming systems
     if ((g->streaming || lr_dual) && fq::tile_supported(g->pot, inter, g->ext)) {
         const char* nt = std::getenv("FQSB_NO_TILES");
         bool ok = !(nt && nt[0] == '1');
@@ -2141,38 +2185,21 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
         }
         lr_tile = lr_tile <= 2 * (int64_t)g->cus ? LR_TILE_WAVE : LR_TILE_PARTICLES;
         for (int64_t r = 0; r < R && ok; ++r) {
-            const fqsb_desc& d = ds[(size_t)r];
             const int64_t N = Ns[(size_t)r];
-            const bool lat = inter == FQSB_INT_LAPLACE2D || inter == FQSB_INT_QUARTICGRADIENT2D;
-            const int64_t cols = d.rank == 1 ? 1 : (int64_t)d.cols;
-            const int64_t rows = (int64_t)d.rows;
-            const bool lr = inter == FQSB_INT_LONGRANGE1D;
-            int64_t step;
-            if (lat) {
-                int64_t rpt = std::max<int64_t>(1, 4096 / cols);
-                rpt = std::min<int64_t>(rpt, rows - 2);
-                ok = rows >= 3 && rpt >= 1;
-                step = rpt * cols;
-            }
-            else {
-                ok = N >= 3;
-                step = lr ? lr_tile : 4096;
-            }
+            const TileShape shape = tile_shape(ds[(size_t)r], N, lr_tile, g->lds_limit);
+            ok = shape.step > 0;
+            lds = std::max(lds, shape.lds);
             first[(size_t)r] = (int32_t)tl.size();
-            for (int64_t p0 = 0; ok && p0 < N; p0 += step) {
+            for (int64_t p0 = 0; ok && p0 < N; p0 += shape.step) {
                 fq::TileDesc td{};
                 td.sys = (int32_t)r;
                 td.p0 = p0;
-                td.p1 = std::min<int64_t>(N, p0 + step);
+                td.p1 = std::min<int64_t>(N, p0 + shape.step);
                 tl.push_back(td);
-                // LDS: the tile's slips and halo (long range: every slip of the
-                // system and the prefactors of the tile's differences)
-                const int64_t nl = lr ? (N <= fq::LR_TILE_PREF_MAX ? 2 * N + step : N) : (td.p1 - td.p0) + 2 * (lat ? cols : 1);
-                lds = std::max<size_t>(lds, sizeof(double) * (size_t)nl);
             }
         }
         first[(size_t)R] = (int32_t)tl.size();
-        if (ok && lds <= g->lds_limit && !tl.empty()) {
+        if (ok && !tl.empty()) {
             g->tiled = true;
             g->ntiles = (int)tl.size();
             g->tile_lds = lds;
@@ -3646,8 +3673,14 @@ int fqsb_ragged_create(const fqsb_desc* descs, uint64_t n, fqsb_ragged** out)
         // over tiles are one size class (their launches do not depend on the
         // size, and a group's operations cost about as long as its slowest
         // system's: three events of 96 systems, 41 groups on the GPU's four
-        // queues: 97 ms, 19 groups: 53 ms)
+        // queues: 97 ms, 19 groups: 63 ms). Not among them: systems without
+        // tiles or whose tiles do not fit (a group steps over tiles as a whole) and long
+        // range, whose tiles take LDS by the size of the group's largest system
         constexpr int TILED = 64;
+        int dev = 0;
+        HIPC(hipGetDevice(&dev));
+        hipDeviceProp_t prop;
+        HIPC(hipGetDeviceProperties(&prop, dev));
         typedef std::tuple<int, int, int, int, int, int> Key;
         std::map<Key, std::vector<uint64_t>> classes;
         rg->sizes.resize((size_t)n);
@@ -3661,8 +3694,14 @@ int fqsb_ragged_create(const fqsb_desc* descs, uint64_t n, fqsb_ragged** out)
             while ((int64_t(1) << lg) < N) {
                 ++lg;
             }
-            if (d.minimisation == FQSB_MIN_OVERDAMPED ? N > NOPASSING_RESIDENT_MAX
-                                                      : resident_max > 0 && N > resident_max) {
+            if (d.minimisation == FQSB_MIN_OVERDAMPED) {
+                if (N > NOPASSING_RESIDENT_MAX) {
+                    lg = TILED;
+                }
+            }
+            else if (resident_max > 0 && N > resident_max && d.interactions != FQSB_INT_LONGRANGE1D &&
+                     fq::tile_supported(d.potential, d.interactions, d.external) &&
+                     tile_shape(d, N, 0, lds_limit_of(prop)).step > 0) {
                 lg = TILED;
             }
             classes[Key(d.rank, d.potential, d.interactions, d.external, d.minimisation, lg)].push_back(i);

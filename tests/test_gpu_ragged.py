@@ -18,6 +18,7 @@ CLASS = {
     "System_SemiSmooth_Laplace": (1, "SemiSmooth", "Laplace1d", 0),
     "System_Smooth_Laplace": (1, "Smooth", "Laplace1d", 0),
     "System_Cuspy_Quartic": (1, "Cuspy", "Quartic1d", 0),
+    "System_Cuspy_LongRange": (1, "Cuspy", "LongRange1d", 0),
     "System_SemiSmooth_Quartic": (1, "SemiSmooth", "Quartic1d", 0),
     "System_Smooth_Quartic": (1, "Smooth", "Quartic1d", 0),
     "Line2d.System_Cuspy_Laplace": (2, "Cuspy", "Laplace2d", 0),
@@ -233,3 +234,27 @@ def test_block_length_of_captured_plans(oracle):
         plans.append(rg.group_info(0)["plans"])
         _assert_same(rg, [s], block)
     assert plans == [1, 2, 2, 3]
+
+
+def test_systems_without_tiles_leave_the_others(oracle):
+    """Lattices whose tiles do not fit (two rows; rows too long for the LDS)
+    and a long-range chain too large for one are in groups of their own: the
+    other large systems of their classes still step over tiles, each with the
+    oracle's results."""
+    from frictionqpotspringblock_amd.ragged import Ragged
+
+    systems = [("Line2d.System_Cuspy_Laplace", _par(r * c, i, shape=[r, c]))
+               for i, (r, c) in enumerate([(50, 60), (2, 1500), (3, 9000), (60, 70)])]
+    systems += [("System_Cuspy_LongRange", _par(N, 9 + i, alpha=1.0)) for i, N in enumerate([2500, 21000])]
+    systems += [("System_Cuspy_Laplace", _par(N, 20 + i)) for i, N in enumerate([2500, 5000])]
+    rg = Ragged(systems)
+    info = [rg.group_info(g) for g in range(rg.groups)]
+    path = {int(i): q["path"] for q in info for i in q["systems"]}
+    assert path == {0: "tiles", 1: "streaming", 2: "streaming", 3: "tiles", 4: "tiles", 5: "streaming", 6: "tiles",
+                    7: "tiles"}
+    assert sum(q["path"] == "tiles" for q in info) == 3
+    singles = [_oracle_system(oracle, n, kw) for n, kw in systems]
+    rg.flowSteps(3, 0.1)
+    for s in singles:
+        s.flowSteps(3, 0.1)
+    _assert_same(rg, singles, "flow")
