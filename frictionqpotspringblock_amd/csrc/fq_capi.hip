@@ -1732,12 +1732,16 @@ struct Group {
             set_iref_current();
             const bool device = !streaming && (!tiled || !own) && minim == FQSB_MIN_INERTIAL &&
                                 (!own || std::getenv("FQSB_HOST_QUASISTATIC") == nullptr);
+            // (long-range chains of a resident workgroup: over tiles while
+            // these fit two per CU, else in k_quasi; the sum is the exact one
+            // in either, so that a replica does not depend on their number)
+            const bool exact = !streaming;
             if (!device || !quasistatic_device(qa, tol, niter_tol, ms)) {
                 if (!own) {
                     throw Error("the quasistatic protocol without allocation needs the device-side driver, which "
                                 "is not compiled for this system class");
                 }
-                ms = quasistatic_host(qa, tol, niter_tol, max_iter);
+                ms = quasistatic_host(qa, tol, niter_tol, max_iter, exact);
             }
             auto fetch = [&](auto* host, const auto* dev) {
                 if (host) {
@@ -1845,8 +1849,9 @@ struct Group {
         return true;
     }
 
-    // the protocol event by event with the group's operations
-    float quasistatic_host(const fq::QsArgs& qa, double tol, uint64_t niter_tol, uint64_t max_iter)
+    // the protocol event by event with the group's operations; exact: long
+    // range by the sequential sum whatever lr_method
+    float quasistatic_host(const fq::QsArgs& qa, double tol, uint64_t niter_tol, uint64_t max_iter, bool exact)
     {
         auto on = [&](int64_t r) { return !mask || mask[r]; };
         auto record = [&](int64_t e, int begin) {
@@ -1893,7 +1898,7 @@ struct Group {
                     ra.tol = tol;
                     ra.tol2 = tol * tol;
                     ra.niter_tol = (int64_t)niter_tol;
-                    minimise_run(ra, max_iter);
+                    exact ? run(ra, max_iter, MIN_BLOCK, false) : minimise_run(ra, max_iter);
                     for (int64_t r = 0; r < R; ++r) {
                         const auto st = hrs[(size_t)r].status;
                         if (on(r) && st != fq::ST_CONVERGED) {

@@ -215,3 +215,33 @@ def test_matrix_quasistatic_full_size():
     assert np.array_equal(qm["inc"], qe["inc"])
     assert np.array_equal(mat.index_at_align, ext.index_at_align)
     assert np.allclose(mat.u, ext.u, rtol=1e-9, atol=1e-9)
+
+
+@pytest.mark.parametrize("method", ["matrix", "exact"])
+def test_quasistatic_does_not_depend_on_the_replicas(method):
+    """The protocol of a long-range batch of at most 2048 particles, whose
+    tiles of one wavefront fit two per compute unit with 4 replicas and not
+    with 60: bit for bit the same, and the single system's (whichever way
+    timeSteps evaluates the forces)."""
+    import frictionqpotspringblock_amd as fq
+    from frictionqpotspringblock_amd.batch import Batch
+
+    N = 600
+    kw = dict(m=1.0, eta=2.0 * np.sqrt(3.0) / 10.0, mu=1.0, k_interactions=1.0, alpha=1.0, k_frame=1.0 / N, dt=0.1,
+              shape=[N], seed=11, distribution="weibull", parameters=[2.0, 1.0, 0.0], offset=-100.0, nchunk=200)
+    u = np.random.default_rng(0).uniform(-0.5, 0.5, size=(60, N))
+    got = []
+    for R in (4, 60):
+        b = Batch(R, seed_stride=N, potential="Cuspy", interactions="LongRange1d", **kw)
+        b.longrange_method = method
+        b.u = u[:R]
+        q = b.quasistatic(1e-3, 3)
+        got.append([b.u, q["S"], q["u_frame"], q["f_frame"], q["inc"]])
+    for x, y in zip(*got):
+        assert np.array_equal(x, y[:4])
+    s = fq.Line1d.System_Cuspy_LongRange(**dict(kw, seed=kw["seed"] + 3 * N))
+    s.u = u[3]
+    q = s.quasistatic(1e-3, 3)
+    assert np.array_equal(s.u, got[1][0][3])
+    for k, x in zip(("S", "u_frame", "f_frame", "inc"), got[1][1:]):
+        assert np.array_equal(q[k], x[3])
