@@ -29,7 +29,7 @@ namespace fq {
 // One entry of k_flow: from the state in memory to the state in memory, until
 // the launch's step budget (of which earlier entries took `launch_done`) or a
 // NaN; without INLINE_REFILL also up to a step that has to move a window
-// (ST_REFILL, `rmask`: this thread's particles). Returns why it stopped.
+// (ST_REFILL, `refill_mask`: this thread's particles). Returns why it stopped.
 template <int POT, int INT, int EXT, int PPT, bool UNIT, bool FULL, bool INLINE_REFILL>
 __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views, const RunArgs& ra,
                                               int64_t& launch_done, uint32_t& refill_mask)
@@ -471,13 +471,15 @@ __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views
         flow_entry<POT, INT, EXT, PPT, UNIT, FULL, false>(views, ra, launch_done, rmask);
     }
     else {
+        bool refilled = false;
         while (flow_entry<POT, INT, EXT, PPT, UNIT, FULL, false>(views, ra, launch_done, rmask) == ST_REFILL) {
             __syncthreads(); // the state of every lane's particles is in memory
-            if (rmask) {
-                views[blockIdx.x].rs->refilled = 1;
-            }
+            refilled = true;
             refill_wave(views, (int64_t)threadIdx.x * PPT, 0, rmask);
             __syncthreads();
+        }
+        if (refilled && threadIdx.x == 0) {
+            views[blockIdx.x].rs->refilled = 1;
         }
     }
 }

@@ -338,6 +338,7 @@ __device__ __forceinline__ void resident_body(const SysView* __restrict__ views,
         ev_done0 = rs->steps;
     }
     int64_t launch_done = 0; // steps of the earlier entries of this launch
+    bool refilled = false;   // an entry ended for a refill
     uint32_t rmask = 0;      // this thread's particles that need a refill (bit i: particle base + i)
     int32_t status;
     int it;
@@ -991,15 +992,19 @@ __device__ __forceinline__ void resident_body(const SysView* __restrict__ views,
         // refill from the written-back state, then reload it: the LDS of this
         // entry must no longer be read when the next one publishes
         __syncthreads(); // the state of every lane's particles is in memory
-        if (rmask) {
-            rs->refilled = 1;
-        }
+        refilled = true;
         refill_wave(views, base, refill_u, rmask);
         refill_u = 0;
         __syncthreads();
     }
 
     if (t == 0) {
+        // (not by each thread beside the refill: that store made the step loop
+        // reload its spilled scalars, 278 instead of 18 v_readlane in the step
+        // of <4, 512>; minimise with time_activity 20 to 50% slower)
+        if (refilled) {
+            rs->refilled = 1;
+        }
         rs->inc = inc;
         rs->u_frame = uf;
         if constexpr (QS) {
