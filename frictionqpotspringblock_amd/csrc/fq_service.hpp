@@ -13,9 +13,10 @@
 namespace fq {
 
 constexpr int SVC_THREADS = 256;
-// workgroups that reduce a whole system (one per system): SVC_THREADS up to
-// that many particles, else this
+// workgroups that reduce a whole system (one per system): at most so many
+// threads (k_qs_record SVC_THREADS up to that many particles)
 constexpr int SVC_SUM_THREADS = 1024;
+constexpr int MAX_UNIFORM_THREADS = 512;
 
 // First window of every particle's landscape: cumsum of nchunk increments,
 // then += offset; align to u (which is 0 at construction).
@@ -205,7 +206,7 @@ __global__ void __launch_bounds__(SVC_THREADS) k_forces(const SysView* __restric
 // maxUniformDisplacement: rs->red0 = min over particles, rs->red_flag = 1 if
 // a SemiSmooth particle is outside the parabolic part of its well.
 template <int POT>
-__global__ void __launch_bounds__(SVC_SUM_THREADS) k_max_uniform(const SysView* __restrict__ views, int32_t direction)
+__global__ void __launch_bounds__(MAX_UNIFORM_THREADS) k_max_uniform(const SysView* __restrict__ views, int32_t direction)
 {
     __shared__ double s_d[RES_MAX_WAVES];
     __shared__ int s_f[RES_MAX_WAVES];
@@ -217,6 +218,10 @@ __global__ void __launch_bounds__(SVC_SUM_THREADS) k_max_uniform(const SysView* 
     // four particles at a time: the load of a well waits for that of its index
     constexpr int C = 4;
     const int64_t T = blockDim.x;
+    auto take = [&](double u, double lo, double hi) {
+        const double x = max_uniform_particle<POT>(S, u, lo, hi, direction, outside);
+        r = x < r ? x : r;
+    };
     for (int64_t p0 = threadIdx.x; p0 < S.N; p0 += C * T) {
         double up[C], yl[C], yr[C];
         int32_t j[C];
@@ -232,14 +237,26 @@ __global__ void __launch_bounds__(SVC_SUM_THREADS) k_max_uniform(const SysView* 
             yl[c] = L.y[p * L.nchunk + j[c]];
             yr[c] = L.y[p * L.nchunk + j[c] + 1];
         }
+        uint32_t left = 0; // particles that left their well (rare)
 #pragma unroll
         for (int c = 0; c < C; ++c) {
-            const int64_t p = p0 + c * T;
-            if (p < S.N) {
-                align_particle(L, p, up[c], yl[c], yr[c], j[c]);
-                const double x = max_uniform_particle<POT>(S, up[c], yl[c], yr[c], direction, outside);
-                r = x < r ? x : r;
+            if (p0 + c * T < S.N) {
+                if (yl[c] <= up[c] && up[c] < yr[c]) {
+                    take(up[c], yl[c], yr[c]);
+                }
+                else {
+                    left |= 1u << c;
+                }
             }
+        }
+        while (left) { // one call of the alignment, not one per particle
+            const int64_t p = p0 + __builtin_ctz(left) * T;
+            left &= left - 1;
+            const double u = S.u[p];
+            int32_t q = L.jloc[p];
+            double lo = L.y[p * L.nchunk + q], hi = L.y[p * L.nchunk + q + 1];
+            align_particle(L, p, u, lo, hi, q);
+            take(u, lo, hi);
         }
     }
     for (int off = 32; off > 0; off >>= 1) {
