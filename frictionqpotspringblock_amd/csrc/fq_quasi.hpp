@@ -119,9 +119,11 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
     // particles per thread: no spills) and one step per loop iteration
     constexpr bool INPLACE = quasi_inplace(PPT, MAXT);
     double sa[PPT], sb[INPLACE ? 1 : PPT], v[PPT], a[PPT];
-    // constants of the current well (well_consts)
-    constexpr bool WC1 = POT != POT_CUSPY;
-    double c0[PPT], c1[WC1 ? PPT : 1];
+    // constants of the current well (well_consts); with 16 particles per thread
+    // the others spill, and only Cuspy's mid-point is kept
+    constexpr bool WC = POT == POT_CUSPY || PPT <= 8;
+    constexpr bool WC1 = POT != POT_CUSPY && WC;
+    double c0[WC ? PPT : 1], c1[WC1 ? PPT : 1];
     int32_t jl[PPT];
     // INPLACE: [PPT][T] the state of the last committed step
     double* const s_keep = s_dyn + (CHAIN ? 4 * (int64_t)T : 2 * N);
@@ -146,14 +148,19 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
     };
     auto set_well = [&](int i, double lo, double hi) {
         set_bounds(i, lo, hi);
-        double k1;
-        well_consts<POT>(P, lo, hi, c0[i], k1);
-        if constexpr (WC1) {
-            c1[i] = k1;
+        if constexpr (WC) {
+            double k1;
+            well_consts<POT>(P, lo, hi, c0[i], k1);
+            if constexpr (WC1) {
+                c1[i] = k1;
+            }
         }
     };
     auto well_force = [&](int i, double x) -> double {
-        return potential_force_wc<POT>(P, x, yl_r[i], yr_r[i], c0[i], c1[WC1 ? i : 0]);
+        if constexpr (!WC) {
+            return potential_force<POT>(P, x, yl_r[i], yr_r[i]);
+        }
+        return potential_force_wc<POT>(P, x, yl_r[i], yr_r[i], c0[WC ? i : 0], c1[WC1 ? i : 0]);
     };
 
     // lattices: for each register the row above, its own and the row below
@@ -690,7 +697,7 @@ k_quasi_chain(const SysView* __restrict__ views, RunArgs ra, QsArgs qa)
         const SysView& W = V();
 #pragma unroll
         for (int i = 0; i < PPT; ++i) {
-            sa[i] = v[i] = a[i] = c0[i] = 0.0;
+            sa[i] = v[i] = a[i] = c0[WC ? i : 0] = 0.0;
             if constexpr (WC1) {
                 c1[i] = 0.0;
             }

@@ -59,6 +59,27 @@ QUASI_SIG = (
 QUASI_FULL = {"cuspy_laplace"}
 
 
+def pipelined(pot, it, ppt, mt):
+    """Whether a variant's quasistatic driver is k_quasi_chain (fq_quasi.hpp)
+    and not k_quasi, and whether minimise alone runs on it as well (else on
+    k_resident). k_quasi_chain needs more registers: where it spills hundreds
+    of them the general kernels are faster. Three events / a quench of 16
+    chains, ms (k_quasi_chain / the general kernels): Cuspy-Laplace of 8192,
+    8 x 1024: 72 / 30, 34 / 10; 16 x 512: 59 / 19, 28 / 7.5; of 4096, 4 x 1024:
+    7.9 / 8.9, 4.0 / 3.9; 16 x 256: 5.3 / 11.8, 2.8 / 5.7. SemiSmooth-Laplace
+    of 8192, 8 x 1024: 188 / 46, 111 / 22; of 4096, 4 x 1024: 43 / 14, 28 / 8.
+    Smooth-Laplace, 16 x 256: 73 / 63, 30 / 23."""
+    if it == "INT_LONGRANGE1D":
+        return False, False
+    if ppt <= 2 or (ppt <= 8 and mt <= 512):
+        return True, True
+    if it not in CHAINS or pot == "POT_SMOOTH":
+        return False, False
+    if (ppt, mt) == (16, 256):
+        return True, True
+    return pot == "POT_CUSPY" and (ppt, mt) == (4, 1024), False
+
+
 def quasi_launcher(name, pot, ints):
     out = [f"bool launch_quasi_{name}({QUASI_SIG})", "{"]
     for it, exts, variants in ints:
@@ -66,9 +87,12 @@ def quasi_launcher(name, pot, ints):
             continue
         for ppt, mt in variants:
             out.append(f"    if (inter == {it} && ppt == {ppt} && maxt == {mt}) {{")
-            # k_quasi_chain (fq_quasi.hpp); lattices with 4 or more particles
-            # per thread and 128 registers would spill there
-            if it in CHAINS or (it != "INT_LONGRANGE1D" and (mt <= 512 or ppt <= 2)):
+            driver, alone = pipelined(pot, it, ppt, mt)
+            if not alone:
+                out.append("        if (qa.plain) { // minimise runs on k_resident")
+                out.append("            return false;")
+                out.append("        }")
+            if driver:
                 forms = [("true", "true", "unit_mass && full"), ("true", "false", "unit_mass")] if name in QUASI_FULL else []
                 if it not in CHAINS:
                     forms = [("true", "false", "unit_mass")]
@@ -83,9 +107,6 @@ def quasi_launcher(name, pot, ints):
                 k = f"k_quasi_chain<{pot}, {it}, {ppt}, {mt}, false, false>"
             else:
                 k = f"k_quasi<{pot}, {it}, {ppt}, {mt}, false>"
-                out.append("        if (qa.plain) { // the protocol only: minimise runs on k_resident")
-                out.append("            return false;")
-                out.append("        }")
             out.append(f"        hipLaunchKernelGGL(({k}), dim3(nsys), dim3(threads), lds, stream, views, ra, qa);")
             out.append("        return true;")
             out.append("    }")

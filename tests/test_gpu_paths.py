@@ -198,6 +198,45 @@ def test_minimise_lattices(cls, extra, shape):
     _minimise(*_pair("Line2d", cls, shape, extra, m=2.0 if shape[0] == 41 else 1.0))
 
 
+@pytest.mark.parametrize("shape,N", [((0, 0), 4097), ((0, 0), 8192), ((4, 1024), 4096), ((16, 256), 4093), ((16, 512), 8191)])
+@pytest.mark.parametrize("pot,inter", [("Cuspy", "Laplace1d"), ("SemiSmooth", "Laplace1d"), ("Smooth", "Laplace1d"), ("Cuspy", "Quartic1d")])
+def test_quasistatic_of_large_variants(pot, inter, shape, N):
+    """The protocol and minimise at the launch shapes whose driver is chosen
+    by class (the pipelined one or the general kernels), the sizes above 4096
+    among them, where no other variant holds a chain."""
+    from frictionqpotspringblock_amd.batch import Batch
+
+    extra = {"Laplace1d": dict(k_interactions=1.0), "Quartic1d": dict(a1=1.0, a2=5.0)}[inter]
+    kw = _kw(N)
+    del kw["k_interactions"]
+    kw.update(extra, offset=-100.0, nchunk=200)
+    if pot == "SemiSmooth":
+        kw["kappa"] = 1.0
+    b = Batch(2, seed_stride=N, potential=pot, interactions=inter, **kw)
+    if shape[0]:
+        b.set_launch(*shape)
+    u = np.random.default_rng(N).uniform(-0.5, 0.5, size=(2, N))
+    b.u = u
+    kicks = pot == "Smooth"
+    q = b.quasistatic(1e-3, 2 if kicks else 3, kicks_only=kicks)
+    o = getattr(pyoracle.Line1d, f"System_{pot}_{inter[:-2]}")(**dict(kw, seed=kw["seed"] + N))
+    o.u = u[1]
+    for k in range(q["S"].shape[1]):
+        if k == 0:
+            o.u_frame = 0.0
+        else:
+            o.eventDrivenStep(1e-3, kicks or k % 2 == 0)
+        if kicks or k % 2 == 0:
+            o.minimise()
+        assert q["u_frame"][1, k] == o.u_frame and q["inc"][1, k] == o.inc
+    assert np.array_equal(b.u[1], o.u)
+    b.u = u
+    b.minimise()
+    o.u = u[1]
+    o.minimise()
+    assert np.array_equal(b.u[1], o.u) and b.inc[1] == o.inc
+
+
 @pytest.mark.parametrize("sub,cls,extra", CLASSES[:4], ids=[c[1] for c in CLASSES[:4]])
 def test_tiles_windows_and_forces(sub, cls, extra):
     """A chain over tiles whose windows move between blocks of steps, and the
