@@ -202,7 +202,14 @@ struct Group {
     // it took, summed until reset
     hipEvent_t evr[2] = {nullptr, nullptr};
     double busy_ms = 0.0, busy_ps = 0.0;
-    int ppt = 0, maxt = 0, threads = 0;
+    // resident launch shapes: particles per thread, the variant's thread bound
+    // and the threads launched (choose_launch)
+    struct Shape {
+        int ppt = 0, maxt = 0, threads = 0;
+    };
+    Shape sh_steps; // timeSteps / flowSteps
+    Shape sh_track; // runs of k_resident that decide after every step
+    Shape sh_quasi; // minimise and the quasistatic driver
     bool streaming = false; // systems too large for a resident workgroup
     // tiled per-step path for streaming groups (fq_tile.hpp); FQSB_NO_TILES=1
     // keeps them on the one-workgroup streaming kernel
@@ -483,8 +490,48 @@ struct Group {
         forces(fq::FF_POT | fq::FF_INT | fq::FF_FRAME | fq::FF_DAMP | fq::FF_TOTAL | (ext ? fq::FF_THERMAL : 0));
     }
 
-    // Pick the resident variant: fewest particles per thread that fits, then
-    // the smallest compiled thread bound (most registers per thread).
+    // Whether every system's particles fill the threads of a shape.
+    bool full_threads(const Shape& sh) const
+    {
+        bool full = true;
+        for (const auto& S : hviews) {
+            full &= S.N % sh.ppt == 0;
+        }
+        return full;
+    }
+
+    // The launch shapes. Requested ones hold for every run. Otherwise the
+    // fewest particles per thread that fit, then the smallest compiled thread
+    // bound (most registers per thread), and for the pipelined driver
+    // (k_quasi_chain) of chains and lattices without external forcing:
+    // variants of at most 512 threads (those of 1024 have 128 registers per
+    // thread, which 4 particles per thread exceed), 4 particles per thread up
+    // to 2048 particles, else 8 (a quench and a kick of 100 chains of 3000, 4 x
+    // 768 / 8 x 384: SemiSmooth-Laplace 43 / 7.8 ms, Smooth-Laplace 104 / 39
+    // ms, Cuspy-Quartic 10.7 / 7.0 ms; of 200 chains of 1537, 2 x 832 / 4 x 448
+    // / 8 x 256: 7.0 / 5.2 / 5.7 ms, 25 / 21 / 24 ms, 5.6 / 4.7 / 5.1 ms). Many
+    // systems (their wavefronts with 4 particles per thread exceed two per
+    // SIMD) take 8 as well, the most particle-steps per unit of time, but for
+    // Smooth, whose sine spills (1024 chains of 1024, 4 x 256 / 8 x 128: Cuspy
+    // 4.9 / 4.0 ms, SemiSmooth 8.2 / 7.5 ms, Smooth 26 / 31 ms). Up to 512
+    // particles the classes beside Cuspy-Laplace have one particle per thread
+    // (64 chains of 300, 1 x 320 / 4 x 128: SemiSmooth 2.2 / 2.9 ms, Smooth 5.3
+    // / 8.3 ms). Lattices: 100 of 40 x 50, 2 x 1024 / 4 x 512: 4.8 / 3.7 ms;
+    // 100 of 50 x 50, 4 x 640 / 8 x 320: 14.5 / 6.3 ms; 600 of 30 x 30, 4 x 256
+    // / 8 x 128: 5.7 / 6.1 ms.
+    //
+    // Cuspy-Laplace chains take that shape for every run. Of the others the
+    // steps alone are fastest with the fewest particles per thread (200
+    // flowSteps, us: SemiSmooth-Laplace, 64 of 700, 1 / 2 / 4 / 8 per thread
+    // 200 / 284 / 328 / 939; 800 of 1300, 2 / 4 / 8 1175 / 1568 / 3019; 64 of
+    // 2500, 4 / 8 766 / 1358; lattices, 64 of 30 x 30, 1 / 2 / 4 / 8 291 / 404 /
+    // 585 / 1089; 300 of 50 x 50, 4 / 8 2036 / 2687). k_resident's other
+    // runs, which decide after every step, follow the steps' shape while the
+    // systems' wavefronts fit two per SIMD (100 steps, us: SemiSmooth, 64 of
+    // 513, 1 / 4 per thread 348 / 382; 64 of 2500, 4 / 8 692 / 801) and the
+    // driver's beyond (300 of 513, 1 / 4 719 / 506; 300 of 1300, 2 / 8 1030 /
+    // 836), up to 2048 particles (300 of 2500, 4 / 8 1500 / 1731) or for Smooth
+    // at any size (1 of 4096, 4 / 8 1393 / 1009).
     void choose_launch(int want_ppt, int want_threads)
     {
         int vp[64], vm[64];
@@ -492,49 +539,7 @@ struct Group {
         if (nv <= 0) {
             throw Error("no resident kernel for this potential / interaction / external combination");
         }
-        // Chains and lattices without external forcing and without a requested shape:
-        // variants of at most 512 threads (those of 1024 have 128 registers
-        // per thread, which 4 particles per thread exceed), 4 particles per
-        // thread up to 2048 particles, else 8 (a quench and a kick of 100
-        // chains of 3000, 4 x 768 / 8 x 384: SemiSmooth-Laplace 43 / 7.8 ms,
-        // Smooth-Laplace 104 / 39 ms, Cuspy-Quartic 10.7 / 7.0 ms; of 200
-        // chains of 1537, 2 x 832 / 4 x 448 / 8 x 256: 7.0 / 5.2 / 5.7 ms,
-        // 25 / 21 / 24 ms, 5.6 / 4.7 / 5.1 ms). Many systems (their
-        // wavefronts with 4 particles per thread exceed two per SIMD) take 8
-        // as well, the most particle-steps per unit of time, but for Smooth,
-        // whose sine spills (1024 chains of 1024, 4 x 256 / 8 x 128: Cuspy 4.9
-        // / 4.0 ms, SemiSmooth 8.2 / 7.5 ms, Smooth 26 / 31 ms). Up to 512
-        // particles the classes beside Cuspy-Laplace have one particle per
-        // thread (64 chains of 300, 1 x 320 / 4 x 128: SemiSmooth 2.2 / 2.9
-        // ms, Smooth 5.3 / 8.3 ms). Lattices: 100 of 40 x 50, 2 x 1024 / 4 x
-        // 512: 4.8 / 3.7 ms; 100 of 50 x 50, 4 x 640 / 8 x 320: 14.5 / 6.3 ms;
-        // 600 of 30 x 30, 4 x 256 / 8 x 128: 5.7 / 6.1 ms.
-        const bool cuspy_laplace = pot == FQSB_POT_CUSPY && inter == FQSB_INT_LAPLACE1D;
-        const bool lattice = inter == FQSB_INT_LAPLACE2D || inter == FQSB_INT_QUARTICGRADIENT2D;
-        if (want_ppt == 0 && want_threads == 0 && inter != FQSB_INT_LONGRANGE1D && ext == FQSB_EXT_NONE && (cuspy_laplace || N > 512)) {
-            for (const int p : {4, 8}) {
-                const int thr = (int)((((N + p - 1) / p) + 63) / 64 * 64);
-                if (thr > 1024 || fq::resident_lds(inter, N, thr) > lds_limit) {
-                    continue;
-                }
-                if (p == 4 && !lattice && pot != FQSB_POT_SMOOTH && R * (int64_t)(thr / 64) > 2 * 4 * (int64_t)cus) {
-                    continue;
-                }
-                int best = -1;
-                for (int i = 0; i < nv; ++i) {
-                    if (vp[i] == p && thr <= vm[i] && vm[i] <= 512 && (best < 0 || vm[i] < vm[best])) {
-                        best = i;
-                    }
-                }
-                if (best >= 0) {
-                    ppt = p;
-                    maxt = vm[best];
-                    threads = thr;
-                    return;
-                }
-            }
-        }
-        int best = -1, best_thr = 0;
+        Shape few;
         for (int i = 0; i < nv; ++i) {
             const int p = vp[i], mt = vm[i];
             if (want_ppt > 0 && p != want_ppt) {
@@ -548,18 +553,47 @@ struct Group {
             if (fq::resident_lds(inter, N, thr) > lds_limit) {
                 continue;
             }
-            if (best < 0 || p < vp[best] || (p == vp[best] && mt < vm[best])) {
-                best = i;
-                best_thr = thr;
+            if (few.ppt == 0 || p < few.ppt || (p == few.ppt && mt < few.maxt)) {
+                few = {p, mt, thr};
             }
         }
-        if (best < 0) {
+        if (few.ppt == 0) {
             throw Error("system size " + std::to_string(N) +
                         " is outside the capacity of the resident kernels for this interaction");
         }
-        ppt = vp[best];
-        maxt = vm[best];
-        threads = best_thr;
+        sh_steps = sh_track = sh_quasi = few;
+        const bool cuspy_laplace = pot == FQSB_POT_CUSPY && inter == FQSB_INT_LAPLACE1D;
+        const bool lattice = inter == FQSB_INT_LAPLACE2D || inter == FQSB_INT_QUARTICGRADIENT2D;
+        if (want_ppt != 0 || want_threads != 0 || inter == FQSB_INT_LONGRANGE1D || ext != FQSB_EXT_NONE ||
+            !(cuspy_laplace || N > 512)) {
+            return;
+        }
+        auto many = [&](const Shape& sh) { return R * (int64_t)(sh.threads / 64) > 2 * 4 * (int64_t)cus; };
+        for (const int p : {4, 8}) {
+            Shape wide{p, 0, (int)((((N + p - 1) / p) + 63) / 64 * 64)};
+            if (wide.threads > 1024 || fq::resident_lds(inter, N, wide.threads) > lds_limit) {
+                continue;
+            }
+            if (p == 4 && !lattice && pot != FQSB_POT_SMOOTH && many(wide)) {
+                continue;
+            }
+            for (int i = 0; i < nv; ++i) {
+                if (vp[i] == p && wide.threads <= vm[i] && vm[i] <= 512 && (wide.maxt == 0 || vm[i] < wide.maxt)) {
+                    wide.maxt = vm[i];
+                }
+            }
+            if (wide.maxt == 0) {
+                continue;
+            }
+            sh_quasi = wide;
+            if (cuspy_laplace || (N > 2048 ? pot == FQSB_POT_SMOOTH : many(few))) {
+                sh_track = wide;
+            }
+            if (cuspy_laplace) {
+                sh_steps = wide;
+            }
+            return;
+        }
     }
 
     // Resident launch shapes (particles per thread, threads) that fit the
@@ -601,17 +635,18 @@ struct Group {
             HIPC(hipGetLastError());
             return;
         }
-        size_t lds = fq::resident_lds(inter, N, threads);
         // timeSteps / flowSteps of chains: the pipelined k_flow (same results)
         const bool chain = inter == FQSB_INT_NONE || inter == FQSB_INT_LAPLACE1D || inter == FQSB_INT_QUARTIC1D ||
                            inter == FQSB_INT_QUARTICGRADIENT1D;
-        bool unit_mass = true, full = true;
+        bool unit_mass = true;
         for (const auto& S : hviews) {
             unit_mass &= S.inv_m == 1.0;
-            full &= S.N % ppt == 0;
         }
+        const Shape& sh = ra.mode == fq::MODE_STEPS ? sh_steps : sh_track;
+        const size_t lds = fq::resident_lds(inter, N, sh.threads);
         if (ra.mode == fq::MODE_STEPS && chain && !general_kernel &&
-            fq::launch_flow(pot, inter, ext, ppt, maxt, threads, lds, views, (int)R, ra, stream, unit_mass, full)) {
+            fq::launch_flow(pot, inter, ext, sh.ppt, sh.maxt, sh.threads, lds, views, (int)R, ra, stream, unit_mass,
+                            full_threads(sh))) {
             HIPC(hipGetLastError());
             return;
         }
@@ -619,16 +654,17 @@ struct Group {
         // steps, which decide the same (without activity tracking and forcing)
         if (ra.mode == fq::MODE_MINIMISE && inter != FQSB_INT_LONGRANGE1D && !ra.time_activity &&
             ext == FQSB_EXT_NONE && !general_kernel) {
-            const size_t qlds = fq::quasi_lds(inter, N, ppt, maxt, threads);
+            const Shape& sq = sh_quasi;
+            const size_t qlds = fq::quasi_lds(inter, N, sq.ppt, sq.maxt, sq.threads);
             fq::QsArgs qa{};
             qa.plain = 1;
-            if (qlds <= lds_limit && fq::launch_quasi(pot, inter, ppt, maxt, threads, qlds, views, (int)R, ra, qa,
-                                                      stream, unit_mass, full)) {
+            if (qlds <= lds_limit && fq::launch_quasi(pot, inter, sq.ppt, sq.maxt, sq.threads, qlds, views, (int)R, ra,
+                                                      qa, stream, unit_mass, full_threads(sq))) {
                 HIPC(hipGetLastError());
                 return;
             }
         }
-        if (!fq::launch_resident(pot, inter, ext, ppt, maxt, threads, lds, views, (int)R, ra, stream)) {
+        if (!fq::launch_resident(pot, inter, ext, sh.ppt, sh.maxt, sh.threads, lds, views, (int)R, ra, stream)) {
             throw Error("no resident kernel variant for this launch shape");
         }
         HIPC(hipGetLastError());
@@ -1799,17 +1835,18 @@ struct Group {
         if (const char* e = std::getenv("FQSB_QS_BLOCK")) {
             ra.max_steps = std::max<int64_t>(1, std::min<int64_t>(std::atoll(e), (int64_t)MIN_BLOCK));
         }
-        const size_t lds = fq::quasi_lds(inter, N, ppt, maxt, threads);
-        bool unit_mass = true, full = true;
+        const Shape& sh = sh_quasi;
+        const size_t lds = fq::quasi_lds(inter, N, sh.ppt, sh.maxt, sh.threads);
+        const bool full = full_threads(sh);
+        bool unit_mass = true;
         for (const auto& S : hviews) {
             unit_mass &= S.inv_m == 1.0;
-            full &= S.N % ppt == 0;
         }
         push();
         HIPC(hipEventRecord(ev0, stream));
         for (bool first_launch = true;; first_launch = false) {
-            if (!fq::launch_quasi(pot, inter, ppt, maxt, threads, lds, views, (int)R, ra, qa, stream, unit_mass,
-                                  full)) {
+            if (!fq::launch_quasi(pot, inter, sh.ppt, sh.maxt, sh.threads, lds, views, (int)R, ra, qa, stream,
+                                  unit_mass, full)) {
                 if (first_launch) {
                     return false;
                 }
@@ -3248,8 +3285,8 @@ int fqsb_batch_set_launch(fqsb_batch* b, int ppt, int threads)
 
 int fqsb_batch_get_launch(const fqsb_batch* b, int* ppt, int* threads)
 {
-    *ppt = b->g->ppt;
-    *threads = b->g->threads;
+    *ppt = b->g->sh_steps.ppt;
+    *threads = b->g->sh_steps.threads;
     return 0;
 }
 
@@ -3769,7 +3806,7 @@ int fqsb_ragged_group_info(const fqsb_ragged* r, uint64_t group, int64_t* info)
             path = FQSB_PATH_STREAMING;
         }
         const bool blocked = g.tiled && g.tile_part_k != nullptr;
-        const int64_t v[13] = {g.R,         g.N,     path,    g.ppt,   g.threads,
+        const int64_t v[13] = {g.R,         g.N,     path,    g.sh_quasi.ppt, g.sh_quasi.threads,
                                blocked ? g.block_steps() : 0,  (int64_t)g.d.rank,
                                g.pot,       g.inter, g.ext,   g.minim, g.total,
                                blocked ? g.tb_kmax : 0};

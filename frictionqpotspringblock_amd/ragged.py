@@ -244,7 +244,7 @@ class Ragged:
                 continue
             if key in known:
                 kind, val = known[key]["choice"]
-                self._apply(g, kind, val)
+                self._apply(g, kind, val, info)
                 out[g] = {"key": key, "path": info["path"], "choice": [kind, val], "trials_ms": None, "cached": True}
                 continue
             if trial is None:
@@ -275,7 +275,7 @@ class Ragged:
                 best = base
             kind, val = best.split(":", 1)
             val = [int(x) for x in val.strip("()").split(",")] if kind == "launch" else int(val)
-            self._apply(g, kind, val)
+            self._apply(g, kind, val, info)
             known[key] = {"choice": [kind, val]}
             out[g] = {"key": key, "path": info["path"], "choice": [kind, val], "trials_ms": times,
                       "trials_ns_per_particle_step": rate, "cached": False}
@@ -284,9 +284,12 @@ class Ragged:
                 json.dump(known, f, indent=1, sort_keys=True)
         return out
 
-    def _apply(self, g, kind, val):
+    def _apply(self, g, kind, val, info=None):
         if kind == "launch":
-            self.set_group_launch(g, *val)
+            # (the automatic choice has shapes of their own for other runs
+            # than the protocol: it stays where the trials end with it)
+            if info is None or tuple(val) != tuple(info["launch"]):
+                self.set_group_launch(g, *val)
         else:
             self.set_group_block(g, val)
 

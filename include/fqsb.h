@@ -224,10 +224,12 @@ int fqsb_batch_create(const fqsb_desc* desc, uint64_t replicas, uint64_t seed_st
 int fqsb_batch_destroy(fqsb_batch* b);
 uint64_t fqsb_batch_replicas(const fqsb_batch* b);
 /* Choose the resident launch shape (particles per thread, threads per
- * workgroup); 0, 0 restores the automatic choice (chains: 4 particles per
- * thread while the replicas' wavefronts fit two per SIMD, else 8, where a
- * kernel variant holds a replica so; otherwise the fewest particles per
- * thread that hold it). Results do not depend on the shape. */
+ * workgroup) of every run; 0, 0 restores the automatic choice: the fewest
+ * particles per thread that hold a replica, or, for Cuspy-Laplace chains and
+ * for minimise and the quasistatic protocol of the other classes, 4 per thread
+ * while the replicas' wavefronts fit two per SIMD, else 8, where a kernel
+ * variant of at most 512 threads holds a replica so. Results do not depend on
+ * the shape. fqsb_batch_get_launch: that of timeSteps / flowSteps. */
 int fqsb_batch_set_launch(fqsb_batch* b, int ppt, int threads);
 int fqsb_batch_get_launch(const fqsb_batch* b, int* ppt, int* threads);
 /* How a batch evaluates LongRange1d (detail.h:846-867):
@@ -419,7 +421,8 @@ enum {
     FQSB_PATH_NOPASSING_RESIDENT = 3,  /* no-passing sweeps, one workgroup per system */
     FQSB_PATH_NOPASSING_TILES = 4      /* no-passing sweeps over tiles */
 };
-/* info[13] = systems, largest N, path, particles per thread, threads, block
+/* info[13] = systems, largest N, path, particles per thread and threads (of the
+ * quasistatic protocol, which the tuner times), block
  * length of the tiled path (0: not blocked), rank, potential, interactions,
  * external, minimisation, particles, longest block the tiles' halos allow
  * (chains 128; lattices: K halo rows, 8 unless FQSB_LATTICE_K is set). */

@@ -237,6 +237,41 @@ def test_quasistatic_of_large_variants(pot, inter, shape, N):
     assert np.array_equal(b.u[1], o.u) and b.inc[1] == o.inc
 
 
+@pytest.mark.parametrize("pot,inter,shape,ppt", [
+    ("Cuspy", "Laplace1d", [513], 4), ("SemiSmooth", "Laplace1d", [513], 1), ("Smooth", "Laplace1d", [2500], 4),
+    ("Cuspy", "Quartic1d", [1537], 2), ("Cuspy", "Laplace2d", [19, 28], 1), ("Cuspy", "Laplace2d", [33, 33], 2)])
+def test_automatic_shapes(pot, inter, shape, ppt):
+    """Steps, runs that decide after every step and the driver each have a
+    launch shape of their own, which depends on the number of replicas as
+    well: two replicas have the results of the first two of 300."""
+    from frictionqpotspringblock_amd.batch import Batch
+
+    N = int(np.prod(shape))
+    kw = _kw(N, offset=-100.0, nchunk=200)
+    kw["shape"] = shape
+    if inter == "Quartic1d":
+        del kw["k_interactions"]
+        kw.update(a1=1.0, a2=5.0)
+    if pot == "SemiSmooth":
+        kw["kappa"] = 1.0
+    u = np.random.default_rng(N).uniform(-0.5, 0.5, size=[300] + shape)
+    got = []
+    for R in (2, 300):
+        b = Batch(R, seed_stride=N, potential=pot, interactions=inter, **kw)
+        if R == 2:
+            assert b.launch[0] == ppt
+        b.u = u[:R]
+        i_n = b.index_at_align
+        b.flowSteps(40, 0.01)
+        got.append([b.u[:2], b.v[:2]])
+        ret = b.minimise_truncate(i_n, S_truncate=N // 8, max_iter=300, max_iter_is_error=False)
+        got[-1] += [ret[:2], b.u[:2]]
+        b.minimise()
+        got[-1] += [b.inc[:2], b.u[:2], b.f[:2], b.index_at_align[:2]]
+    for k, (x, y) in enumerate(zip(*got)):
+        assert np.array_equal(x, y), k
+
+
 @pytest.mark.parametrize("sub,cls,extra", CLASSES[:4], ids=[c[1] for c in CLASSES[:4]])
 def test_tiles_windows_and_forces(sub, cls, extra):
     """A chain over tiles whose windows move between blocks of steps, and the
