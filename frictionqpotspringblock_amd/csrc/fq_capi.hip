@@ -623,7 +623,9 @@ struct Group {
         return out;
     }
 
-    void launch_resident(const fq::RunArgs& ra)
+    // moves: k_flow's form that moves windows inside the launch, where there
+    // are two
+    void launch_resident(const fq::RunArgs& ra, bool moves = true)
     {
         if (minim == FQSB_MIN_OVERDAMPED) {
             throw Error("dynamics are not available for no-passing systems");
@@ -646,7 +648,7 @@ struct Group {
         const size_t lds = fq::resident_lds(inter, N, sh.threads);
         if (ra.mode == fq::MODE_STEPS && chain && !general_kernel &&
             fq::launch_flow(pot, inter, ext, sh.ppt, sh.maxt, sh.threads, lds, views, (int)R, ra, stream, unit_mass,
-                            full_threads(sh))) {
+                            full_threads(sh), moves)) {
             HIPC(hipGetLastError());
             return;
         }
@@ -865,8 +867,10 @@ struct Group {
             HIPC(hipEventRecord(ev0, stream));
         }
         ra.max_steps = (int64_t)std::min<uint64_t>(block, (uint64_t)std::numeric_limits<int32_t>::max());
+        // k_flow's form with refills holds 16 wavefronts per CU
+        bool moves = R <= (int64_t)cus * (16 / std::max(1, std::min(16, sh_steps.threads / 64)));
         while (total > 0) {
-            launch_resident(ra);
+            launch_resident(ra, moves);
             pull();
             bool refill = false, more = false;
             for (const auto& r : hrs) {
@@ -874,6 +878,7 @@ struct Group {
                 more |= (r.status == fq::ST_RUNNING || r.status == fq::ST_BUDGET) && r.steps < r.target;
             }
             if (refill) {
+                moves = true;
                 HIPC(fq::launch_refill(views, (int)R, N, stream));
                 ++refills;
                 for (auto& r : hrs) {

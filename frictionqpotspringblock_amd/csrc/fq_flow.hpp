@@ -28,9 +28,12 @@ namespace fq {
 
 // One entry of k_flow: from the state in memory to the state in memory, until
 // the launch's step budget (of which earlier entries took `launch_done`) or a
-// NaN; without INLINE_REFILL also up to a step that has to move a window
-// (ST_REFILL, `refill_mask`: this thread's particles). Returns why it stopped.
-template <int POT, int INT, int EXT, int PPT, bool UNIT, bool FULL, bool INLINE_REFILL>
+// NaN; but for REFILL_INLINE also up to a step that has to move a window
+// (ST_REFILL; REFILL_ENTRY: `refill_mask`, this thread's particles). Returns
+// why it stopped. WC: the well's constants are kept.
+enum FlowRefill { REFILL_HOST, REFILL_ENTRY, REFILL_INLINE };
+
+template <int POT, int INT, int EXT, int PPT, bool UNIT, bool FULL, FlowRefill REFILL, bool WC>
 __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views, const RunArgs& ra,
                                               int64_t& launch_done, uint32_t& refill_mask)
 {
@@ -43,7 +46,7 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
     const int limit = uniform_i((int)(room < budget ? (room > 0 ? room : 0) : budget));
 
     __shared__ int s_nan[2];
-    __shared__ int s_refill[2];
+    __shared__ int s_refill[2]; // (but for REFILL_INLINE)
     __shared__ int s_scan_w[RES_MAX_WAVES];
     __shared__ long long s_min_w[RES_MAX_WAVES];
     extern __shared__ double s_dyn[];
@@ -76,24 +79,29 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
     // branch: a full wavefront skips it).
     double sa[PPT], sb[PPT], v[PPT], a[PPT], yl[PPT], yr[PPT], fth[PPT];
     // constants of the current well (well_consts)
-    constexpr bool WC1 = POT != POT_CUSPY;
-    double c0[PPT], c1[WC1 ? PPT : 1];
+    constexpr bool WC1 = POT != POT_CUSPY && WC;
+    double c0[WC ? PPT : 1], c1[WC1 ? PPT : 1];
     auto set_well = [&](int i, double lo, double hi) {
         yl[i] = lo;
         yr[i] = hi;
-        double k1;
-        well_consts<POT>(P, lo, hi, c0[i], k1);
-        if constexpr (WC1) {
-            c1[i] = k1;
+        if constexpr (WC) {
+            double k1;
+            well_consts<POT>(P, lo, hi, c0[i], k1);
+            if constexpr (WC1) {
+                c1[i] = k1;
+            }
         }
     };
     auto well_force = [&](int i, double x) -> double {
-        return potential_force_wc<POT>(P, x, yl[i], yr[i], c0[i], c1[WC1 ? i : 0]);
+        if constexpr (!WC) {
+            return potential_force<POT>(P, x, yl[i], yr[i]);
+        }
+        return potential_force_wc<POT>(P, x, yl[i], yr[i], c0[WC ? i : 0], c1[WC1 ? i : 0]);
     };
     int32_t jl[PPT];
 #pragma unroll
     for (int i = 0; i < PPT; ++i) {
-        sa[i] = sb[i] = v[i] = a[i] = c0[i] = fth[i] = 0.0;
+        sa[i] = sb[i] = v[i] = a[i] = c0[WC ? i : 0] = fth[i] = 0.0;
         if constexpr (WC1) {
             c1[i] = 0.0;
         }
@@ -124,8 +132,10 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
     if (t == 0) {
         s_nan[0] = 0;
         s_nan[1] = 0;
-        s_refill[0] = 0;
-        s_refill[1] = 0;
+        if constexpr (REFILL != REFILL_INLINE) {
+            s_refill[0] = 0;
+            s_refill[1] = 0;
+        }
     }
     int64_t inc = uniform_ll(rs->inc); // scalar: its increment is a scalar add
     double uf = rs->u_frame;
@@ -163,8 +173,8 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
 
     // slips of step `it` from the state x into y, and publication into
     // exchange buffer it&1; pend: some slip of this thread leaves its well (or
-    // is NaN), so that the commit of the step walks only then. Without
-    // INLINE_REFILL their reachability as well (rmask, s_refill).
+    // is NaN), so that the commit of the step walks only then. But for
+    // REFILL_INLINE their reachability as well (rmask, s_refill).
     int pend = 0;
     uint32_t rmask = 0;
     auto prepare = [&](int it, const double(&x)[PPT], double(&y)[PPT]) {
@@ -176,8 +186,8 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
             out |= !(yl[i] <= y[i] && y[i] < yr[i]);
         }
         pend = out;
-        if constexpr (!INLINE_REFILL) {
-            rmask = 0;
+        if constexpr (REFILL != REFILL_INLINE) {
+            uint32_t mask = 0;
             if (out) { // rare: some slip leaves its well
                 // opaque copies: the addresses and comparisons of this rare
                 // path stay in it instead of being evaluated for every step
@@ -189,12 +199,15 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
                     __asm__ volatile("" : "+v"(z));
                     if (!(yl[i] <= z && z < yr[i]) && __builtin_isfinite(z) &&
                         !reachable(Y + (bq + i) * nch, jl[i], yl[i], yr[i], z, jmin, jmax)) {
-                        rmask |= 1u << i;
+                        mask |= 1u << i;
                     }
                 }
-                if (rmask) {
+                if (mask) {
                     s_refill[b] = it;
                 }
+            }
+            if constexpr (REFILL == REFILL_ENTRY) {
+                rmask = mask;
             }
         }
         publish(y, b);
@@ -235,7 +248,7 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
         if (it > limit) {
             return false;
         }
-        if constexpr (!INLINE_REFILL) {
+        if constexpr (REFILL != REFILL_INLINE) {
             if (uniform_i(s_refill[b]) == it) {
                 status = ST_REFILL;
                 return false;
@@ -314,7 +327,7 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
                         jl[i] = j;
                         set_well(i, lo, hi);
                     }
-                    else if (INLINE_REFILL && __builtin_isfinite(z)) {
+                    else if (REFILL == REFILL_INLINE && __builtin_isfinite(z)) {
                         need |= 1u << i;
                     }
                 }
@@ -325,7 +338,7 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
         }
         // windows that have to move (rare): one particle at a time by the
         // whole wavefront, the other wavefronts do not wait for it
-        if (INLINE_REFILL && __builtin_expect(__any(need != 0), 0)) {
+        if (REFILL == REFILL_INLINE && __builtin_expect(__any(need != 0), 0)) {
 #pragma unroll
             for (int i = 0; i < PPT; ++i) {
                 uint64_t lanes = __ballot((need >> i) & 1u);
@@ -444,7 +457,7 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
     }
 }
 
-// Windows that have to move are handled inside the launch: variants of up to
+// Windows that have to move are handled inside the launch (MOVES): variants of up to
 // 512 threads (256 registers) call the refill from the commit of the step, by
 // the wavefronts that need it; in variants of 1024 threads (128 registers)
 // that call would spill the step loop's registers (4 x 1024 on 1024 chains of
@@ -454,7 +467,12 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
 // the host relaunches it after k_refill. Sliding chains (256 x 1999, windows
 // of 100, 4 x 512; a window moves somewhere in nearly every step): 13 ms per
 // 1000 steps, against 273 ms with a relaunch each time.
-template <int POT, int INT, int EXT, int PPT, int MAXT, bool UNIT, bool FULL = false>
+// One particle per thread: the step alone takes 64 registers, with the refill's
+// call 124, half as many wavefronts per SIMD. Batches whose workgroups do not
+// all fit that way start with the form that leaves refills to the host (MOVES
+// false) and go on with the other one once a window has to move (800 chains of
+// 300, 300 steps, us: SemiSmooth-Laplace 576 with the call, Cuspy-Quartic 500).
+template <int POT, int INT, int EXT, int PPT, int MAXT, bool UNIT, bool FULL = false, bool MOVES = true>
 __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views, RunArgs ra)
 {
     static_assert(is_chain<INT>(), "k_flow handles chains");
@@ -465,14 +483,18 @@ __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views
     int64_t launch_done = 0;
     uint32_t rmask = 0;
     if constexpr (MAXT <= 512) {
-        flow_entry<POT, INT, EXT, PPT, UNIT, FULL, true>(views, ra, launch_done, rmask);
+        flow_entry<POT, INT, EXT, PPT, UNIT, FULL, REFILL_INLINE, true>(views, ra, launch_done, rmask);
     }
-    else if constexpr (PPT > 2) {
-        flow_entry<POT, INT, EXT, PPT, UNIT, FULL, false>(views, ra, launch_done, rmask);
+    else if constexpr (PPT > 2 || !MOVES) {
+        // (more than two per thread: the well's constants would spill: SemiSmooth, 100 chains of 4096, 300
+        // steps 1.36 ms with them)
+        flow_entry<POT, INT, EXT, PPT, UNIT, FULL, REFILL_HOST, PPT <= 2 || POT == POT_CUSPY>(
+            views, ra, launch_done, rmask);
     }
     else {
         bool refilled = false;
-        while (flow_entry<POT, INT, EXT, PPT, UNIT, FULL, false>(views, ra, launch_done, rmask) == ST_REFILL) {
+        while (flow_entry<POT, INT, EXT, PPT, UNIT, FULL, REFILL_ENTRY, true>(views, ra, launch_done, rmask) ==
+               ST_REFILL) {
             __syncthreads(); // the state of every lane's particles is in memory
             refilled = true;
             refill_wave(views, (int64_t)threadIdx.x * PPT, 0, rmask);

@@ -34,10 +34,10 @@ inline bool launch_resident(int pot, int inter, int ext, int ppt, int maxt, int 
 // full: every system has N divisible by ppt
 inline bool launch_flow(int pot, int inter, int ext, int ppt, int maxt, int threads, size_t lds,
                         const SysView* views, int nsys, const RunArgs& ra, hipStream_t stream, bool unit_mass,
-                        bool full)
+                        bool full, bool moves)
 {
 #define X(u)                                                                                                   \
-    if (launch_flow_##u(inter, ext, ppt, maxt, threads, lds, views, nsys, ra, stream, unit_mass, full)) {    \
+    if (launch_flow_##u(inter, ext, ppt, maxt, threads, lds, views, nsys, ra, stream, unit_mass, full, moves)) { \
         return true;                                                                                           \
     }
     FQ_TRY_POT(POT_CUSPY, )

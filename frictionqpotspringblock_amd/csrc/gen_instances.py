@@ -26,6 +26,8 @@ CHAINS = {"INT_NONE", "INT_LAPLACE1D", "INT_QUARTIC1D", "INT_QUARTICGRADIENT1D"}
 # k_flow shapes: those whose registers fit without large spills (other shapes
 # of timeSteps / flowSteps run on k_resident)
 FLOW_SHAPES = {(1, 1024), (2, 1024), (4, 1024), (4, 512), (8, 512), (8, 256), (16, 256)}
+# the one with a form that leaves every refill to the host (fq_flow.hpp)
+FLOW_FIXED = (1, 1024)
 
 # unit name -> (potential, [(interaction, forcing values, variants)])
 UNITS = {
@@ -48,7 +50,7 @@ SIG = (
     "int inter, int ext, int ppt, int maxt, int threads, size_t lds, const SysView* views, int nsys, "
     "const RunArgs& ra, hipStream_t stream"
 )
-FLOW_SIG = SIG + ", bool unit_mass, bool full"
+FLOW_SIG = SIG + ", bool unit_mass, bool full, bool moves"
 QUASI_SIG = (
     "int inter, int ppt, int maxt, int threads, size_t lds, const SysView* views, int nsys, const RunArgs& ra, "
     "const QsArgs& qa, hipStream_t stream, bool unit_mass, bool full"
@@ -133,6 +135,14 @@ def launcher(name, kernel, pot, ints, chains_only):
                             ("false", "false"): "!unit_mass",
                         }[(unit, full)]
                         out.append(f"        if ({cond}) {{")
+                        if (ppt, mt) == FLOW_FIXED:
+                            out.append("            if (!moves) {")
+                            out.append(
+                                f"                hipLaunchKernelGGL(({k[:-1]}, false>), dim3(nsys), dim3(threads), lds, "
+                                "stream, views, ra);"
+                            )
+                            out.append("                return true;")
+                            out.append("            }")
                         out.append(
                             f"            hipLaunchKernelGGL(({k}), dim3(nsys), dim3(threads), lds, stream, views, ra);"
                         )

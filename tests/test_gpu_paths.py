@@ -58,6 +58,29 @@ def test_windows_move_inside_flow(ppt, threads, N, v_frame):
     _same(b, ref)
 
 
+def test_windows_move_in_many_replicas():
+    """More replicas of one particle per thread than fit the compute units with
+    the refill's registers: the launch ends at the first window that moves
+    and the run goes on with the form that moves them itself."""
+    from frictionqpotspringblock_amd.batch import Batch
+
+    N, R = 65, 2050
+    kw = _kw(N)
+    b = Batch(R, seed_stride=N, potential="Cuspy", interactions="Laplace1d", **kw)
+    b.set_launch(1, 128)
+    b.advanceToFixedForce(0.5, allow_plastic=True)
+    i0 = b.index_at_align
+    b.flowSteps(200, 0.5)
+    assert np.abs(b.index_at_align - i0).max() > 15
+    start = b._get_state("start").reshape(R, -1)
+    for r in (0, 1027, R - 1):
+        s = pyoracle.Line1d.System_Cuspy_Laplace(**dict(kw, seed=kw["seed"] + r * N))
+        s.advanceToFixedForce(0.5, allow_plastic=True)
+        s.flowSteps(200, 0.5)
+        assert np.array_equal(b.u[r], s.u) and np.array_equal(b.f[r], s.f)
+        assert np.array_equal(start[r], s.chunk.start)
+
+
 def test_window_jumps_inside_flow():
     """Slips that leave the window altogether (fast particles) and slips that
     stay where they are (a particle at rest next to them)."""
