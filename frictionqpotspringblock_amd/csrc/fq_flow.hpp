@@ -486,9 +486,10 @@ __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views
         flow_entry<POT, INT, EXT, PPT, UNIT, FULL, REFILL_INLINE, true>(views, ra, launch_done, rmask);
     }
     else if constexpr (PPT > 2 || !MOVES) {
-        // (more than two per thread: the well's constants would spill: SemiSmooth, 100 chains of 4096, 300
-        // steps 1.36 ms with them)
-        flow_entry<POT, INT, EXT, PPT, UNIT, FULL, REFILL_HOST, PPT <= 2 || POT == POT_CUSPY>(
+        // (more than two per thread: the well's constants would spill;
+        // SemiSmooth, 100 chains of 4096, 300 steps 1.04 ms, with them 1.36;
+        // a forced Cuspy chain of 4096, 400 steps 1.88 ms, with them 2.40)
+        flow_entry<POT, INT, EXT, PPT, UNIT, FULL, REFILL_HOST, PPT <= 2 || (POT == POT_CUSPY && EXT == 0)>(
             views, ra, launch_done, rmask);
     }
     else {
