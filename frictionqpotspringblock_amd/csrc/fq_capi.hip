@@ -122,11 +122,14 @@ constexpr uint64_t STEP_BLOCK = 1u << 16;
 // LR_TILE_PARTICLES particles (one per thread), each tile holding every slip
 // of the chain in LDS
 constexpr int64_t LR_RESIDENT_MAX = 2048;
-// ... and, while their tiles of one wavefront fit two per CU, above this size:
-// timeSteps, flowSteps and minimise over tiles, everything else resident. A
-// step of one chain takes (resident / tiles, us): N = 448 13.6 / 11.6, 576
-// 22 / 14, 1000 56 / 20, 2000 323 / 36; below 512 a minimise loses what its
-// steps gain to the launches of the last block of steps.
+// ... and, while their tiles of one wavefront all fit the device
+// (lr_wave_tiles), above this size: timeSteps, flowSteps and minimise over
+// tiles, everything else resident. A step of one chain takes (resident /
+// tiles, us): N = 448 13.6 / 11.6, 576 22 / 14, 1000 56 / 20, 2000 323 / 36;
+// below 512 a minimise loses what its steps gain to the launches of the last
+// block of steps. Calls of a few steps, whose launches are captured at the
+// first call of that length: N = 513, 1 step 124 / 151 us, 10 steps 301 / 304;
+// N = 700, 1 step 172 / 158.
 constexpr int64_t LR_TILE_MIN = 512;
 constexpr int64_t LR_TILE_PARTICLES = 256;
 constexpr int64_t LR_TILE_WAVE = 64;
@@ -1399,8 +1402,8 @@ struct Group {
     }
 
     // timeSteps / flowSteps with LongRange1d in matrix form: per step one
-    // k_lr_gemm (interaction forces of all replicas) and one k_lr_elem (rest
-    // of timeStep). The host checks the run states every `block` steps; a
+    // k_lr_fft or k_lr_gemm (interaction forces of all replicas) and one
+    // k_lr_elem (rest of timeStep). The host checks the run states every `block` steps; a
     // replica whose next slips need a landscape refill stops (ST_REFILL)
     // until k_refill and k_lr_prologue ran, then catches up (per-replica
     // step target).
@@ -1478,9 +1481,8 @@ struct Group {
     }
 
     // minimise (detail.h:1754-1785) of every system: batches of long-range
-    // chains in matrix form run it on the FP64 matrix cores (the forces of all
-    // replicas as one product per step), others on the resident / tiled /
-    // streaming kernels
+    // chains in matrix form run it with the forces of all replicas as one
+    // product per step, others on the resident / tiled / streaming kernels
     float minimise_run(fq::RunArgs ra, uint64_t max_iter)
     {
         if (lr_method == FQSB_LR_MATRIX && !ra.time_activity) {
@@ -2058,6 +2060,24 @@ TileShape tile_shape(const fqsb_desc& d, int64_t N, int64_t lr_tile, size_t lds_
     return t;
 }
 
+// Whether the tiles of one wavefront of long-range chains all fit the device at
+// once: two per CU where their LDS allows it (up to about 5000 particles), else
+// one. A step's time is that of one tile's sums, so a second round doubles it
+// (20 steps of 3 chains of 8192, 384 tiles of one wavefront 5.1 ms, 96 tiles of
+// 256 particles 2.9 ms).
+bool lr_wave_tiles(const std::vector<int64_t>& Ns, int cus, const hipDeviceProp_t& prop)
+{
+    int64_t tiles = 0, N = 0;
+    for (const int64_t n : Ns) {
+        tiles += (n + LR_TILE_WAVE - 1) / LR_TILE_WAVE;
+        N = std::max(N, n);
+    }
+    fqsb_desc d{};
+    d.interactions = FQSB_INT_LONGRANGE1D;
+    const size_t lds = tile_shape(d, N, LR_TILE_WAVE, SIZE_MAX).lds + 1024;
+    return tiles <= (int64_t)cus * (2 * lds <= prop.sharedMemPerBlock ? 2 : 1);
+}
+
 // A group of systems that share rank, potential, interactions, external
 // forcing and minimisation (one kernel instantiation), each with its own size
 // and parameters. Fields are stored system after system ([sum N]); the
@@ -2200,12 +2220,8 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
         }
         // long-range chains that also fit a workgroup: tiles for the runs that
         // have them
-        int64_t waves = 0;
-        for (const int64_t N : Ns) {
-            waves += (N + LR_TILE_WAVE - 1) / LR_TILE_WAVE;
-        }
-        lr_dual = !g->streaming && inter == FQSB_INT_LONGRANGE1D && g->N > LR_TILE_MIN && waves <= 2 * (int64_t)g->cus &&
-                  fq::tile_supported(g->pot, inter, g->ext);
+        lr_dual = !g->streaming && inter == FQSB_INT_LONGRANGE1D && g->N > LR_TILE_MIN &&
+                  lr_wave_tiles(Ns, g->cus, prop) && fq::tile_supported(g->pot, inter, g->ext);
         if (g->streaming || lr_dual) {
             g->u2 = dalloc<double>(RN);
             g->v2 = dalloc<double>(RN);
@@ -2225,12 +2241,8 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
         std::vector<fq::TileDesc> tl;
         std::vector<int32_t> first((size_t)R + 1, 0);
         size_t lds = 0;
-        // long range: tiles of one wavefront while they fit two per CU
-        int64_t lr_tile = 0;
-        for (const int64_t N : Ns) {
-            lr_tile += (N + LR_TILE_WAVE - 1) / LR_TILE_WAVE;
-        }
-        lr_tile = lr_tile <= 2 * (int64_t)g->cus ? LR_TILE_WAVE : LR_TILE_PARTICLES;
+        const int64_t lr_tile = inter == FQSB_INT_LONGRANGE1D && lr_wave_tiles(Ns, g->cus, prop) ? LR_TILE_WAVE
+                                                                                                 : LR_TILE_PARTICLES;
         for (int64_t r = 0; r < R && ok; ++r) {
             const int64_t N = Ns[(size_t)r];
             const TileShape shape = tile_shape(ds[(size_t)r], N, lr_tile, g->lds_limit);
