@@ -2416,9 +2416,7 @@ Group* build_group_multi(const std::vector<fqsb_desc>& ds, int64_t resident_max 
         S.k4 = d.k4;
         S.k4_4 = 0.25 * d.k4;
         S.alpha = d.alpha;
-        S.lr_m = (N - N % 2) / 2;
         const size_t o = (size_t)g->off[(size_t)r];
-        S.pref = g->pref ? g->pref + o : nullptr;
         S.prefx = g->prefx ? g->prefx + 2 * o : nullptr;
         S.u = g->u + o;
         S.v = g->v + o;

@@ -159,8 +159,6 @@ struct SysView {
     int32_t pot, inter, ext, pad;
     double m, inv_m, eta, mu, kappa, k_frame, dt;
     double k, a1, a2, k2, k4, k4_4, alpha;
-    int64_t lr_m;
-    double* pref;  // LongRange1d prefactor [N]
     double* prefx; // LongRange1d prefactor of the difference d in [-(N-1), N-1], at d + N - 1 (0 at d = 0)
     double *u, *v, *a, *f, *f_pot, *f_int, *f_frame, *f_damp, *f_th;
     // streaming path (systems larger than a resident workgroup): second state
