@@ -81,6 +81,41 @@ def test_windows_move_in_many_replicas():
         assert np.array_equal(start[r], s.chunk.start)
 
 
+@pytest.mark.parametrize("ppt,threads,N", [(1, 128, 65), (2, 64, 127), (4, 128, 257), (8, 64, 509)])
+@pytest.mark.parametrize("cls", ["SemiSmooth_Laplace", "Smooth_Laplace", "Cuspy_Quartic", "Cuspy_Laplace_RandomForcing"])
+def test_windows_move_in_every_class(cls, ppt, threads, N):
+    """The same for other potentials and interactions and with random forcing
+    (chains thrown forwards, whose windows move while they come to rest)."""
+    from frictionqpotspringblock_amd.batch import Batch
+
+    pot, inter = cls.split("_")[:2]
+    kw = _kw(N, **(dict(kappa=1.0) if pot == "SemiSmooth" else {}))
+    if inter == "Quartic":
+        del kw["k_interactions"]
+        kw.update(a1=1.0, a2=5.0)
+    more = {}
+    if "Forcing" in cls:
+        kw.update(mean=0.0, stddev=0.1, seed_forcing=7, dinc_init=5, dinc=10)
+        more["external"] = "RandomNormalForcing"
+    b = Batch(2, seed_stride=N, potential=pot, interactions=inter + "1d", **kw, **more)
+    ref = []
+    for r in range(2):
+        k = dict(kw, seed=kw["seed"] + r * N)
+        if more:
+            k.update(seed_forcing=kw["seed_forcing"] + r * N, dinc_init=[5] * N, dinc=[10] * N)
+        ref.append(getattr(pyoracle.Line1d, f"System_{cls}")(**k))
+    b.set_launch(ppt, threads)
+    v = np.full(N, 20.0)
+    b.v = np.broadcast_to(v, [2, N])
+    i0 = b.index_at_align
+    b.flowSteps(100, 0.1, block=37)
+    for s in ref:
+        s.v = v
+        s.flowSteps(100, 0.1)
+    assert np.abs(b.index_at_align - i0).min() > 30 and b._get_state("start").max() > 0
+    _same(b, ref)
+
+
 def test_window_jumps_inside_flow():
     """Slips that leave the window altogether (fast particles) and slips that
     stay where they are (a particle at rest next to them)."""
@@ -139,7 +174,7 @@ def test_longrange_exact_sum(N):
     assert np.array_equal(g.chunk.index_at_align, o.chunk.index_at_align)
 
 
-@pytest.mark.parametrize("N", [255, 256, 257, 511, 512, 513, 1024, 2049, 4095, 4097, 8191, 8192, 8193, 16384])
+@pytest.mark.parametrize("N", [255, 256, 257, 511, 512, 513, 1024, 1025, 2047, 2049, 4095, 4096, 4097, 8191, 8192, 8193, 16384])
 def test_longrange_product(N):
     """The batched long-range forces at the sizes where the transforms change
     (powers of two, one more, one less; the matrix product below 257 and above
