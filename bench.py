@@ -74,7 +74,7 @@ FP64_PEAK_TFLOPS = 78.6  # MI355X FP64 vector (= FP64 matrix) peak
 # each scaled by the ratio of the true bytes of a 1 GiB device copy to what
 # the same counter reads for it (reads x 2.000, writes x 1.000);
 # profiles/k_flow_cuspy_laplace_flow_R1024_N4096.md
-FLOW_TRAFFIC_BYTES = (520_371 * 2.000 + 869_879 * 1.000) * 1024
+FLOW_TRAFFIC_BYTES = (501_980 * 2.000 + 954_390 * 1.000) * 1024
 
 LR_R = 256
 LR_N = 8192

@@ -479,8 +479,9 @@ class Batch:
     @property
     def longrange_method(self):
         """How LongRange1d forces are evaluated: "exact" (the reference's
-        sequential sum) or "matrix" (circulant product on the matrix cores,
-        the default for Cuspy batches)."""
+        sequential sum) or "matrix" (one circulant product per step for all
+        replicas, the default for Cuspy batches; timeSteps, flowSteps and
+        minimise, and quasistatic above 2048 particles)."""
         m = C.c_int()
         _check(capi().fqsb_batch_get_longrange_method(self._h, C.byref(m)))
         return {v: k for k, v in LONGRANGE_METHOD.items()}[m.value]

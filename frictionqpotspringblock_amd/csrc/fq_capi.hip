@@ -113,8 +113,8 @@ constexpr int64_t ADJ_RECORD_RING = 4096;
 // In ragged sets, systems above this size run on the tiled path (many
 // workgroups per system): with a few hundred systems the resident path
 // leaves a large system to one workgroup, the tiled path spreads it over the
-// chip (three events of 96 systems of 512 to 65536 particles: 53 ms at 2048,
-// 60 ms at 1024, 86 ms at 4096).
+// chip (three events of 96 systems of 512 to 65536 particles: 62 to 72 ms at
+// 2048, 64 at 1024, 75 at 4096).
 constexpr int64_t RAGGED_RESIDENT_MAX = 2048;
 // steps per resident launch of timeSteps / flowSteps
 constexpr uint64_t STEP_BLOCK = 1u << 16;
@@ -1698,7 +1698,7 @@ struct Group {
     // recording after event e, at [r * nevents + e] of the host arrays (any
     // may be null): S (sum of well-index changes), u_frame, mean f_frame, inc.
     // Systems that fit a resident workgroup run the whole protocol on the
-    // device (k_quasi, one launch per step budget, refill or end); the others
+    // device (k_quasi_chain or k_quasi, one launch per step budget or end); the others
     // are driven event by event from here. Returns the time around the device
     // work (ms).
     // `records`: device memory for the records (4 x R x nevents words, no
@@ -1816,7 +1816,7 @@ struct Group {
         return ms;
     }
 
-    // k_quasi for the whole protocol; false if it is not instantiated for this
+    // The driver for the whole protocol; false if none is instantiated for this
     // group (the caller then drives the events from the host)
     bool quasistatic_device(const fq::QsArgs& qa, double tol, uint64_t niter_tol, float& ms)
     {

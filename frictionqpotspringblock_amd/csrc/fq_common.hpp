@@ -69,7 +69,7 @@ constexpr int64_t LR_LDS_PREF_MAX = 4096;
 // prefactors (up to here they fit 160 KB).
 constexpr int64_t LR_TILE_PREF_MAX = 9728;
 
-// The quasistatic driver for chains (k_quasi_chain) keeps the state of the
+// The pipelined quasistatic driver (k_quasi_chain) keeps the state of the
 // last committed step in LDS (8 bytes per particle, beyond the exchange
 // buffers) instead of a second register array for these launch variants
 // (particles per thread, max threads).
@@ -78,7 +78,7 @@ FQ_HD constexpr bool quasi_inplace(int ppt, int maxt)
     return (ppt == 8 || ppt == 4) && maxt <= 512;
 }
 
-// Phase of the quasistatic driver (k_quasi) within an event.
+// Phase of the quasistatic drivers (k_quasi_chain, k_quasi) within an event.
 enum QsPhase : int32_t {
     QS_BEGIN = 0,    // the event's displacement is still to be applied
     QS_MINIMISE = 1, // minimising after the displacement
@@ -138,7 +138,7 @@ struct RunState {
     // reductions written by service kernels
     double red0;
     int32_t red_flag;
-    int32_t refilled; // set by a run whose kernel moved a landscape window inside the launch
+    int32_t refilled; // set by k_resident and k_flow: a launch moved a landscape window
     // uniform displacement of the particles applied by k_forces(FF_ADD_U)
     double du_add;
     // quasistatic driver: next event of the run (0-based), its phase, and the
@@ -280,7 +280,7 @@ struct RunArgs {
     int64_t A_truncate, S_truncate;
 };
 
-// Arguments of the quasistatic driver (k_quasi): events k = first + e,
+// Arguments of the quasistatic drivers: events k = first + e,
 // e < nevents, of the protocol
 //   k == 0:       u_frame = 0, then minimise
 //   k odd:        eventDrivenStep(eps, kick = false)

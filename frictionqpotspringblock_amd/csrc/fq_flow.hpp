@@ -472,7 +472,8 @@ __device__ __forceinline__ int32_t flow_entry(const SysView* __restrict__ views,
 // call 124, half as many wavefronts per SIMD. Batches whose workgroups do not
 // all fit that way start with the form that leaves refills to the host (MOVES
 // false) and go on with the other one once a window has to move (800 chains of
-// 300, 300 steps, us: SemiSmooth-Laplace 576 with the call, Cuspy-Quartic 500).
+// 300, 300 steps, us, with / without the call: SemiSmooth-Laplace 576 / 346,
+// Cuspy-Quartic 500 / 297).
 template <int POT, int INT, int EXT, int PPT, int MAXT, bool UNIT, bool FULL = false, bool MOVES = true>
 __global__ void __launch_bounds__(MAXT) k_flow(const SysView* __restrict__ views, RunArgs ra)
 {

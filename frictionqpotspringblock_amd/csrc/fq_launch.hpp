@@ -47,8 +47,9 @@ inline bool launch_flow(int pot, int inter, int ext, int ppt, int maxt, int thre
     return false;
 }
 
-// The quasistatic driver (no external forcing): k_quasi_chain for chains,
-// k_quasi otherwise; false if not instantiated for this potential /
+// The quasistatic driver (no external forcing): k_quasi_chain for the variants
+// of chains and lattices whose registers hold it (gen_instances.py:
+// pipelined), k_quasi otherwise; false if not instantiated for this potential /
 // interaction / shape (unit_mass: every system has m = 1; full: every system
 // has N divisible by ppt)
 inline bool launch_quasi(int pot, int inter, int ppt, int maxt, int threads, size_t lds, const SysView* views,

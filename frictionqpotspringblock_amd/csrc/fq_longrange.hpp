@@ -4,8 +4,9 @@
 //           = (K (u[r] - ub[r]))[p] - c (u[r][p] - ub[r]),
 // K[p][i] = pref[d(i, p)] (zero diagonal), c = sum_i K[p][i] (the same for
 // every p), ub[r] = u[r][0] (a per-replica shift that keeps the operands small
-// and the cancellation benign). The product runs on the FP64 matrix cores
-// (v_mfma_f64_16x16x4f64); K is never stored: each K-block's operand comes
+// and the cancellation benign). Up to 2^13 complex points (fq_lrfft.hpp) the
+// product is a cyclic convolution; beyond, it runs on the FP64 matrix cores
+// (v_mfma_f64_16x16x4f64): K is never stored: each K-block's operand comes
 // from a window of g[m] = pref[fold(m)], m = p - i, staged in LDS.
 // This path accumulates in a different order (and with fused multiply-add)
 // than the reference's sequential sum, so it is compared to the exact path

@@ -4,8 +4,8 @@ header fq_res_units.hpp that declares them.
 Each unit instantiates, for its (potential, interaction, forcing) classes and
 the variant table of each, k_resident<POT, INT, EXT, PPT, MAXT> (all modes),
 for chains k_flow<POT, INT, EXT, PPT, MAXT> (timeSteps / flowSteps), and,
-without external forcing, the quasistatic driver (k_quasi_chain; k_quasi for
-long range and large lattices); it exposes
+without external forcing, the quasistatic driver (k_quasi_chain, or k_quasi:
+see pipelined()); it exposes
 launch_resident_<unit>(), launch_flow_<unit>(), launch_quasi_<unit>() and
 resident_variants_<unit>(). Small units let hipcc compile them in parallel.
 The build (build_ext.py) generates them before compiling; by hand:

@@ -234,15 +234,18 @@ int fqsb_batch_set_launch(fqsb_batch* b, int ppt, int threads);
 int fqsb_batch_get_launch(const fqsb_batch* b, int* ppt, int* threads);
 /* How a batch evaluates LongRange1d (detail.h:846-867):
  * FQSB_LR_EXACT  -- the reference's sequential sum per particle, in the
- *                   resident or streaming kernels; bit-identical to a single
- *                   system of the same seed.
+ *                   resident, tiled or streaming kernels; bit-identical to a
+ *                   single system of the same seed.
  * FQSB_LR_MATRIX -- (default for Cuspy batches) the forces of all replicas as
- *                   one product with the circulant matrix on the FP64 matrix
- *                   cores; a different summation order, so each force differs
- *                   from the sequential sum by a few units in the last place
- *                   of the largest term. Used by timeSteps / flowSteps;
- *                   minimise and the event-driven steps always use the exact
- *                   sum. Fails on a batch without long-range interactions. */
+ *                   one product with the circulant matrix per step (transforms
+ *                   in LDS or the FP64 matrix cores, by the chain's size); a
+ *                   different summation order, so each force differs from the sequential sum by a few units in
+ *                   the last place of the largest term. Used by timeSteps,
+ *                   flowSteps and minimise (without activity,
+ *                   truncation or a count of events); in the quasistatic
+ *                   protocol only above 2048 particles. Everything else uses
+ *                   the exact sum. Fails on a batch without long-range
+ *                   interactions. */
 enum { FQSB_LR_EXACT = 0, FQSB_LR_MATRIX = 1 };
 int fqsb_batch_set_longrange_method(fqsb_batch* b, int method);
 int fqsb_batch_get_longrange_method(const fqsb_batch* b, int* method);
